@@ -128,14 +128,13 @@ PSCBFM_HD uint32_t dil_sub(uint32_t a, uint32_t b, uint32_t M) {
 // (dx&7, dy&7, dz&7) the reference feeds into linearizeBondVectorIndex
 // (CRITICAL.cu:243-261), only bit-interleaved.  The host permutes the
 // 512-entry bond table into this order once.
-constexpr uint32_t kBondWinX = 0x049u;  // bits 0,3,6
-constexpr uint32_t kBondWinY = 0x092u;  // bits 1,4,7
-constexpr uint32_t kBondWinZ = 0x124u;  // bits 2,5,8
-
+//
+// Bitwise subtraction of the three axes at once: a borrow of one axis moves
+// up three code bits, to that axis' next bit, and never meets another axis.
 PSCBFM_HD uint32_t bond_key(uint32_t partner, uint32_t self) {
-    return (((partner & kBondWinX) - (self & kBondWinX)) & kBondWinX) |
-           (((partner & kBondWinY) - (self & kBondWinY)) & kBondWinY) |
-           (((partner & kBondWinZ) - (self & kBondWinZ)) & kBondWinZ);
+    const uint32_t first = (~partner & self) << 3;                             // borrows out of bits 0..2
+    const uint32_t borrow = (~partner & self) | (~(partner ^ self) & first);   // right up to bit 5
+    return (partner ^ self ^ (borrow << 3)) & 0x1FFu;
 }
 
 // ---------------------------------------------------------------------------

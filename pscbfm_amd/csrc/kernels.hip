@@ -125,12 +125,6 @@ __device__ __forceinline__ ColorInfo load_color(gptr<const ColorInfo> colors, ui
 // << kDirShift, high = old code.
 __device__ __forceinline__ uint64_t pack_entry(uint32_t x, uint32_t y) { return uint64_t(x) | (uint64_t(y) << 32); }
 
-struct Move {
-    uint32_t to;        // code of the new corner
-    uint32_t cell[9];   // the 3x3 plane in front of the move
-    bool wraps;         // the axis coordinate crosses the periodic boundary
-};
-
 // The Z-curve masks of x, y and z as values in scalar registers.  Passing
 // the descriptor's array instead lets the compiler turn the per-lane choice
 // of an axis into a per-lane load from the argument segment, one more
@@ -146,58 +140,118 @@ __device__ __forceinline__ AxisMasks axis_masks(const SysDesc& d) {
     return m;
 }
 
-// Direction d: 0:-x 1:+x 2:-y 3:+y 4:-z 5:+z (UpdaterGPUScBFM_AB_Type.cu:534-545).
-// Front plane: p + 2 e_d + a e_u + b e_v, a,b in {-1,0,1} (CRITICAL.cu:62-176).
-__device__ __forceinline__ Move make_move(uint32_t m, uint32_t dir, const AxisMasks& mask) {
-    const uint32_t axis = dir >> 1;
-    const bool plus = (dir & 1u) != 0;
-    const uint32_t Ma = axis == 0 ? mask.x : (axis == 1 ? mask.y : mask.z);
-    const uint32_t Mu = axis == 0 ? mask.y : mask.x;
-    const uint32_t Mv = axis == 2 ? mask.y : mask.z;
-    const uint32_t oneA = Ma & (~Ma + 1u);
-    const uint32_t stepA = plus ? oneA : Ma;  // +1 or -1 in dilated form
+// A move's axis and sign.  Direction d: 0:-x 1:+x 2:-y 3:+y 4:-z 5:+z
+// (UpdaterGPUScBFM_AB_Type.cu:534-545); two flags name the axis.
+struct Dir {
+    bool x, z;  // axis x, axis z (else y)
+    bool plus;
+    __device__ __forceinline__ uint32_t number() const { return (x ? 0u : (z ? 4u : 2u)) + (plus ? 1u : 0u); }
+};
+__device__ __forceinline__ Dir dir_of_number(uint32_t d) { return {d < 2u, d >= 4u, (d & 1u) != 0u}; }
+// Direction rn % 6 of a hash (CRITICAL.cu:321-323).  rn % 6 is
+// 2 * ((rn >> 1) % 3) + (rn & 1), and h % 3 is read off the fraction h / 3:
+// for h = 3q + r < 2^31, h * ceil(2^32 / 3) modulo 2^32 is 2q + r * ceil(2^32 / 3),
+// which stays in the r-th third of the range (2q < 2^32 / 3).  One multiply
+// and two compares, whose results are the axis flags themselves.
+__device__ __forceinline__ Dir dir_of_hash(uint32_t rn) {
+    const uint32_t f = (rn >> 1) * 0x55555556u;
+    return {f < 0x55555556u, f >= 0xAAAAAAACu, (rn & 1u) != 0u};
+}
+
+struct Move {
+    uint32_t to;                  // code of the new corner
+    uint32_t c00, c02, c20, c22;  // corner cells of the 3x3 plane in front: (u-1, v-1), (u-1, v+1), (u+1, v-1), (u+1, v+1)
+};
+
+// Front plane: p + 2 e_d + a e_u + b e_v, a,b in {-1,0,1} (CRITICAL.cu:62-176),
+// with (u, v) = (y, z), (x, z), (x, y) for a move along x, y, z.  The lowest
+// code bits of x, y and z are bits 0, 1 and 2, their second bits 3, 4 and 5.
+__device__ __forceinline__ Move make_move(uint32_t m, const Dir& d, const AxisMasks& mask) {
+    const uint32_t Ma = d.x ? mask.x : (d.z ? mask.z : mask.y);
+    const uint32_t Mu = d.x ? mask.y : mask.x;
+    const uint32_t Mv = d.z ? mask.y : mask.z;
+    const uint32_t oneA = d.x ? 1u : (d.z ? 4u : 2u);
+    const uint32_t oneU = d.x ? 2u : 1u, oneV = d.z ? 2u : 4u;
+    const uint32_t step1 = d.plus ? oneA : Ma;              // +1 or -1 in dilated form
+    const uint32_t step2 = d.plus ? oneA << 3 : Ma ^ oneA;  // +2 or -2
     Move mv;
-    const uint32_t qa = dil_add(m, Ma, stepA);
-    mv.to = (m & ~Ma) | qa;
-    mv.wraps = plus ? ((m & Ma) == Ma) : ((m & Ma) == 0u);
-    const uint32_t fa = dil_add(qa, Ma, stepA);
-    const uint32_t u0 = m & Mu, v0 = m & Mv;
-    const uint32_t oneU = Mu & (~Mu + 1u), oneV = Mv & (~Mv + 1u);
-    const uint32_t u[3] = {dil_add(u0, Mu, Mu), u0, dil_add(u0, Mu, oneU)};
-    const uint32_t v[3] = {dil_add(v0, Mv, Mv), v0, dil_add(v0, Mv, oneV)};
-#pragma unroll
-    for (int a = 0; a < 3; ++a)
-#pragma unroll
-        for (int b = 0; b < 3; ++b) mv.cell[3 * a + b] = fa | u[a] | v[b];
+    const uint32_t ta = m | ~Ma, tu = m | ~Mu, tv = m | ~Mv;
+    mv.to = (m & ~Ma) | ((ta + step1) & Ma);
+    const uint32_t fa = (ta + step2) & Ma;
+    const uint32_t u0 = (tu + Mu) & Mu, u2 = (tu + oneU) & Mu;
+    const uint32_t v0 = (tv + Mv) & Mv, v2 = (tv + oneV) & Mv;
+    mv.c00 = fa | u0 | v0;
+    mv.c02 = fa | u0 | v2;
+    mv.c20 = fa | u2 | v0;
+    mv.c22 = fa | u2 | v2;
     return mv;
+}
+
+// Whether the axis coordinate of a move crosses the periodic boundary.
+__device__ __forceinline__ bool wraps(uint32_t m, const Dir& d, const AxisMasks& mask) {
+    const uint32_t Ma = d.x ? mask.x : (d.z ? mask.z : mask.y);
+    return (m & Ma) == (d.plus ? Ma : 0u);
+}
+
+// All ones when bit b of m is set, else 0.
+__device__ __forceinline__ uint32_t spread_bit(uint32_t m, uint32_t b) {
+    return uint32_t(int32_t(m << (31u - b)) >> 31);
 }
 
 // Whether any of the nine front-plane cells is set, read as 64-bit words.
 // The low code bits interleave x, y and z, so a 64-bit word of the 1-bit
 // lattice (64 cells, SHIFT 6) is an aligned 4x4x4 block and one of the byte
 // lattice (8 cells, SHIFT 3) an aligned 2x2x2 block.  In either case the 3x3
-// plane touches at most four words, those of (u-1 or u+1) x (v-1 or v+1):
-// four 8-byte gathers replace nine narrow ones, and the middle row/column
-// takes the word of whichever outer row/column shares its block.
+// plane touches at most four words, those of its corner cells, and four
+// 8-byte gathers replace nine narrow ones.
+//
+// The cells are picked from the words with masks, in 32-bit halves.  (Nine
+// 64-bit shifts, one per cell, took 65 VALU instructions per move; this takes
+// about 35: the 512^3 melt's pass 1 was bound by VALU issue.)
+//  * 4x4x4 words: the plane's own coordinate is a +- 2, the same residue
+//    modulo 4 for both signs, and its transverse coordinates are all residues
+//    but that of u + 2 (v + 2).  So with E_k = the cells whose coordinate k
+//    has the residue of m's plus 2, the plane is E_a & ~E_u & ~E_v.  A cell of
+//    residue 2 or 3 in u lies in the word of u-1, one of residue 0 or 1 in
+//    that of u+1 (where the two differ), so the words are merged by constant
+//    masks of the second coordinate bit: first over v, then over u.
+//  * 2x2x2 words: the plane has the residue of a; the word of u-1 holds only
+//    residue 1 of the plane when u is even, that of u+1 only residue 0 when u
+//    is odd, and both residues otherwise.
 template <int SHIFT>
-__device__ __forceinline__ uint32_t plane_any(gptr<const uint64_t> words, const Move& mv) {
-    const uint64_t w00 = words[mv.cell[0] >> SHIFT];  // (u-1, v-1)
-    const uint64_t w02 = words[mv.cell[2] >> SHIFT];  // (u-1, v+1)
-    const uint64_t w20 = words[mv.cell[6] >> SHIFT];  // (u+1, v-1)
-    const uint64_t w22 = words[mv.cell[8] >> SHIFT];  // (u+1, v+1)
-    // does the middle u (v) share the block of u-1 (v-1)?
-    const bool uLow = ((mv.cell[3] ^ mv.cell[0]) >> SHIFT) == 0u;
-    const bool vLow = ((mv.cell[1] ^ mv.cell[0]) >> SHIFT) == 0u;
-    const uint64_t wRow0 = vLow ? w00 : w02, wRow2 = vLow ? w20 : w22;  // words of (u-1, v), (u+1, v)
-    const uint64_t w10 = uLow ? w00 : w20, w12 = uLow ? w02 : w22;      // words of (u, v-1), (u, v+1)
-    const uint64_t w11 = uLow ? wRow0 : wRow2;                          // word of (u, v)
-    const uint64_t w[9] = {w00, wRow0, w02, w10, w11, w12, w20, wRow2, w22};
-    constexpr uint32_t kLow = (1u << SHIFT) - 1u;
-    constexpr uint32_t kUnit = SHIFT == 6 ? 1u : 8u;  // bits per cell inside the word
-    uint64_t any = 0;
-#pragma unroll
-    for (int c = 0; c < 9; ++c) any |= w[c] >> ((mv.cell[c] & kLow) * kUnit);
-    return uint32_t(any & (SHIFT == 6 ? 1u : 0xFFu));
+__device__ __forceinline__ bool plane_any(gptr<const uint64_t> words, uint32_t m, const Dir& d, const Move& mv) {
+    const uint64_t w00 = words[mv.c00 >> SHIFT], w02 = words[mv.c02 >> SHIFT];
+    const uint64_t w20 = words[mv.c20 >> SHIFT], w22 = words[mv.c22 >> SHIFT];
+    const uint32_t a0 = uint32_t(w00), a1 = uint32_t(w00 >> 32), b0 = uint32_t(w02), b1 = uint32_t(w02 >> 32);
+    const uint32_t c0 = uint32_t(w20), c1 = uint32_t(w20 >> 32), e0 = uint32_t(w22), e1 = uint32_t(w22 >> 32);
+    const uint32_t sx = spread_bit(m, 0), sy = spread_bit(m, 1), sz = spread_bit(m, 2);
+    if constexpr (SHIFT == 6) {
+        const uint32_t tx = spread_bit(m, 3), ty = spread_bit(m, 4), tz = spread_bit(m, 5);
+        // E_x and E_y are alike in both halves; E_z's second bit is the half itself
+        const uint32_t ex = (0x55555555u ^ sx) & (0xFF00FF00u ^ tx);
+        const uint32_t ey = (0x33333333u ^ sy) & (0xFFFF0000u ^ ty);
+        const uint32_t ez = 0x0F0F0F0Fu ^ sz;
+        const uint32_t nx = d.x ? 0u : ~0u, nz = d.z ? 0u : ~0u, ny = d.x || d.z ? ~0u : 0u;
+        const uint32_t exy = (ex ^ nx) & (ey ^ ny);
+        const uint32_t plane0 = ((ez & tz) ^ nz) & exy, plane1 = ((ez & ~tz) ^ nz) & exy;
+        const uint32_t su = d.x ? 0xFFFF0000u : 0xFF00FF00u;
+        const uint32_t sv0 = d.z ? 0xFFFF0000u : 0u, sv1 = d.z ? 0xFFFF0000u : ~0u;
+        auto pick = [](uint32_t s, uint32_t a, uint32_t b) { return (a & s) | (b & ~s); };
+        const uint32_t any0 = pick(su, pick(sv0, a0, b0), pick(sv0, c0, e0));
+        const uint32_t any1 = pick(su, pick(sv1, a1, b1), pick(sv1, c1, e1));
+        return ((any0 & plane0) | (any1 & plane1)) != 0u;
+    } else {
+        const uint32_t lx = 0xFF00FF00u | sx, hx = ~(0xFF00FF00u & sx);
+        const uint32_t ly = 0xFFFF0000u | sy, hy = ~(0xFFFF0000u & sy);
+        const uint32_t ul = d.x ? ly : lx, uh = d.x ? hy : hx;
+        const uint32_t vl0 = d.z ? ly : sz, vl1 = d.z ? ly : ~0u;
+        const uint32_t vh0 = d.z ? hy : ~0u, vh1 = d.z ? hy : ~sz;
+        const uint32_t pxy = d.x ? 0x00FF00FFu ^ sx : 0x0000FFFFu ^ sy;
+        const uint32_t plane0 = d.z ? ~sz : pxy, plane1 = d.z ? sz : pxy;
+        const uint32_t any0 = (((a0 & vl0) | (b0 & vh0)) & ul) | (((c0 & vl0) | (e0 & vh0)) & uh);
+        const uint32_t any1 = (((a1 & vl1) | (b1 & vh1)) & ul) | (((c1 & vl1) | (e1 & vh1)) & uh);
+        return ((any0 & plane0) | (any1 & plane1)) != 0u;
+    }
 }
 
 // Rank of this lane among the lanes of its wave whose bit is set in `mask`.
@@ -316,16 +370,27 @@ __device__ __forceinline__ void check_body(const SysDesc& d, uint64_t t, Substep
     }
     // Second batch: partner codes and the front plane.  CRITICAL.cu:322-323: the
     // draw is keyed by the species-local index in the reference's order.
-    uint32_t dir[SLOTS], to[SLOTS], partnerCode[SLOTS][MAXDEG], occ[SLOTS];
+    // The plane words of moves that fail the bond test are not needed.  On the
+    // byte lattice (eight times the plane bytes) and with more than two bonds
+    // (more moves fail) it pays to wait for the test and read them for the
+    // others only; with two bonds on the bit lattice the reads go out with the
+    // partners'.  us per substep, together against bonds first: 256^3 melt,
+    // uint8 13.9 against 13.2; dense star network 11.4 against 11.3; 512^3
+    // melt, bit 39.2 against 39.7.
+    constexpr bool kBondsFirst = LAT == kLatticeU8 || MAXDEG > 2;
+    constexpr int kShift = LAT == kLatticeU8 ? 3 : 6;
+    uint32_t partnerCode[SLOTS][MAXDEG];
+    Dir dir[SLOTS];
+    Move mv[SLOTS];
+    bool occ[SLOTS];
 #pragma unroll
     for (int s = 0; s < SLOTS; ++s) {
-        dir[s] = move_hash(hj[s] ^ draw.seed) % 6u;
-        const Move mv = make_move(m[s], dir[s], masks);
-        to[s] = mv.to;
+        dir[s] = dir_of_hash(move_hash(hj[s] ^ draw.seed));
+        mv[s] = make_move(m[s], dir[s], masks);
 #pragma unroll
         for (int r = 0; r < MAXDEG; ++r)
             partnerCode[s][r] = posAll[partner[s][r] != kNoNeighbor ? partner[s][r] : 0u];
-        occ[s] = plane_any<LAT == kLatticeU8 ? 3 : 6>(lattice, mv);
+        if constexpr (!kBondsFirst) occ[s] = plane_any<kShift>(lattice, m[s], dir[s], mv[s]);
     }
     if (threadIdx.x == 0) {
 #pragma unroll
@@ -339,10 +404,18 @@ __device__ __forceinline__ void check_body(const SysDesc& d, uint64_t t, Substep
         uint32_t bad = 0;
 #pragma unroll
         for (int r = 0; r < MAXDEG; ++r) {
-            const uint32_t key = bond_key(partnerCode[s][r], to[s]);
+            const uint32_t key = bond_key(partnerCode[s][r], mv[s].to);
             if (partner[s][r] != kNoNeighbor) bad |= sForbidden[key >> 5] >> (key & 31u);
         }
-        ok[s] = live[s] && !(bad & 1u) && occ[s] == 0u;
+        ok[s] = live[s] && !(bad & 1u);
+    }
+#pragma unroll
+    for (int s = 0; s < SLOTS; ++s) {
+        if constexpr (kBondsFirst) {
+            if (ok[s]) ok[s] = !plane_any<kShift>(lattice, m[s], dir[s], mv[s]);
+        } else {
+            ok[s] = ok[s] && !occ[s];
+        }
     }
 
     // Mark targets and append survivors to this workgroup's list: one LDS
@@ -363,8 +436,8 @@ __device__ __forceinline__ void check_body(const SysDesc& d, uint64_t t, Substep
 #pragma unroll
     for (int s = 0; s < SLOTS; ++s) {
         if (ok[s]) {
-            __hip_atomic_fetch_or(&T[to[s] >> 5], 1u << (to[s] & 31u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            list[waveBase + before[s] + lane_rank(mask[s])] = pack_entry(j[s] | (dir[s] << kDirShift), m[s]);
+            __hip_atomic_fetch_or(&T[mv[s].to >> 5], 1u << (mv[s].to & 31u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            list[waveBase + before[s] + lane_rank(mask[s])] = pack_entry(j[s] | (dir[s].number() << kDirShift), m[s]);
         }
     }
     __syncthreads();
@@ -399,7 +472,7 @@ __device__ __forceinline__ void add_accepted(const Launch& L, gptr<uint64_t> acc
 // of the old and new corner, and the periodic image counter on a wrap.
 template <int LAT>
 __device__ __forceinline__ void apply_move(const SysDesc& d, gptr<uint32_t> pos, gptr<uint8_t> lat, uint32_t slot,
-                                           uint32_t m, uint32_t dir, const Move& mv) {
+                                           uint32_t m, const Dir& dir, const AxisMasks& mask, const Move& mv) {
     pos[slot] = mv.to;
     if (LAT == kLatticeU8) {
         lat[m] = 0;
@@ -416,10 +489,9 @@ __device__ __forceinline__ void apply_move(const SysDesc& d, gptr<uint32_t> pos,
         if (bFrom != bTo) lat[bFrom] = 0;
         lat[bTo] = uint8_t(1u << (mv.to & 7u));
     }
-    if (mv.wraps) {
-        const uint32_t axis = dir >> 1;
-        const gptr<int32_t> img = axis == 0 ? d.imgX.global() : (axis == 1 ? d.imgY.global() : d.imgZ.global());
-        img[slot] += (dir & 1u) ? 1 : -1;
+    if (wraps(m, dir, mask)) {
+        const gptr<int32_t> img = dir.x ? d.imgX.global() : (dir.z ? d.imgZ.global() : d.imgY.global());
+        img[slot] += dir.plus ? 1 : -1;
     }
 }
 
@@ -448,11 +520,11 @@ __device__ __forceinline__ void perform_body(const SysDesc& d, const Launch& L, 
     for (uint32_t idx = threadIdx.x; idx < count; idx += B) {
         const uint64_t e = list[idx];
         const uint32_t jj = uint32_t(e) & ((1u << kDirShift) - 1u);
-        const uint32_t dir = uint32_t(e) >> kDirShift;
+        const Dir dir = dir_of_number(uint32_t(e) >> kDirShift);
         const uint32_t m = uint32_t(e >> 32);
         const Move mv = make_move(m, dir, masks);
-        if (plane_any<6>(T64, mv)) continue;
-        apply_move<LAT>(d, pos, lat, ci.slotOffset + jj, m, dir, mv);
+        if (plane_any<6>(T64, m, dir, mv)) continue;
+        apply_move<LAT>(d, pos, lat, ci.slotOffset + jj, m, dir, masks, mv);
         ++accepted;
     }
     add_accepted(L, accSlot, accepted);
@@ -523,21 +595,21 @@ __global__ __launch_bounds__(256) void k_perform_lists(SysDesc d, uint32_t k, ui
         // Entries past the count are stale: their lanes test the plane of
         // code 0 (in bounds) and drop the result.
         Move mv[DEPTH];
-        uint32_t hit[DEPTH];
-        bool valid[DEPTH];
+        Dir dir[DEPTH];
+        bool hit[DEPTH], valid[DEPTH];
 #pragma unroll
         for (int r = 0; r < DEPTH; ++r) {
             valid[r] = base + lane + uint32_t(r) * group < count;
             const uint32_t m = valid[r] ? uint32_t(e[r] >> 32) : 0u;
-            const uint32_t dir = valid[r] ? uint32_t(e[r]) >> kDirShift : 0u;
-            mv[r] = make_move(m, dir, masks);
-            hit[r] = plane_any<6>(T64, mv[r]);
+            dir[r] = dir_of_number(valid[r] ? uint32_t(e[r]) >> kDirShift : 0u);
+            mv[r] = make_move(m, dir[r], masks);
+            hit[r] = plane_any<6>(T64, m, dir[r], mv[r]);
         }
 #pragma unroll
         for (int r = 0; r < DEPTH; ++r) {
             if (!valid[r] || hit[r]) continue;
             const uint32_t jj = uint32_t(e[r]) & ((1u << kDirShift) - 1u);
-            apply_move<LAT>(d, pos, lat, slotOffset + jj, uint32_t(e[r] >> 32), uint32_t(e[r]) >> kDirShift, mv[r]);
+            apply_move<LAT>(d, pos, lat, slotOffset + jj, uint32_t(e[r] >> 32), dir[r], masks, mv[r]);
             ++accepted;
         }
     }
