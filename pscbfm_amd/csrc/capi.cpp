@@ -650,7 +650,7 @@ int pscbfm_autotune(pscbfm_updater* h, uint32_t mcs, uint32_t* block, uint32_t* 
         if (!u.initialized()) throw std::runtime_error("[autotune] initialize has not been called");
         if (mcs == 0) throw std::invalid_argument("[autotune] mcs must be positive");
         const pscbfm::TuneResult r = pscbfm::autotune_system(u.gpu(), u.layout(), u.latticeKind(), u.seed(), mcs);
-        u.setLaunchShape(r.best.block, r.best.slots);
+        u.applyTunedShape(r.best.block, r.best.slots);
         report_tune(r, block, slots, trial_ms);
     });
 }

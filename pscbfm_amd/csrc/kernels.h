@@ -44,6 +44,19 @@ hipError_t launch_perform(const SysDesc& d, uint32_t k, const LaunchShape& s, hi
 // DevState::substep += count (after a block of substeps).
 hipError_t launch_advance(DevState* state, uint32_t count, hipStream_t st);
 
+// Resident sweep (resident.hip): one workgroup runs up to `substeps` substeps
+// (to the stop point at most) of a system that fits its LDS, with at most
+// eight members of a species per thread; a later
+// launch_advance counts them.  block: 64..1024, a multiple of 64.
+constexpr uint64_t kResidentLds = 160u * 1024u;
+// Substeps of one launch: at most some 30 ms of one workgroup's work.
+constexpr uint32_t kResidentSubsteps = 4096;
+uint64_t resident_lds_bytes(const SysDesc& d);
+// Threads of the workgroup for a system on its own, or 0 where the two-pass
+// kernels are faster or its state does not fit.
+uint32_t resident_block(const SysDesc& d);
+hipError_t launch_resident(const SysDesc& d, uint32_t substeps, uint32_t block, hipStream_t st);
+
 // A batch of independent systems swept by one launch per pass.
 struct BatchLaunch {
     const SysDesc* descs;     // device table of replica descriptors

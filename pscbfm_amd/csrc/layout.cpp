@@ -180,6 +180,7 @@ SystemLayout build_layout(const SystemInput& in, const std::vector<uint8_t>* col
     std::vector<uint32_t> count(nColors, 0), maxDeg(nColors, 0);
     for (uint32_t i = 0; i < n; ++i) {
         ++count[L.color[i]];
+        L.lone = L.lone || in.bonds.degree(i) == 0;
         maxDeg[L.color[i]] = std::max(maxDeg[L.color[i]], in.bonds.degree(i));
     }
     for (uint32_t c = 0; c < nColors; ++c)

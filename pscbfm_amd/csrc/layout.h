@@ -45,6 +45,7 @@ struct SystemLayout {
     // species, and the kernels hash it instead of reading the key.
     std::vector<uint32_t> key;
     bool spatialOrder = false;
+    bool lone = false;                   // some monomer has no bond
     std::vector<int32_t> img[3];         // per slot, periodic images
     std::vector<uint32_t> nbr;           // neighbour matrices (slot ids)
     // Compressed partner ids: member j of species c has W 16-bit codes at

@@ -1,0 +1,362 @@
+// Resident sweep: one workgroup holds a whole small system in LDS and runs
+// many substeps in one launch.
+//
+// A substep of the two-pass kernels (kernels.hip) is two launches, 6 to 7 us
+// on a system of any size up to some hundred thousand monomers, nearly all of
+// it the kernel boundaries and the round trips of a few dependent loads.  Here
+// the boundary between the passes is a workgroup barrier and the gathers are
+// LDS reads, so a substep costs what its vector instructions cost on one
+// compute unit: 1.0 us for 192 members of the drawn species (two passes: 5.9),
+// then about 1.05 us per 1000 members (160 instructions per member and wave).
+//
+// LDS: the occupancy lattice and one proposal lattice (1 bit per cell, Z-curve
+// order, whatever lattice kind the system has in memory), the code of every
+// slot and the bond table as bytes.  Draw keys and partner ids stay in memory;
+// those of the next substep are read while this one's moves are resolved.
+//
+// Thread i handles members i + k*blockDim of the drawn species, k < ROUNDS, in
+// registers from the draw to the resolution: the second pass tests the same
+// plane cells with the same masks, on the proposal lattice.  (Compacting the
+// moves that pass the bond test, and the survivors, into per-wave lists cost
+// more than the idle lanes: 3.85 against 2.78 us per substep for 1850 members,
+// 7.24 against 6.19 for 4921.)  What depends on the direction alone, and the
+// plane's cells, are LDS tables: LDS has cycles to spare, the vector units not.
+//
+// The system's buffers in memory are as if the two-pass kernels had run: codes,
+// images, lattice, accepted counts, log and both proposal buffers.
+#include <algorithm>
+#include <mutex>
+#include <set>
+
+#include "kernels.h"
+#include "sweep_device.h"
+
+namespace pscbfm {
+
+namespace {
+
+// Largest species of a system on its own: us per substep, resident against two
+// passes, on 64^3: 4000 members 4.91 and 7.07, 4921 6.19 and 6.96 (byte
+// lattice 6.67 and 7.61), 6400 7.88 and 6.87.  Five rounds of 1024 threads.
+constexpr uint32_t kResidentMaxSpecies = 5120;
+
+// LDS addresses.  The kernels have no static LDS, so their dynamic LDS starts
+// at address 0; plain numbers let the compiler put the fixed parts into the
+// instructions' offset fields.
+constexpr uint32_t kBond = 0;                  // 512 bytes by bond key
+// Six direction records: masks of the axis, of u and of v, the step in dilated
+// form; two steps, one in u, one in v, the cells of the words of u-1.
+constexpr uint32_t kDirs = kBond + 512;
+constexpr uint32_t kPlanes = kDirs + 6 * 32;   // plane cells by axis and low six code bits
+constexpr uint32_t kPos = kPlanes + 192 * 8;   // codes of the slots, then occupancy, then proposals
+static_assert(kPos % 16 == 0, "16-byte LDS accesses");
+
+template <class T>
+using lptr = __attribute__((address_space(3))) T*;
+template <class T>
+__device__ __forceinline__ lptr<T> lds(uint32_t address) {
+    return (lptr<T>)(uintptr_t)address;
+}
+
+// A move from its draw to its resolution.
+struct Held {
+    uint32_t to, record;          // new corner; LDS address of the direction record
+    uint32_t q00, q02, q20, q22;  // 64-cell words of the front plane
+    uint32_t low, high;           // its cells in a word
+};
+
+// Whether a cell of the plane is set in the lattice at LDS address `words`
+// (plane_any of sweep_device.h).
+__device__ __forceinline__ bool held_any(uint32_t words, const Held& h, uint32_t su, bool z) {
+    const uint64_t w00 = *lds<const uint64_t>(words + (h.q00 << 3)), w02 = *lds<const uint64_t>(words + (h.q02 << 3));
+    const uint64_t w20 = *lds<const uint64_t>(words + (h.q20 << 3)), w22 = *lds<const uint64_t>(words + (h.q22 << 3));
+    return merged_any(w00, w02, w20, w22, PlaneMask{h.low, h.high, su, z ? 0xFFFF0000u : 0u, z ? 0xFFFF0000u : ~0u});
+}
+
+__device__ __forceinline__ uint32_t lane_value(uint32_t v, uint32_t lane) {
+    return uint32_t(__builtin_amdgcn_readlane(int32_t(v), int32_t(lane)));
+}
+
+// A substep's draw and its species' record, the same for every lane.
+struct Substep {
+    uint32_t seed, slotOffset, count, nbrOffset, pitch, degree;
+};
+
+// The next 64 substeps, one in each lane.
+struct Ahead {
+    uint32_t seed = 0, slotOffset = 0, count = 0, nbrOffset = 0, pitch = 0, degree = 0;
+    __device__ __forceinline__ void fill(const SysDesc& d, uint64_t t, gptr<const uint64_t> table, uint64_t drawBase) {
+        SubstepDraw draw;
+        if (table == nullptr) {
+            draw = substep_draw(d.seed, t, d.nColors);
+        } else {
+            const uint64_t e = table[t - drawBase];
+            draw.species = uint32_t(e);
+            draw.seed = uint32_t(e >> 32);
+        }
+        const ColorInfo ci = load_color(d.colors.global(), draw.species);
+        seed = draw.seed;
+        slotOffset = ci.slotOffset;
+        count = ci.count;
+        nbrOffset = ci.nbrOffset;
+        pitch = ci.nbrPitch;
+        degree = ci.maxDegree;
+    }
+    __device__ __forceinline__ Substep at(uint32_t i) const {
+        return {lane_value(seed, i),      lane_value(slotOffset, i), lane_value(count, i),
+                lane_value(nbrOffset, i), lane_value(pitch, i),      lane_value(degree, i)};
+    }
+};
+
+// Draw keys and partner ids of a thread's members.  A lane past the species
+// reads its last member's, a row past the species' degree the codes' own
+// buffer; both are dropped by the user.
+template <int ROUNDS, int MAXDEG>
+struct Static {
+    uint32_t key[ROUNDS], id[ROUNDS][MAXDEG];
+    __device__ __forceinline__ void load(const SysDesc& d, const Substep& s) {
+        const gptr<const uint32_t> codes = (gptr<const uint32_t>)d.pos.global() + s.slotOffset;
+        const gptr<const uint32_t> keys = d.keyed != 0u ? (gptr<const uint32_t>)d.key.global() + s.slotOffset : codes;
+        gptr<const uint32_t> row[MAXDEG];
+#pragma unroll
+        for (uint32_t r = 0; r < uint32_t(MAXDEG); ++r)
+            row[r] = r < s.degree ? (gptr<const uint32_t>)d.nbr.global() + s.nbrOffset + r * s.pitch : codes;
+#pragma unroll
+        for (uint32_t k = 0; k < uint32_t(ROUNDS); ++k) {
+            const uint32_t j = min(threadIdx.x + k * blockDim.x, s.count - 1u);
+            key[k] = keys[j];
+#pragma unroll
+            for (int r = 0; r < MAXDEG; ++r) id[k][r] = row[r][j];
+        }
+    }
+};
+
+template <int ROUNDS, int MAXDEG>
+__device__ __forceinline__ void resident_body(const SysDesc& d, uint32_t substeps) {
+    const uint32_t B = blockDim.x, tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t wave64 = uint32_t(__builtin_amdgcn_readfirstlane(int32_t(tid & ~63u)));
+    const uint32_t latWords = d.latWords;
+    const uint32_t sLat = kPos + 4u * ((d.nSlots + 3u) & ~3u), sProp = sLat + 4u * latWords;
+
+    const gptr<const u32x4> w = (gptr<const u32x4>)d.state.global();
+    const u32x4 w0 = w[0], w1 = w[1], w2 = w[2], w3 = w[3];  // DevState field order
+    const uint64_t t0 = join64(w0.x, w0.y), stopAt = join64(w0.z, w0.w);
+    if (t0 >= stopAt || substeps == 0u) return;
+    const uint32_t n = uint32_t(min(uint64_t(substeps), stopAt - t0));
+    const gptr<const uint64_t> table = (gptr<const uint64_t>)(uintptr_t(join64(w1.x, w1.y)));
+    const uint64_t drawBase = join64(w1.z, w1.w);
+    const gptr<uint32_t> log = (gptr<uint32_t>)(uintptr_t(join64(w2.x, w2.y)));
+    const uint64_t logFirst = join64(w2.z, w2.w), logCapacity = join64(w3.x, w3.y);
+    const gptr<uint64_t> accepted = (gptr<uint64_t>)(uintptr_t(join64(w3.z, w3.w)));
+
+    // Load.  The byte lattice packs to bits: four 0/1 bytes times
+    // 2^24 + 2^17 + 2^10 + 2^3 have their bits side by side in bits 24..27.
+    const gptr<uint32_t> posAll = d.pos.global();
+    for (uint32_t i = tid; i < latWords; i += B) {
+        uint32_t v = 0;
+        if (d.latticeKind == kLatticeU8) {
+            const gptr<const uint32_t> cells = (gptr<const uint32_t>)d.lattice.global() + 8u * i;
+#pragma unroll
+            for (uint32_t q = 0; q < 8u; ++q) v |= ((((cells[q] & 0x01010101u) * 0x01020408u) >> 24) & 15u) << (4u * q);
+        } else {
+            v = ((gptr<const uint32_t>)d.lattice.global())[i];
+        }
+        *lds<uint32_t>(sLat + 4u * i) = v;
+    }
+    for (uint32_t i = tid; i < d.nSlots; i += B) *lds<uint32_t>(kPos + 4u * i) = posAll[i];
+    for (uint32_t i = tid; i < 512u; i += B)
+        *lds<uint8_t>(kBond + i) = uint8_t((d.bondMask.global()[i >> 5] >> (i & 31u)) & 1u);
+    const AxisMasks masks = axis_masks(d);
+    for (uint32_t i = tid; i < 6u; i += B) {
+        const Dir dir = dir_of_number(i);
+        const uint32_t Ma = dir.x ? masks.x : (dir.z ? masks.z : masks.y), oneA = dir.x ? 1u : (dir.z ? 4u : 2u);
+        *lds<u32x4>(kDirs + 32u * i) =
+            u32x4{Ma, dir.x ? masks.y : masks.x, dir.z ? masks.y : masks.z, dir.plus ? oneA : Ma};
+        *lds<u32x4>(kDirs + 32u * i + 16u) = u32x4{dir.plus ? oneA << 3 : Ma ^ oneA, dir.x ? 2u : 1u, dir.z ? 2u : 4u,
+                                                   dir.x ? 0xFFFF0000u : 0xFF00FF00u};
+    }
+    for (uint32_t i = tid; i < 192u; i += B) {
+        const PlaneMask p = plane_mask(i & 63u, dir_of_number(2u * (i >> 6)));
+        *lds<uint64_t>(kPlanes + 8u * i) = join64(p.low, p.high);
+    }
+    uint64_t total = 0;
+
+    // Few values per thread: read one substep ahead.  Else at the substep's
+    // start, ahead of the clear and its barrier.
+    constexpr bool kReadAhead = ROUNDS * (1 + MAXDEG) <= 12;
+    Ahead ahead;
+    ahead.fill(d, t0 + min(lane, n - 1u), table, drawBase);
+    Substep s = ahead.at(0);
+    Static<ROUNDS, MAXDEG> st;
+    if constexpr (kReadAhead) st.load(d, s);
+
+    for (uint32_t step = 0; step < n; ++step) {
+        if constexpr (!kReadAhead) st.load(d, s);
+        // The last substep's proposals: read before the barrier that ended it.
+        for (uint32_t i = tid; i < latWords / 4u; i += B) *lds<u32x4>(sProp + 16u * i) = u32x4{0u, 0u, 0u, 0u};
+        __syncthreads();
+
+        Held held[ROUNDS];
+        uint32_t ok = 0;  // bit k: the move of round k stands
+#pragma unroll
+        for (uint32_t k = 0; k < uint32_t(ROUNDS); ++k) {
+            if (wave64 + k * B >= s.count) break;  // the same for the whole wave
+            const uint32_t j = tid + k * B, jj = min(j, s.count - 1u);
+            Held& h = held[k];
+            const uint32_t m = *lds<uint32_t>(kPos + 4u * (s.slotOffset + jj));
+            uint32_t code[MAXDEG];
+            // A monomer with fewer bonds tests its first one again (every
+            // monomer of a resident system has one).
+#pragma unroll
+            for (uint32_t r = 0; r < uint32_t(MAXDEG); ++r) {
+                uint32_t id = st.id[k][r];
+                if (r > 0u) id = r < s.degree && id != kNoNeighbor ? id : st.id[k][0];
+                code[r] = *lds<uint32_t>(kPos + 4u * id);
+            }
+            const uint32_t hj = d.keyed != 0u ? st.key[k] : move_hash(jj);
+            const uint32_t rn = move_hash(hj ^ s.seed);
+            const Dir dir = dir_of_hash(rn);
+            const uint32_t axis = dir.x ? 0u : (dir.z ? 128u : 64u);
+            h.record = axis | (rn & 1u) << 5;
+            const u32x4 ra = *lds<const u32x4>(kDirs + h.record), rb = *lds<const u32x4>(kDirs + h.record + 16u);
+            const uint64_t cells = *lds<const uint64_t>(kPlanes + 8u * (axis | (m & 63u)));
+            h.low = uint32_t(cells);
+            h.high = uint32_t(cells >> 32);
+            const uint32_t ta = m | ~ra.x, tu = m | ~ra.y, tv = m | ~ra.z;
+            h.to = (m & ~ra.x) | ((ta + ra.w) & ra.x);
+            uint32_t bad = 0;
+#pragma unroll
+            for (int r = 0; r < MAXDEG; ++r) bad |= *lds<const uint8_t>(kBond + bond_key(code[r], h.to));
+            const uint32_t fa = (ta + rb.x) & ra.x;
+            const uint32_t u0 = fa | ((tu + ra.y) & ra.y), u2 = fa | ((tu + rb.y) & ra.y);
+            const uint32_t v0 = (tv + ra.z) & ra.z, v2 = (tv + rb.z) & ra.z;
+            h.q00 = __builtin_amdgcn_ubfe(u0 | v0, 6, 26);
+            h.q02 = __builtin_amdgcn_ubfe(u0 | v2, 6, 26);
+            h.q20 = __builtin_amdgcn_ubfe(u2 | v0, 6, 26);
+            h.q22 = __builtin_amdgcn_ubfe(u2 | v2, 6, 26);
+            const bool blocked = held_any(sLat, h, rb.w, dir.z);
+            if (j < s.count && bad == 0u && !blocked) {
+                ok |= 1u << k;
+                atomicOr((uint32_t*)lds<uint32_t>(sProp + 4u * (h.to >> 5)), 1u << (h.to & 31u));
+            }
+        }
+
+        const uint32_t slot0 = s.slotOffset + tid;
+        if (step + 1u < n) {
+            if (((step + 1u) & 63u) == 0u) ahead.fill(d, t0 + min(step + 1u + lane, n - 1u), table, drawBase);
+            s = ahead.at((step + 1u) & 63u);
+            if constexpr (kReadAhead) st.load(d, s);
+        }
+        __syncthreads();
+
+        uint32_t moved = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < uint32_t(ROUNDS); ++k) {
+            const Held& h = held[k];
+            bool go = (ok >> k & 1u) != 0u;
+            if (__ballot(go) == 0u) continue;
+            if (go) {
+                go = !held_any(sProp, h, h.record < 64u ? 0xFFFF0000u : 0xFF00FF00u, h.record >= 128u);
+                if (go) {
+                    const uint32_t slot = slot0 + k * B, m = *lds<uint32_t>(kPos + 4u * slot);
+                    *lds<uint32_t>(kPos + 4u * slot) = h.to;
+                    // one writer per byte, as in apply_move (kernels.hip)
+                    const uint32_t bFrom = m >> 3, bTo = h.to >> 3;
+                    if (bFrom != bTo) *lds<uint8_t>(sLat + bFrom) = 0;
+                    *lds<uint8_t>(sLat + bTo) = uint8_t(1u << (h.to & 7u));
+                    // a step up has the larger code unless it wraps, a step down the smaller
+                    const bool plus = (h.record & 32u) != 0u;
+                    if ((h.to > m) != plus) {
+                        const gptr<int32_t> img = h.record < 64u    ? d.imgX.global()
+                                                  : h.record < 128u ? d.imgY.global()
+                                                                    : d.imgZ.global();
+                        __hip_atomic_fetch_add(&img[slot], plus ? 1 : -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    }
+                }
+            }
+            moved += uint32_t(__popcll(__ballot(go)));
+        }
+        total += moved;
+        if (log != nullptr && lane == 0u && moved != 0u) {
+            const uint64_t idx = t0 + step - logFirst;
+            if (idx < logCapacity)
+                __hip_atomic_fetch_add(&log[idx], moved, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        __syncthreads();
+    }
+
+    // Store.
+    if (lane == 0u && total != 0u)
+        __hip_atomic_fetch_add(&accepted[0], total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (uint32_t i = tid; i < d.nSlots; i += B) posAll[i] = *lds<uint32_t>(kPos + 4u * i);
+    const gptr<uint32_t> marks = d.proposal.global();
+    const uint32_t last = uint32_t((t0 + n - 1u) & 1u);
+    for (uint32_t i = tid; i < latWords; i += B) {
+        const uint32_t v = *lds<uint32_t>(sLat + 4u * i);
+        if (d.latticeKind == kLatticeU8) {
+            const gptr<uint32_t> cells = (gptr<uint32_t>)d.lattice.global() + 8u * i;
+#pragma unroll
+            for (uint32_t q = 0; q < 8u; ++q) cells[q] = (((v >> (4u * q)) & 15u) * 0x00204081u) & 0x01010101u;
+        } else {
+            ((gptr<uint32_t>)d.lattice.global())[i] = v;
+        }
+        marks[last * latWords + i] = *lds<uint32_t>(sProp + 4u * i);
+        marks[(last ^ 1u) * latWords + i] = 0u;
+    }
+}
+
+template <int ROUNDS, int MAXDEG>
+__global__ __launch_bounds__(1024) void k_resident(SysDesc d, uint32_t substeps) {
+    resident_body<ROUNDS, MAXDEG>(d, substeps);
+}
+
+using ResidentKernel = void (*)(SysDesc, uint32_t);
+template <int ROUNDS>
+ResidentKernel resident_by_degree(uint32_t maxDegree) {
+    return maxDegree <= 2u ? k_resident<ROUNDS, 2> : (maxDegree <= 4u ? k_resident<ROUNDS, 4> : k_resident<ROUNDS, 8>);
+}
+ResidentKernel resident_kernel(uint32_t rounds, uint32_t maxDegree) {
+    if (rounds <= 1u) return resident_by_degree<1>(maxDegree);
+    if (rounds <= 2u) return resident_by_degree<2>(maxDegree);
+    if (rounds <= 3u) return resident_by_degree<3>(maxDegree);
+    if (rounds <= 4u) return resident_by_degree<4>(maxDegree);
+    if (rounds <= 5u) return resident_by_degree<5>(maxDegree);
+    if (rounds <= 6u) return resident_by_degree<6>(maxDegree);
+    return resident_by_degree<8>(maxDegree);
+}
+
+// Dynamic LDS beyond 64 KiB is granted per kernel and device, once.
+hipError_t allow_full_lds(const void* kernel) {
+    static std::mutex mu;
+    static std::set<std::pair<int, const void*>> done;
+    int dev = 0;
+    hipError_t err = hipGetDevice(&dev);
+    if (err != hipSuccess) return err;
+    std::lock_guard<std::mutex> lock(mu);
+    if (done.count({dev, kernel})) return hipSuccess;
+    err = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, int(kResidentLds));
+    if (err == hipSuccess) done.insert({dev, kernel});
+    return err;
+}
+
+}  // namespace
+
+uint64_t resident_lds_bytes(const SysDesc& d) {
+    return kPos + 4ull * ((uint64_t(d.nSlots) + 3u) & ~3ull) + 8ull * d.latWords;
+}
+
+uint32_t resident_block(const SysDesc& d) {
+    if (d.maxColorCount == 0u || d.maxColorCount > kResidentMaxSpecies || d.lone != 0u) return 0u;
+    const uint32_t block = std::min((d.maxColorCount + 63u) / 64u * 64u, 1024u);
+    return resident_lds_bytes(d) <= kResidentLds ? block : 0u;
+}
+
+hipError_t launch_resident(const SysDesc& d, uint32_t substeps, uint32_t block, hipStream_t st) {
+    const ResidentKernel kernel = resident_kernel((d.maxColorCount + block - 1u) / block, d.maxDegree);
+    const hipError_t err = allow_full_lds(reinterpret_cast<const void*>(kernel));
+    if (err != hipSuccess) return err;
+    hipLaunchKernelGGL(kernel, dim3(1), dim3(block), uint32_t(resident_lds_bytes(d)), st, d, substeps);
+    return hipGetLastError();
+}
+
+}  // namespace pscbfm

@@ -214,6 +214,14 @@ void Updater::setLaunchShape(uint32_t block, uint32_t slots) {
         throw std::invalid_argument("[setLaunchShape] slots per thread must be 1, 2 or 4");
     blockOverride_ = block;
     slotsOverride_ = slots;
+    shapePinned_ = block != 0 || slots != 0;
+    if (initialized_) applyLaunchShape();
+}
+
+void Updater::applyTunedShape(uint32_t block, uint32_t slots) {
+    const bool pinned = shapePinned_;
+    setLaunchShape(block, slots);
+    shapePinned_ = pinned;
     if (initialized_) applyLaunchShape();
 }
 
@@ -271,6 +279,8 @@ void Updater::applyLaunchShape() {
     shape_.grid = grid_for(layout_.maxColorCount, shape_.block * shape_.slots);
     shape_.clearPass = clearPassOverride_ ? clearPassOverride_ : automatic_clear_pass(layout_, latticeKind_);
     performGridMax_ = std::max(performGridMax_, shape_.passTwoGrid());
+    const bool pinned = shapePinned_ || performOverride_ || walkGroupOverride_ || clearPassOverride_;
+    residentBlock_ = pinned ? 0u : resident_block(dev_.desc);
     dropGraphs();
 }
 
@@ -482,6 +492,7 @@ void Updater::prepareGraphs(int32_t nMCS) {
         throw std::runtime_error("[prepareGraphs] initialize has not been called");
     if (nMCS <= 0 || nColors() == 0 || n_ == 0) return;
     hip_check(hipSetDevice(gpu_), "hipSetDevice");
+    if (residentBlock_) return;  // runs without graphs
     const uint64_t S = uint64_t(nMCS) * nColors();
     const uint64_t drawCap = drawChunk_ ? std::min(drawChunk_, kMaxDrawSubsteps) : kMaxDrawSubsteps;
     const uint64_t chunk = r250Mode_ ? std::max<uint64_t>(1u, drawCap / nColors()) * nColors() : S;
@@ -565,8 +576,9 @@ void Updater::runChunk(uint64_t S, uint32_t* log, bool profile, bool useGraph, v
     // Every graph the replays need is captured, instantiated and uploaded
     // first: before the start event, so that the timed window holds device
     // work only, and before this run enqueues anything on the stream.
+    const bool resident = residentBlock_ != 0 && !profile;
     GraphPlan plan;
-    if (!profile && useGraph) plan = planGraphs(S);
+    if (!profile && useGraph && !resident) plan = planGraphs(S);
 
     // Species and kernel seed of every substep, as the kernels will draw them.
     std::vector<uint32_t> species(S);
@@ -642,7 +654,13 @@ void Updater::runChunk(uint64_t S, uint32_t* log, bool profile, bool useGraph, v
         }
     } else {
         uint64_t left = S;
-        if (useGraph) {
+        while (resident && left > 0) {
+            const uint32_t part = uint32_t(std::min<uint64_t>(left, kResidentSubsteps));
+            hip_check(launch_resident(dev_.desc, part, residentBlock_, stream_), "launch resident sweep");
+            hip_check(launch_advance(dev_.desc.state, part, stream_), "launch advance");
+            left -= part;
+        }
+        if (useGraph && left > 0) {
             // the bulk graph, then the remainder's graph, so every substep
             // runs from a graph
             for (uint64_t r = 0; r < plan.bulkCount; ++r)

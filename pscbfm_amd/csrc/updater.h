@@ -82,7 +82,13 @@ public:
     void setCheckOnInitialize(bool on) { checkOnInit_ = on; }
     void setColors(const uint8_t* colors, uint32_t n);
     // Threads per workgroup (0 = 256) and monomers per pass-1 thread (0 = 2).
+    // A system small enough for the resident sweep (resident_block, kernels.h)
+    // runs that instead, unless this, setPerformBlock, setPerformWalk or
+    // setClearPass states a shape of the two-pass kernels.
     void setLaunchShape(uint32_t block, uint32_t slots);
+    // The autotuner's choice: the shape of the two-pass kernels where they
+    // run, without pinning a small system to them as setLaunchShape does.
+    void applyTunedShape(uint32_t block, uint32_t slots);
     // Substeps of the bulk graph (0 = nColors * max(1, 256 / nColors)); a
     // run replays it, then one graph of the remaining substeps.
     // invalid_argument above kMaxGraphChunk (each substep is two kernel nodes).
@@ -227,6 +233,8 @@ private:
     hipStream_t stream_ = nullptr;
     DeviceSystem dev_;
     LaunchShape shape_;
+    bool shapePinned_ = false;    // setLaunchShape stated a shape
+    uint32_t residentBlock_ = 0;  // threads of the resident sweep's workgroup; 0: two-pass kernels
     std::map<uint32_t, hipGraphExec_t> graphs_;  // by substeps per replay
     uint32_t performGridMax_ = 0;  // largest pass-2 grid used (entries of acceptedByBlock)
     uint64_t substep_ = 0;

@@ -1,0 +1,119 @@
+"""The resident sweep (one workgroup, many substeps per launch) against the CPU
+oracle and the two-pass kernels, which setLaunchShape pins.
+
+All results are whole numbers, so every comparison is exact.  Sizes are chosen
+around the workgroup's rounds: a species of 64 and 65 members (one wave and
+two), 1024 and 1025 (one round and two), and 5120 and 5121 (the largest that
+runs resident and the first that does not)."""
+import numpy as np
+import pytest
+
+import oracle
+import pscbfm_amd as P
+from helpers import GOLDEN, chains, make_updater, ordered_chains, oracle_for, stars
+
+pytestmark = pytest.mark.gpu
+
+KINDS = [P.LATTICE_BIT, P.LATTICE_U8]
+
+
+def _dimers(box, n):
+    """n ordered dimers: two species of exactly n members."""
+    return ordered_chains(box, n, 2)
+
+
+SYSTEMS = {
+    "one_wave": lambda: _dimers((32, 32, 32), 64),
+    "two_waves": lambda: _dimers((32, 32, 32), 65),
+    "one_round": lambda: _dimers((64, 32, 32), 1024),
+    "two_rounds": lambda: _dimers((64, 32, 32), 1025),
+    "five_rounds": lambda: _dimers((64, 64, 64), 5120),
+    "too_large": lambda: _dimers((64, 64, 64), 5121),
+    "smallest_box": lambda: chains((8, 8, 8), 2, 5, seed=3),
+    "flat_box": lambda: chains((64, 16, 8), 9, 21, seed=4),
+    "network": lambda: stars((64, 64, 64), 60, 4, 7, seed=5),
+    "eight_arms": lambda: stars((64, 32, 64), 40, 8, 6, seed=6),
+    "lone_monomers": lambda: chains((32, 32, 32), 100, 1, seed=7),
+}
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("name", sorted(SYSTEMS))
+def test_resident_equals_oracle_and_two_pass(name, kind):
+    s = SYSTEMS[name]()
+    print(f"{name}: {s.n} monomers, kind {kind}", flush=True)
+    cells = int(np.prod(s.box))
+    seen = []
+    for shape, spatial in (((0, 0), None), ((0, 0), True), ((0, 0), False), ((256, 2), None)):
+        u = make_updater(s, 11, kind, block=shape[0], slots=shape[1], spatial=spatial)
+        colors = u.colors(s.n)
+        logs = [u.run(m, log=True)[1] for m in (1, 70, 3)]  # the second crosses 64 substeps
+        seen.append((np.concatenate(logs), u.getPositions(s.n), u.downloadLattice(cells), u.proposalBits(),
+                     u.counters()))
+        u.cleanup()
+    o = oracle_for(s, colors, 11)
+    _, olog = o.run(0, 74 * (int(colors.max()) + 1))
+    assert np.array_equal(seen[0][0], olog) and np.array_equal(seen[0][1], o.xyz)
+    for other in seen[1:]:
+        assert all(np.array_equal(a, b) for a, b in zip(seen[0], other))
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_both_paths_continue_each_other(kind):
+    """Resident, two-pass and eager runs of one handle follow one trajectory:
+    each leaves the buffers the other expects, whatever the substeps' parity."""
+    s = chains((32, 64, 32), 60, 13, seed=8)
+    u = make_updater(s, 21, kind)
+    colors = u.colors(s.n)
+    nc = int(colors.max()) + 1
+    logs = []
+    plan = [(3, (0, 0), False), (2, (128, 1), False), (1, (0, 0), False), (4, (0, 0), True), (2, (256, 2), False),
+            (5, (0, 0), False)]
+    for m, shape, profile in plan:
+        u.setLaunchShape(*shape)
+        logs.append(u.run(m, log=True, profile=profile)[1])
+        u.setLaunchShape(0, 0)
+    o = oracle_for(s, colors, 21)
+    _, olog = o.run(0, 17 * nc)
+    assert np.array_equal(np.concatenate(logs), olog)
+    assert np.array_equal(u.getPositions(s.n), o.xyz)
+    u.cleanup()
+
+
+def test_r250_draws_and_the_launch_limit():
+    """Explicit draws, and a run longer than one launch covers."""
+    s = chains((32, 32, 32), 20, 16, seed=9)
+    u = make_updater(s, 1)
+    u.loadR250SeedFile(GOLDEN / "resultNormPscBFM.seeds", 2)
+    u.setDrawChunk(300)
+    colors = u.colors(s.n)
+    nc = int(colors.max()) + 1
+    mcs = 4200 // nc + 1
+    _, log = u.run(mcs, log=True)
+    r = oracle.R250.from_seed_file(GOLDEN / "resultNormPscBFM.seeds")
+    r.rand32(), r.rand32()
+    o = oracle_for(s, colors, 0)
+    o.draws = r.substep_draws(mcs * nc, nc)
+    _, olog = o.run(0, mcs * nc)
+    assert np.array_equal(log, olog) and np.array_equal(u.getPositions(s.n), o.xyz)
+    u.cleanup()
+
+    v = make_updater(s, 5)
+    w = make_updater(s, 5, block=256, slots=2)
+    (sv, _), (sw, _) = v.run(4200), w.run(4200)
+    assert (sv.accepted, sv.attempted, sv.substeps) == (sw.accepted, sw.attempted, sw.substeps)
+    assert sv.substeps > 4096 and np.array_equal(v.getPositions(s.n), w.getPositions(s.n))
+    v.cleanup()
+    w.cleanup()
+
+
+def test_tuned_small_system_stays_exact():
+    """The autotuner's choice does not pin a small system to the two-pass kernels' results only."""
+    s = chains((32, 32, 32), 24, 16, seed=10)
+    a, b = make_updater(s, 3), make_updater(s, 3, block=64, slots=1)
+    a.autotune(2)
+    a.run(20)
+    b.run(20)
+    assert np.array_equal(a.getPositions(s.n), b.getPositions(s.n))
+    a.cleanup()
+    b.cleanup()
