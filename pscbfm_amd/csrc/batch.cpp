@@ -21,6 +21,7 @@
 namespace pscbfm {
 
 namespace {
+constexpr size_t kComputeUnits = 256;
 constexpr uint32_t kSpreadTiles = 64;  // replicas with at least this many workgroups use every XCD
 
 uint32_t degree_bucket(uint32_t d) { return d <= 2 ? 2u : (d <= 4 ? 4u : 8u); }
@@ -47,10 +48,16 @@ Batch::Batch(int gpu, uint32_t latticeKind, uint32_t tileCapacity, uint32_t repl
     shape_.performBlock = default_perform_block(block);
     shape_.grid = tileCap_;
     hip_check(hipSetDevice(gpu_), "hipSetDevice");
+    // created together: the runtime deals its hardware queues out in turn, and
+    // streams on one queue would not overlap
     hip_check(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking), "hipStreamCreate");
+    for (hipStream_t& s : side_) hip_check(hipStreamCreateWithFlags(&s, hipStreamNonBlocking), "hipStreamCreate");
+    for (hipEvent_t& e : sideDone_) hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
+    hip_check(hipEventCreateWithFlags(&fork_, hipEventDisableTiming), "hipEventCreate");
     hip_check(hipMalloc(&dDescs_, sizeof(SysDesc) * replicaCap_), "hipMalloc descs");
     hip_check(hipMalloc(&dStops_, sizeof(uint64_t) * replicaCap_), "hipMalloc stops");
     hip_check(hipMalloc(&dGather_, sizeof(uint64_t) * 3 * replicaCap_), "hipMalloc gather");
+    hip_check(hipMalloc(&dResident_, sizeof(uint32_t) * replicaCap_), "hipMalloc resident ids");
     jobsCap_ = std::max<uint32_t>(replicaCap_, 64u);
     hip_check(hipMalloc(&dJobs_, sizeof(UnfoldJob) * jobsCap_), "hipMalloc unfold jobs");
     descs_.assign(replicaCap_, SysDesc{});
@@ -91,10 +98,15 @@ void Batch::growTiles(uint32_t needed) {
 Batch::~Batch() {
     if (stream_) (void)hipStreamSynchronize(stream_);
     dropGraphs();
+    for (hipStream_t s : side_)
+        if (s) (void)hipStreamDestroy(s);
+    for (hipEvent_t e : sideDone_)
+        if (e) (void)hipEventDestroy(e);
+    if (fork_) (void)hipEventDestroy(fork_);
     for (auto& r : replicas_) r.dev.reset();
     for (void* p : {static_cast<void*>(dDescs_), static_cast<void*>(dTiles_), static_cast<void*>(dLists_),
                     static_cast<void*>(dListCounts_), static_cast<void*>(dStops_), static_cast<void*>(dGather_),
-                    static_cast<void*>(dJobs_), static_cast<void*>(dXyz_)})
+                    static_cast<void*>(dJobs_), static_cast<void*>(dXyz_), static_cast<void*>(dResident_)})
         if (p) (void)hipFree(p);
     if (hXyz_) (void)hipHostFree(hXyz_);
     if (stream_) (void)hipStreamDestroy(stream_);
@@ -104,6 +116,8 @@ void Batch::setPerformBlock(uint32_t block) {
     if (block != 0 && (block % 64 != 0 || block > 256)) throw std::invalid_argument("perform block must be 64..256, multiple of 64");
     hip_check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
     shape_.performBlock = block ? block : default_perform_block(shape_.block);
+    pinned_ = block != 0;
+    tablesDirty_ = true;
     dropGraphs();
 }
 
@@ -120,6 +134,133 @@ void Batch::reserveReadBack(uint64_t monomers) {
     hip_check(hipMalloc(&dXyz_, cap * 12), "hipMalloc read-back");
     hip_check(hipHostMalloc(reinterpret_cast<void**>(&hXyz_), cap * 12, hipHostMallocDefault), "hipHostMalloc read-back");
     xyzCap_ = cap;
+}
+
+// Workgroup slots of a replica that the two-pass kernels sweep.
+void Batch::takeTiles(uint32_t id) {
+    Replica& r = replicas_[id];
+    const uint32_t nT = r.info.tiles;
+    // one XCD for a small replica, all XCDs for a large one
+    r.tileSlots.reserve(nT);
+    if (nT >= kSpreadTiles) {
+        uint32_t x = 0;
+        while (r.tileSlots.size() < nT) {
+            for (uint32_t tries = 0; tries < 8 && freeSlots_[x].empty(); ++tries) x = (x + 1) % 8;
+            r.tileSlots.push_back(freeSlots_[x].back());
+            freeSlots_[x].pop_back();
+            x = (x + 1) % 8;
+        }
+    } else {
+        while (r.tileSlots.size() < nT) {
+            uint32_t best = 0;
+            for (uint32_t x = 1; x < 8; ++x)
+                if (freeSlots_[x].size() > freeSlots_[best].size()) best = x;
+            const uint32_t take = std::min<uint32_t>(nT - uint32_t(r.tileSlots.size()), uint32_t(freeSlots_[best].size()));
+            for (uint32_t k = 0; k < take; ++k) {
+                r.tileSlots.push_back(freeSlots_[best].back());
+                freeSlots_[best].pop_back();
+            }
+        }
+    }
+    for (uint32_t c = 0; c < nT; ++c) tiles_[r.tileSlots[c]] = Tile{id, c, nT, 0};
+}
+
+void Batch::releaseTiles(uint32_t id) {
+    Replica& r = replicas_[id];
+    if (r.tileSlots.empty()) return;
+    for (uint32_t w : r.tileSlots) {
+        tiles_[w] = Tile{kNoReplica, 0, 0, 0};
+        freeSlots_[w % 8].push_back(w);
+    }
+    for (auto& f : freeSlots_) std::sort(f.begin(), f.end(), std::greater<uint32_t>());
+    r.tileSlots.clear();
+}
+
+// Which replicas the resident sweep takes, and their launches.  A replica
+// that fits a workgroup's LDS takes its own compute unit.  A large one then
+// needs longer per substep than the two-pass kernels would alone, so it does
+// so only when the replicas that must use those kernels need longer still:
+// they were measured at about 7 us per substep and 75 members of the drawn
+// species per ns on the replica mix.
+void Batch::assignPaths() {
+    double twoPassUs = 7.0;
+    for (uint32_t i = 0; i < replicaCap_; ++i)
+        if (replicas_[i].live && (pinned_ || !resident_fits(descs_[i])))
+            twoPassUs += double(replicas_[i].info.nMonomers) / std::max(1u, replicas_[i].info.nColors) / 75e3;
+    std::vector<std::pair<ResidentClass, uint32_t>> chosen;
+    twoPassUsed_ = 0;
+    for (uint32_t i = 0; i < replicaCap_; ++i) {
+        if (!replicas_[i].live) continue;
+        SysDesc& d = descs_[i];
+        const bool resident = !pinned_ && resident_fits(d) && (resident_always(d) || resident_substep_us(d) <= twoPassUs);
+        d.resident = resident ? 1u : 0u;
+        if (resident) {
+            releaseTiles(i);
+            ResidentClass c;
+            c.lds = uint32_t(resident_lds_bytes(d));
+            c.maxDegree = d.maxDegree;
+            chosen.emplace_back(c, i);
+        } else {
+            if (replicas_[i].tileSlots.empty()) takeTiles(i);
+            ++twoPassUsed_;
+        }
+    }
+    // At most two launches, one to a stream, since launches of one stream wait
+    // for each other.  Up to one replica per compute unit, each gets a full
+    // workgroup; beyond that small ones take small workgroups, several to a
+    // compute unit.  Large replicas first.
+    const bool few = chosen.size() <= kComputeUnits;
+    for (auto& [c, id] : chosen) {
+        const uint32_t species = descs_[id].maxColorCount;
+        const bool small = !few && species <= 1024u && c.lds <= kResidentLds / 4u;
+        c.block = small ? 256u : 1024u;
+    }
+    auto key = [&](const ResidentClass& c) { return c.block; };
+    std::sort(chosen.begin(), chosen.end(), [&](const auto& a, const auto& b) {
+        const auto ka = key(a.first), kb = key(b.first);
+        if (ka != kb) return ka > kb;
+        const uint32_t na = descs_[a.second].maxColorCount, nb = descs_[b.second].maxColorCount;
+        return na != nb ? na > nb : a.second < b.second;
+    });
+    classes_.clear();
+    residentIds_.clear();
+    for (const auto& [c, id] : chosen) {
+        if (classes_.empty() || key(classes_.back()) != key(c)) {
+            classes_.push_back(c);
+            classes_.back().first = uint32_t(residentIds_.size());
+            classes_.back().count = 0;
+        }
+        ResidentClass& q = classes_.back();
+        q.lds = std::max(q.lds, c.lds);
+        q.maxDegree = std::max(q.maxDegree, c.maxDegree);
+        q.rounds = std::max(q.rounds, (descs_[id].maxColorCount + q.block - 1u) / q.block);
+        ++q.count;
+        residentIds_.push_back(id);
+    }
+}
+
+// The resident launches of `substeps` substeps, beside whatever stream_ gets
+// next; join() makes stream_ wait for them.
+void Batch::launchResident(uint64_t substeps) {
+    if (classes_.empty()) return;
+    hip_check(hipEventRecord(fork_, stream_), "hipEventRecord");
+    for (size_t q = 0; q < classes_.size(); ++q)
+        hip_check(hipStreamWaitEvent(side_[q], fork_, 0), "hipStreamWaitEvent");
+    for (size_t k = 0; k < classes_.size(); ++k)
+        for (uint64_t left = substeps; left > 0;) {
+            const uint32_t part = uint32_t(std::min<uint64_t>(left, kResidentSubsteps));
+            hip_check(launch_resident_batch(dDescs_, dResident_, classes_[k], part, side_[k]),
+                      "launch resident sweep");
+            left -= part;
+        }
+}
+
+void Batch::joinResident() {
+    if (classes_.empty()) return;
+    for (size_t q = 0; q < classes_.size(); ++q) {
+        hip_check(hipEventRecord(sideDone_[q], side_[q]), "hipEventRecord");
+        hip_check(hipStreamWaitEvent(stream_, sideDone_[q], 0), "hipStreamWaitEvent");
+    }
 }
 
 uint32_t Batch::tilesNeeded(const SystemLayout& L) const {
@@ -154,29 +295,6 @@ uint32_t Batch::add(const SystemLayout& L, uint64_t seed, uint64_t startMcs) {
     st.stopAt = start;  // idle until a target is set
     r.dev->writeState(st, stream_);
 
-    // Workgroup slots: one XCD for a small replica, all XCDs for a large one.
-    r.tileSlots.reserve(nT);
-    if (nT >= kSpreadTiles) {
-        uint32_t x = 0;
-        while (r.tileSlots.size() < nT) {
-            for (uint32_t tries = 0; tries < 8 && freeSlots_[x].empty(); ++tries) x = (x + 1) % 8;
-            r.tileSlots.push_back(freeSlots_[x].back());
-            freeSlots_[x].pop_back();
-            x = (x + 1) % 8;
-        }
-    } else {
-        while (r.tileSlots.size() < nT) {
-            uint32_t best = 0;
-            for (uint32_t x = 1; x < 8; ++x)
-                if (freeSlots_[x].size() > freeSlots_[best].size()) best = x;
-            const uint32_t take = std::min<uint32_t>(nT - uint32_t(r.tileSlots.size()), uint32_t(freeSlots_[best].size()));
-            for (uint32_t k = 0; k < take; ++k) {
-                r.tileSlots.push_back(freeSlots_[best].back());
-                freeSlots_[best].pop_back();
-            }
-        }
-    }
-    for (uint32_t c = 0; c < nT; ++c) tiles_[r.tileSlots[c]] = Tile{id, c, nT, 0};
     usedTiles_ += nT;
     descs_[id] = r.dev->desc;
     r.live = true;
@@ -208,12 +326,9 @@ void Batch::remove(uint32_t id) {
     if (id >= replicaCap_ || !replicas_[id].live) throw std::invalid_argument("batch: no such replica");
     hip_check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
     Replica& r = replicas_[id];
-    for (uint32_t w : r.tileSlots) {
-        tiles_[w] = Tile{kNoReplica, 0, 0, 0};
-        freeSlots_[w % 8].push_back(w);
-    }
-    for (auto& f : freeSlots_) std::sort(f.begin(), f.end(), std::greater<uint32_t>());
-    usedTiles_ -= uint32_t(r.tileSlots.size());
+    releaseTiles(id);
+    usedTiles_ -= r.info.tiles;
+    r.live = false;
     descs_[id] = SysDesc{};
     // the tables must not point at freed memory when the next launch runs
     tablesDirty_ = true;
@@ -233,10 +348,15 @@ void Batch::setTarget(uint32_t id, uint64_t nMCS) {
 
 void Batch::uploadTables() {
     if (tablesDirty_) {
+        assignPaths();
         hip_check(hipMemcpyAsync(dDescs_, descs_.data(), sizeof(SysDesc) * replicaCap_, hipMemcpyHostToDevice, stream_),
                   "descs H2D");
         hip_check(hipMemcpyAsync(dTiles_, tiles_.data(), sizeof(Tile) * tileCap_, hipMemcpyHostToDevice, stream_),
                   "tiles H2D");
+        if (!residentIds_.empty())
+            hip_check(hipMemcpyAsync(dResident_, residentIds_.data(), sizeof(uint32_t) * residentIds_.size(),
+                                     hipMemcpyHostToDevice, stream_),
+                      "resident ids H2D");
         // the host tables may change as soon as this returns
         hip_check(hipStreamSynchronize(stream_), "sync tables");
         tablesDirty_ = false;
@@ -298,6 +418,7 @@ hipGraphExec_t Batch::graphFor(uint32_t grid, uint32_t substeps) {
 
 Batch::GraphPlan Batch::planGraphs(uint64_t substeps) {
     GraphPlan p;
+    if (twoPassUsed_ == 0) return p;
     const uint32_t grid = activeGrid_;
     p.bulkCount = substeps / kGraphSubsteps;
     if (p.bulkCount) p.bulk = graphFor(grid, kGraphSubsteps);
@@ -312,8 +433,10 @@ Batch::GraphPlan Batch::planGraphs(uint64_t substeps) {
 }
 
 void Batch::enqueue(const GraphPlan& plan, uint64_t substeps) {
+    launchResident(substeps);
     for (uint64_t r = 0; r < plan.bulkCount; ++r) hip_check(hipGraphLaunch(plan.bulk, stream_), "hipGraphLaunch");
     for (hipGraphExec_t g : plan.tail) hip_check(hipGraphLaunch(g, stream_), "hipGraphLaunch");
+    joinResident();
     launched_ += substeps;
 }
 
@@ -459,7 +582,7 @@ uint32_t Batch::liveReplicas() const {
 uint64_t Batch::deviceBytes() const {
     uint64_t b = sizeof(SysDesc) * uint64_t(replicaCap_) + sizeof(Tile) * uint64_t(tileCap_) +
                  sizeof(uint2) * uint64_t(tileCap_) * shape_.block * shape_.slots + 4ull * tileCap_ +
-                 32ull * replicaCap_ + sizeof(UnfoldJob) * uint64_t(jobsCap_) + 12 * xyzCap_;
+                 36ull * replicaCap_ + sizeof(UnfoldJob) * uint64_t(jobsCap_) + 12 * xyzCap_;
     for (const auto& r : replicas_)
         if (r.live) b += r.dev->bytes;
     return b;

@@ -75,7 +75,8 @@ public:
     uint32_t replicaCapacity() const { return replicaCap_; }
     uint64_t deviceBytes() const;
     const LaunchShape& shape() const { return shape_; }
-    // Pass-2 threads per workgroup (0 = the pass-1 block).
+    // Pass-2 threads per workgroup (0 = automatic).  A stated value also keeps
+    // every replica on the two-pass kernels.
     void setPerformBlock(uint32_t block);
     uint64_t launchedSubsteps() const { return launched_; }
 
@@ -85,11 +86,16 @@ private:
         SystemLayout layout;
         std::unique_ptr<DeviceSystem> dev;
         uint64_t seed = 0;
-        std::vector<uint32_t> tileSlots;
+        std::vector<uint32_t> tileSlots;  // workgroups; none while the resident sweep has the replica
         BatchReplicaInfo info;
         uint64_t pendingStop = 0;
     };
     void uploadTables();
+    void assignPaths();
+    void takeTiles(uint32_t id);
+    void releaseTiles(uint32_t id);
+    void launchResident(uint64_t substeps);
+    void joinResident();
     // Captured graph of `substeps` substeps over workgroups [0, grid) plus
     // their counter advance, instantiated and uploaded on first use.
     hipGraphExec_t graphFor(uint32_t grid, uint32_t substeps);
@@ -125,7 +131,17 @@ private:
     std::vector<Tile> tiles_;
     std::vector<std::vector<uint32_t>> freeSlots_;  // per XCD
     std::vector<Replica> replicas_;
-    uint32_t usedTiles_ = 0;
+    uint32_t usedTiles_ = 0;  // of every live replica, whichever kernels sweep it
+    // Resident sweep: replicas by launch, and the streams the launches run on
+    // beside the two-pass kernels.
+    bool pinned_ = false;
+    uint32_t twoPassUsed_ = 0;  // live replicas on the two-pass kernels
+    std::vector<ResidentClass> classes_;
+    std::vector<uint32_t> residentIds_;
+    uint32_t* dResident_ = nullptr;
+    hipStream_t side_[2] = {};
+    hipEvent_t sideDone_[2] = {};
+    hipEvent_t fork_ = nullptr;
     bool growable_ = false;
     bool tablesDirty_ = true;
     bool stopsDirty_ = false;

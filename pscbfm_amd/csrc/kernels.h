@@ -46,16 +46,33 @@ hipError_t launch_advance(DevState* state, uint32_t count, hipStream_t st);
 
 // Resident sweep (resident.hip): one workgroup runs up to `substeps` substeps
 // (to the stop point at most) of a system that fits its LDS, with at most
-// eight members of a species per thread; a later
-// launch_advance counts them.  block: 64..1024, a multiple of 64.
+// eight members of a species per thread, and counts them in
+// DevState::substep.  block: 64..1024, a multiple of 64.
 constexpr uint64_t kResidentLds = 160u * 1024u;
-// Substeps of one launch: at most some 30 ms of one workgroup's work.
+// Substeps of one launch: at most some 40 ms of one workgroup's work.
 constexpr uint32_t kResidentSubsteps = 4096;
 uint64_t resident_lds_bytes(const SysDesc& d);
 // Threads of the workgroup for a system on its own, or 0 where the two-pass
 // kernels are faster or its state does not fit.
 uint32_t resident_block(const SysDesc& d);
 hipError_t launch_resident(const SysDesc& d, uint32_t substeps, uint32_t block, hipStream_t st);
+
+// Replicas of a batch that share a launch of the resident sweep, one
+// workgroup each: workgroup w serves descs[ids[first + w]].
+struct ResidentClass {
+    uint32_t block = 0, rounds = 0;  // threads; members of a species per thread (4 or 8)
+    uint32_t lds = 0;                // bytes: the largest of the class
+    uint32_t maxDegree = 0;
+    uint32_t first = 0, count = 0;   // range of `ids`
+};
+// Whether a replica of a batch can run resident.
+bool resident_fits(const SysDesc& d);
+// Whether the replica is worth its own compute unit whatever else the batch
+// holds; else the time of its substep against the others' decides.
+bool resident_always(const SysDesc& d);
+double resident_substep_us(const SysDesc& d);
+hipError_t launch_resident_batch(const SysDesc* descs, const uint32_t* ids, const ResidentClass& c, uint32_t substeps,
+                                 hipStream_t st);
 
 // A batch of independent systems swept by one launch per pass.
 struct BatchLaunch {
@@ -69,7 +86,8 @@ struct BatchLaunch {
 };
 hipError_t launch_check_batch(const BatchLaunch& b, uint32_t k, const LaunchShape& s, hipStream_t st);
 hipError_t launch_perform_batch(const BatchLaunch& b, uint32_t k, const LaunchShape& s, hipStream_t st);
-// For every replica with a state: substep = min(substep + count, stopAt).
+// For every replica with a state that the two-pass kernels sweep:
+// substep = min(substep + count, stopAt).
 hipError_t launch_advance_batch(const SysDesc* descs, uint32_t nDescs, uint32_t count, hipStream_t st);
 // stopAt of replica r = stops[r] (replicas without a state are skipped).
 hipError_t launch_set_stops(const SysDesc* descs, uint32_t nDescs, const uint64_t* stops, hipStream_t st);

@@ -452,10 +452,10 @@ __global__ void k_advance(DevState* st, uint32_t count) {
         atomicAdd(reinterpret_cast<unsigned long long*>(&st->substep), (unsigned long long)count);
 }
 
-// Every live replica: substep = min(substep + count, stopAt).
+// Every live replica of the two-pass kernels: substep = min(substep + count, stopAt).
 __global__ void k_advance_batch(const SysDesc* descs, uint32_t nDescs, uint32_t count) {
     const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= nDescs) return;
+    if (r >= nDescs || descs[r].resident != 0u) return;
     const gptr<DevState> st = descs[r].state.global();
     if (st == nullptr) return;
     const uint64_t next = st->substep + count;

@@ -303,11 +303,18 @@ __device__ __forceinline__ void resident_body(const SysDesc& d, uint32_t substep
         marks[last * latWords + i] = *lds<uint32_t>(sProp + 4u * i);
         marks[(last ^ 1u) * latWords + i] = 0u;
     }
+    if (tid == 0u) d.state.global()->substep = t0 + n;
 }
 
 template <int ROUNDS, int MAXDEG>
 __global__ __launch_bounds__(1024) void k_resident(SysDesc d, uint32_t substeps) {
     resident_body<ROUNDS, MAXDEG>(d, substeps);
+}
+
+template <int ROUNDS, int MAXDEG>
+__global__ __launch_bounds__(1024) void k_resident_batch(const SysDesc* __restrict__ descs,
+                                                         const uint32_t* __restrict__ ids, uint32_t substeps) {
+    resident_body<ROUNDS, MAXDEG>(descs[ids[blockIdx.x]], substeps);
 }
 
 using ResidentKernel = void (*)(SysDesc, uint32_t);
@@ -320,9 +327,13 @@ ResidentKernel resident_kernel(uint32_t rounds, uint32_t maxDegree) {
     if (rounds <= 2u) return resident_by_degree<2>(maxDegree);
     if (rounds <= 3u) return resident_by_degree<3>(maxDegree);
     if (rounds <= 4u) return resident_by_degree<4>(maxDegree);
-    if (rounds <= 5u) return resident_by_degree<5>(maxDegree);
-    if (rounds <= 6u) return resident_by_degree<6>(maxDegree);
-    return resident_by_degree<8>(maxDegree);
+    return resident_by_degree<5>(maxDegree);
+}
+using ResidentBatchKernel = void (*)(const SysDesc*, const uint32_t*, uint32_t);
+template <int ROUNDS>
+ResidentBatchKernel resident_batch_by_degree(uint32_t maxDegree) {
+    return maxDegree <= 2u ? k_resident_batch<ROUNDS, 2>
+                           : (maxDegree <= 4u ? k_resident_batch<ROUNDS, 4> : k_resident_batch<ROUNDS, 8>);
 }
 
 // Dynamic LDS beyond 64 KiB is granted per kernel and device, once.
@@ -356,6 +367,24 @@ hipError_t launch_resident(const SysDesc& d, uint32_t substeps, uint32_t block, 
     const hipError_t err = allow_full_lds(reinterpret_cast<const void*>(kernel));
     if (err != hipSuccess) return err;
     hipLaunchKernelGGL(kernel, dim3(1), dim3(block), uint32_t(resident_lds_bytes(d)), st, d, substeps);
+    return hipGetLastError();
+}
+
+bool resident_fits(const SysDesc& d) {
+    return d.maxColorCount != 0u && d.maxColorCount <= 8u * 1024u && d.lone == 0u && resident_lds_bytes(d) <= kResidentLds;
+}
+
+bool resident_always(const SysDesc& d) { return d.maxColorCount <= kResidentMaxSpecies; }
+double resident_substep_us(const SysDesc& d) { return 1.0 + 1.1e-3 * double(d.maxColorCount); }
+
+hipError_t launch_resident_batch(const SysDesc* descs, const uint32_t* ids, const ResidentClass& c, uint32_t substeps,
+                                 hipStream_t st) {
+    if (c.count == 0u) return hipSuccess;
+    const ResidentBatchKernel kernel =
+        c.rounds <= 4u ? resident_batch_by_degree<4>(c.maxDegree) : resident_batch_by_degree<8>(c.maxDegree);
+    const hipError_t err = allow_full_lds(reinterpret_cast<const void*>(kernel));
+    if (err != hipSuccess) return err;
+    hipLaunchKernelGGL(kernel, dim3(c.count), dim3(c.block), c.lds, st, descs, ids + c.first, substeps);
     return hipGetLastError();
 }
 

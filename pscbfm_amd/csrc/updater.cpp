@@ -657,7 +657,6 @@ void Updater::runChunk(uint64_t S, uint32_t* log, bool profile, bool useGraph, v
         while (resident && left > 0) {
             const uint32_t part = uint32_t(std::min<uint64_t>(left, kResidentSubsteps));
             hip_check(launch_resident(dev_.desc, part, residentBlock_, stream_), "launch resident sweep");
-            hip_check(launch_advance(dev_.desc.state, part, stream_), "launch advance");
             left -= part;
         }
         if (useGraph && left > 0) {

@@ -10,7 +10,7 @@ import pytest
 
 import oracle
 import pscbfm_amd as P
-from helpers import GOLDEN, chains, make_updater, ordered_chains, oracle_for, stars
+from helpers import GOLDEN, chains, make_updater, oracle_for, ordered_chains, stage_updater, stars
 
 pytestmark = pytest.mark.gpu
 
@@ -117,3 +117,50 @@ def test_tuned_small_system_stays_exact():
     assert np.array_equal(a.getPositions(s.n), b.getPositions(s.n))
     a.cleanup()
     b.cleanup()
+
+
+def _batch_systems():
+    """Replicas of every path: resident always (up to 5120 members), resident
+    only beside long two-pass work (beyond), too large for LDS, and one whose
+    monomers without bonds the resident sweep does not take."""
+    return [chains((32, 32, 32), 24, 16, seed=1), ordered_chains((64, 64, 64), 800, 16),
+            stars((64, 64, 32), 30, 4, 9, seed=2), chains((128, 64, 128), 100, 50, seed=3),
+            chains((32, 32, 32), 80, 1, seed=4), chains((16, 64, 32), 30, 11, seed=5),
+            chains((128, 128, 64), 20, 40, seed=6)]
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_batch_paths_equal_runs_alone(kind):
+    systems = _batch_systems()
+    batch = P.Batch(0, len(systems), kind)
+    ids = [batch.add(stage_updater(s, 30 + i, kind)) for i, s in enumerate(systems)]
+    for m, block in ((5, 0), (3, 128), (66, 0), (2, 64)):  # automatic paths, then all on two passes, twice
+        batch.set_perform_block(block)
+        batch.run(m)
+    batch.remove(ids[0])
+    batch.set_perform_block(0)
+    batch.run(4)
+    for i, (rid, s) in enumerate(zip(ids, systems)):
+        if i == 0:
+            continue
+        u = make_updater(s, 30 + i, kind, block=256, slots=2)
+        st, _ = u.run(80)
+        assert np.array_equal(batch.positions(rid, s.n), u.getPositions(s.n)), i
+        assert batch.info(rid).accepted == st.accepted and batch.info(rid).substeps == u.counters()[0]
+        u.cleanup()
+
+
+def test_batch_with_more_replicas_than_compute_units():
+    """Small replicas share compute units in small workgroups beside full ones."""
+    small = chains((16, 16, 16), 4, 12, seed=1)
+    large = ordered_chains((64, 64, 64), 150, 16)
+    staged = [(small, 100 + i) for i in range(270)] + [(large, 50), (large, 51)]
+    batch = P.Batch(0, len(staged))
+    ids = [batch.add(stage_updater(s, seed)) for s, seed in staged]
+    batch.run(9)
+    for k in (0, 1, 135, 269, 270, 271):
+        s, seed = staged[k]
+        u = make_updater(s, seed, block=64, slots=1)
+        u.run(9)
+        assert np.array_equal(batch.positions(ids[k], s.n), u.getPositions(s.n)), k
+        u.cleanup()
