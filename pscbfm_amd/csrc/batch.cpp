@@ -21,6 +21,7 @@
 namespace pscbfm {
 
 namespace {
+constexpr uint32_t kMaxWaves = 4;  // of a pass-2 workgroup: each keeps a total of accepted moves
 constexpr size_t kComputeUnits = 256;
 constexpr uint32_t kSpreadTiles = 64;  // replicas with at least this many workgroups use every XCD
 
@@ -268,7 +269,7 @@ uint32_t Batch::tilesNeeded(const SystemLayout& L) const {
 }
 
 uint64_t Batch::footprint(const SystemLayout& L) const {
-    return DeviceSystem::footprint(L, latticeKind_, false, tilesNeeded(L));
+    return DeviceSystem::footprint(L, latticeKind_, false, kMaxWaves * tilesNeeded(L));
 }
 
 uint32_t Batch::add(const SystemLayout& L, uint64_t seed, uint64_t startMcs) {
@@ -288,7 +289,7 @@ uint32_t Batch::add(const SystemLayout& L, uint64_t seed, uint64_t startMcs) {
     r.layout = L;
     r.seed = seed;
     r.dev.reset(new DeviceSystem());
-    r.dev->allocate(L, latticeKind_, seed, /*withLists=*/false, nT, stream_);
+    r.dev->allocate(L, latticeKind_, seed, /*withLists=*/false, kMaxWaves * nT, stream_);
     const uint64_t start = startMcs * uint64_t(L.colors.size());
     DevState st = r.dev->readState(stream_);
     st.substep = start;

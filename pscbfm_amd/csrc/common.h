@@ -215,12 +215,11 @@ struct ColorInfo {
     uint32_t pad_;
 };
 
-// Accepted moves are not counted with atomics: workgroup w of the pass-2
-// kernel adds its count to its own running total acceptedByBlock[w] (one
-// writer per entry, kernels ordered on the stream), and the host sums the
-// entries.  Thousands of workgroups adding to one address would serialise on
-// a single memory channel.
-constexpr uint32_t kMaxPerformBlocks = 1u << 16;
+// Accepted moves are not counted with atomics: each wave of the pass-2 kernel
+// adds its count to its own running total in acceptedByBlock (one writer per
+// entry, kernels ordered on the stream), and the host sums the entries.
+// Thousands of waves adding to one address would serialise on a single memory
+// channel.
 
 // Mutable per-system state that lives on the device so that a captured
 // graph can replay any number of substeps without host involvement.
@@ -236,7 +235,7 @@ struct DevState {
     uint32_t* log;             // optional per-substep accepted counts
     uint64_t logFirst;         // substep index stored in log[0]
     uint64_t logCapacity;      // entries in log
-    uint64_t* acceptedByBlock; // kMaxPerformBlocks running totals
+    uint64_t* acceptedByBlock; // running totals of accepted moves
 };
 static_assert(sizeof(DevState) == 64, "DevState is one 64-byte line");
 static_assert(offsetof(DevState, drawBase) == 24, "the launch words are the first 32 bytes");

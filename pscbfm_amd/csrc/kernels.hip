@@ -247,12 +247,34 @@ __device__ __forceinline__ uint32_t wave_sum_small(uint32_t v) {
     return total;
 }
 
-// Adds a wave's accepted moves to its workgroup's running total and to the
-// substep's log entry, without waiting: atomics whose results are unused.
-__device__ __forceinline__ void add_accepted(const Launch& L, gptr<uint64_t> accSlot, uint32_t accepted) {
+// A wave's running total of accepted moves: entry `wave` of those of its
+// workgroup, read at the start of pass 2 and written at its end, so that the
+// kernel ends without an atomic (which is executed beyond the L2: us per
+// substep with atomics and without, 128^3 melt 7.0 and 6.7, 256^3 11.1 and 10.8,
+// 512^3 39.3 and 38.6).  Only a finer launch shape than the entries
+// were sized for shares one entry per workgroup, with atomics.
+struct AcceptedTotal {
+    gptr<uint64_t> entry;
+    uint64_t before;
+    bool own;
+};
+__device__ __forceinline__ AcceptedTotal accepted_total(const Launch& L, const SysDesc& d, uint32_t workgroup,
+                                                        uint32_t workgroups) {
+    const uint32_t waves = blockDim.x >> 6;
+    const uint32_t wave = uint32_t(__builtin_amdgcn_readfirstlane(int32_t(threadIdx.x >> 6)));
+    AcceptedTotal a;
+    a.own = workgroups * waves <= d.accEntries;
+    a.entry = L.acceptedByBlock + (a.own ? workgroup * waves + wave : workgroup);
+    a.before = *a.entry;
+    return a;
+}
+__device__ __forceinline__ void add_accepted(const Launch& L, const AcceptedTotal& a, uint32_t accepted) {
     const uint32_t total = wave_sum_small(accepted);
     if ((threadIdx.x & 63u) == 0u && total != 0u) {
-        __hip_atomic_fetch_add(&accSlot[0], uint64_t(total), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (a.own)
+            *a.entry = a.before + total;
+        else
+            __hip_atomic_fetch_add(a.entry, uint64_t(total), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (L.log != nullptr) {
             const uint64_t idx = L.t - L.logFirst;
             if (idx < L.logCapacity)
@@ -290,15 +312,16 @@ __device__ __forceinline__ void apply_move(const SysDesc& d, gptr<uint32_t> pos,
 }
 
 // Pass 2 of substep t over one pass-1 list.  The accepted count is added to
-// *accSlot, an entry only this workgroup's waves add to.  With `clear` it
-// also zeroes slice lb of nb of the other parity's proposals.
+// the totals of workgroup `owner` of nb.  With `clear` it also zeroes slice lb
+// of nb of the other parity's proposals.
 template <int LAT>
 __device__ __forceinline__ void perform_body(const SysDesc& d, const Launch& L, uint32_t lb, uint32_t nb, bool clear,
-                                             gptr<const uint64_t> list, uint32_t count, gptr<uint64_t> accSlot) {
+                                             gptr<const uint64_t> list, uint32_t count, uint32_t owner) {
     const uint64_t t = L.t;
     const SubstepDraw draw = L.draw;
     const ColorInfo ci = load_color(d.colors.global(), draw.species);
     const uint32_t B = blockDim.x;
+    const AcceptedTotal total = accepted_total(L, d, owner, nb);
 
     if (clear) clear_other_parity(d, t, lb, nb);
 
@@ -321,7 +344,7 @@ __device__ __forceinline__ void perform_body(const SysDesc& d, const Launch& L, 
         apply_move<LAT>(d, pos, lat, ci.slotOffset + jj, m, dir, masks, mv);
         ++accepted;
     }
-    add_accepted(L, accSlot, accepted);
+    add_accepted(L, total, accepted);
 }
 
 // ---- single system ----------------------------------------------------------------
@@ -344,7 +367,7 @@ __global__ __launch_bounds__(256) void k_perform(SysDesc d, uint32_t k, uint32_t
     const uint32_t lb = xcd_block();  // same numbering as pass 1: list lb
     perform_body<LAT>(d, L, lb, gridDim.x, clear != 0u,
                       (gptr<const uint64_t>)d.list.global() + size_t(lb) * listStride, d.listCount.global()[lb],
-                      L.acceptedByBlock + blockIdx.x);
+                      blockIdx.x);
 }
 
 // Pass 2 of a single system with several lists per workgroup: each group
@@ -370,6 +393,7 @@ __global__ __launch_bounds__(256) void k_perform_lists(SysDesc d, uint32_t k, ui
     Launch L;
     if (!begin_substep(d, k, L)) return;
     if (!haveList) count = 0;
+    const AcceptedTotal total = accepted_total(L, d, blockIdx.x, gridDim.x);
     const uint64_t t = L.t;
     const uint32_t slotOffset =
         ((gptr<const uint32_t>)(d.colors.global() + L.draw.species))[offsetof(ColorInfo, slotOffset) / 4];
@@ -407,7 +431,7 @@ __global__ __launch_bounds__(256) void k_perform_lists(SysDesc d, uint32_t k, ui
             ++accepted;
         }
     }
-    add_accepted(L, L.acceptedByBlock + blockIdx.x, accepted);
+    add_accepted(L, total, accepted);
 }
 
 // ---- batch of replicas ---------------------------------------------------------------
@@ -444,7 +468,7 @@ __global__ __launch_bounds__(256) void k_perform_batch(const SysDesc* __restrict
     if (!begin_substep(d, k, L)) return;
     perform_body<LAT>(d, L, tile.chunk, tile.chunks, true,
                       global_ptr(reinterpret_cast<const uint64_t*>(lists)) + size_t(blockIdx.x) * listStride,
-                      global_ptr(listCounts)[blockIdx.x], L.acceptedByBlock + tile.chunk);
+                      global_ptr(listCounts)[blockIdx.x], tile.chunk);
 }
 
 __global__ void k_advance(DevState* st, uint32_t count) {

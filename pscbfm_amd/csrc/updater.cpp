@@ -278,7 +278,8 @@ void Updater::applyLaunchShape() {
     }
     shape_.grid = grid_for(layout_.maxColorCount, shape_.block * shape_.slots);
     shape_.clearPass = clearPassOverride_ ? clearPassOverride_ : automatic_clear_pass(layout_, latticeKind_);
-    performGridMax_ = std::max(performGridMax_, shape_.passTwoGrid());
+    const uint32_t waveTotals = shape_.passTwoGrid() * (shape_.passTwoBlock() / 64u);
+    acceptedMax_ = std::max(acceptedMax_, std::min(waveTotals, dev_.accEntries));
     const bool pinned = shapePinned_ || performOverride_ || walkGroupOverride_ || clearPassOverride_;
     residentBlock_ = pinned ? 0u : resident_block(dev_.desc);
     dropGraphs();
@@ -425,7 +426,7 @@ void Updater::initialize() {
     dev_.allocate(layout_, latticeKind_, seed_, /*withLists=*/true, uint32_t(max_grid(layout_.maxColorCount)),
                   stream_);
 
-    performGridMax_ = 0;
+    acceptedMax_ = 0;
     applyLaunchShape();
     substep_ = startMcs_ * nColors();
     if (substep_ != 0) {
@@ -555,7 +556,7 @@ void Updater::runImpl(int32_t nMCS, uint32_t* log, bool profile, bool useGraph, 
     lastRun_ = total;
     if (readBack_) syncFromDevice();
     const DevState st = dev_.readState(stream_);
-    std::vector<uint64_t> perBlock(performGridMax_);
+    std::vector<uint64_t> perBlock(acceptedMax_);
     hip_check(hipMemcpy(perBlock.data(), st.acceptedByBlock, perBlock.size() * sizeof(uint64_t), hipMemcpyDeviceToHost),
               "accepted D2H");
     uint64_t acc = 0;

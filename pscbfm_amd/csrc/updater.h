@@ -236,7 +236,7 @@ private:
     bool shapePinned_ = false;    // setLaunchShape stated a shape
     uint32_t residentBlock_ = 0;  // threads of the resident sweep's workgroup; 0: two-pass kernels
     std::map<uint32_t, hipGraphExec_t> graphs_;  // by substeps per replay
-    uint32_t performGridMax_ = 0;  // largest pass-2 grid used (entries of acceptedByBlock)
+    uint32_t acceptedMax_ = 0;  // entries of acceptedByBlock that any launch shape so far uses
     uint64_t substep_ = 0;
     uint64_t acceptedTotal_ = 0;
     uint64_t cells_ = 0;
