@@ -10,13 +10,13 @@
 //   proposal 2 x 1 bit per cell   double-buffered by substep parity
 //   colors   ColorInfo per species
 //   bond     64 bytes             forbidden bond keys (512 bits)
-//   state    DevState
-//   acc      uint64 per workgroup accepted-move running totals
 //   ids      16-bit partner codes, two per word (uint8 lattice only)
 //   rowBase  uint32 per (species, row): base slot of the codes (uint8 lattice only)
 //   slotOf   uint32 per monomer   slot of each monomer (coordinate read-back)
-//   xyz      3 int32 per monomer  unfolded coordinates decoded for read-back (only with withLists)
 //   key      uint32 per slot      inner move hash of the member's reference index
+//   xyz      3 int32 per monomer  unfolded coordinates decoded for read-back (only with withLists)
+//   state    DevState
+//   acc      uint64 per wave      accepted-move running totals
 #include "device_system.h"
 
 #include <algorithm>
@@ -40,8 +40,9 @@ namespace {
 
 uint64_t align_up(uint64_t v, uint64_t a) { return (v + a - 1) / a * a; }
 
-enum { P_POS, P_IMGX, P_IMGY, P_IMGZ, P_LIST, P_LCOUNT, P_NBR, P_LAT, P_PROP, P_COLORS, P_BOND, P_STATE, P_ACC, P_IDS, P_ROWB,
-       P_SLOTOF, P_XYZ, P_KEY, P_N };
+// P_XYZ, P_STATE and P_ACC in this order: an updater reads them back in one copy.
+enum { P_POS, P_IMGX, P_IMGY, P_IMGZ, P_LIST, P_LCOUNT, P_NBR, P_LAT, P_PROP, P_COLORS, P_BOND, P_IDS, P_ROWB,
+       P_SLOTOF, P_KEY, P_XYZ, P_STATE, P_ACC, P_N };
 
 struct Plan {
     uint64_t bytes[P_N];
@@ -132,6 +133,8 @@ void DeviceSystem::allocate(const SystemLayout& L, uint32_t latticeKind, uint64_
     desc.maxColorCount = L.maxColorCount;
     desc.accEntries = this->accEntries;
     slotOfDev = reinterpret_cast<uint32_t*>(base + p.off[P_SLOTOF]);
+    stateAt = p.off[P_STATE] - p.off[P_XYZ];
+    totalsAt = p.off[P_ACC] - p.off[P_XYZ];
     xyzDev = withLists ? reinterpret_cast<int32_t*>(base + p.off[P_XYZ]) : nullptr;
 
     hip_check(hipMemsetAsync(arena, 0, p.total, stream), "hipMemsetAsync");
@@ -205,17 +208,6 @@ uint64_t DeviceSystem::acceptedTotal(uint32_t entries, hipStream_t stream) const
     uint64_t total = 0;
     for (uint64_t x : v) total += x;
     return total;
-}
-
-void DeviceSystem::positions(const SystemLayout& L, int32_t* xyzOut, hipStream_t stream) const {
-    if (!L.nMonomers) return;
-    if (!xyzDev) throw std::logic_error("positions: this system decodes into its batch's buffer");
-    // decoded on the device in the caller's order: 12 bytes per monomer
-    // cross the bus and the host only receives them
-    hip_check(launch_unfold(desc, slotOfDev, L.nMonomers, xyzDev, stream), "launch unfold");
-    hip_check(hipMemcpyAsync(xyzOut, xyzDev, uint64_t(L.nMonomers) * 12, hipMemcpyDeviceToHost, stream),
-              "positions D2H");
-    hip_check(hipStreamSynchronize(stream), "sync");
 }
 
 UnfoldJob DeviceSystem::unfoldJob(uint32_t first, uint32_t count, uint64_t out) const {

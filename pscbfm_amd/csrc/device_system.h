@@ -26,10 +26,12 @@ struct DeviceSystem {
     uint32_t accEntries = 0;  // entries of DevState::acceptedByBlock
     SysDesc desc{};
     // The slot of every monomer, for decoding coordinates on the device, and
-    // (systems with their own launches, withLists) the buffer positions()
-    // decodes them into.  Batch replicas decode into the batch's buffer.
+    // (systems with their own launches, withLists) the buffer they are decoded
+    // into.  Batch replicas decode into the batch's buffer.
     uint32_t* slotOfDev = nullptr;
     int32_t* xyzDev = nullptr;
+    // Bytes from xyzDev to the state and to the accepted totals.
+    size_t stateAt = 0, totalsAt = 0;
 
     // Bytes allocate() would take.  `withLists`: the system runs its own
     // launches (pass-1 lists inside the allocation); batch replicas use the
@@ -44,8 +46,6 @@ struct DeviceSystem {
     DevState readState(hipStream_t stream) const;
     void writeState(const DevState& s, hipStream_t stream);
     uint64_t acceptedTotal(uint32_t entries, hipStream_t stream) const;
-    // Unfolded coordinates in the caller's monomer order (withLists systems).
-    void positions(const SystemLayout& L, int32_t* xyzOut, hipStream_t stream) const;
     // The job that decodes monomers [first, first + count) into records
     // out.. of a shared buffer (launch_unfold_jobs; firstBlock left 0).
     UnfoldJob unfoldJob(uint32_t first, uint32_t count, uint64_t out) const;

@@ -8,6 +8,7 @@
 #include <limits>
 #include <sstream>
 #include <stdexcept>
+#include <thread>
 
 #include "autotune.h"
 #include "noalloc.h"
@@ -20,6 +21,32 @@ constexpr uint64_t kMaxDrawSubsteps = uint64_t(1) << 22;
 namespace {
 
 bool is_pow2(uint32_t v) { return v != 0 && (v & (v - 1)) == 0; }
+
+// Systems from this size on read back into pinned memory: a copy into
+// pageable memory goes through the runtime's staging buffers, at 12 instead
+// of over 50 GB/s (1.0 ms for 2^20 monomers, 8 ms for 2^23).
+constexpr uint32_t kPinMonomers = 1u << 15;
+
+// memcpy by up to eight threads, 2 MiB or more each: one thread copies at
+// about 10 GB/s and spends as long again on the first touch of new memory.
+void copy_out(void* dst, const void* src, size_t bytes) {
+    const size_t parts = std::min<size_t>(8, std::max<size_t>(1, bytes >> 21));
+    const size_t per = (bytes / parts + 4095) / 4096 * 4096;
+    std::vector<std::thread> pool;
+    auto part = [&](size_t k) {
+        const size_t lo = std::min(bytes, k * per), hi = k + 1 == parts ? bytes : std::min(bytes, lo + per);
+        std::memcpy(static_cast<char*>(dst) + lo, static_cast<const char*>(src) + lo, hi - lo);
+    };
+    for (size_t k = 1; k < parts; ++k) {
+        try {
+            pool.emplace_back(part, k);
+        } catch (...) {
+            part(k);  // no thread available
+        }
+    }
+    part(0);
+    for (std::thread& t : pool) t.join();
+}
 
 }  // namespace
 
@@ -62,7 +89,7 @@ void Updater::setNrOfAllMonomers(uint32_t n) {
         throw std::invalid_argument("[UpdaterGPUScBFM_AB_Type::setNrOfAllMonomers] at most 2^28 monomers are supported");
     n_ = n;
     nSet_ = true;
-    xyz_.assign(3 * size_t(n), 0);
+    host_.allocate(12 * size_t(n), 0, false);
     attr_.assign(n, 0);
     degree_.assign(n, 0);
     nbrIds_.assign(size_t(n) * kMaxConnectivity, 0);
@@ -99,16 +126,16 @@ void Updater::setMonomerCoordinates(uint32_t i, int32_t x, int32_t y, int32_t z)
     if (initialized_)
         throw std::runtime_error(
             "[UpdaterGPUScBFM_AB_Type::setMonomerCoordinates] coordinates are owned by the device after initialize");
-    xyz_[3 * size_t(i) + 0] = x;
-    xyz_[3 * size_t(i) + 1] = y;
-    xyz_[3 * size_t(i) + 2] = z;
+    xyz()[3 * size_t(i) + 0] = x;
+    xyz()[3 * size_t(i) + 1] = y;
+    xyz()[3 * size_t(i) + 2] = z;
 }
 
 void Updater::setMonomerCoordinatesBulk(const int32_t* xyz, uint32_t n) {
     requireMonomers("setMonomerCoordinatesBulk");
     if (n != n_) throw std::invalid_argument("[setMonomerCoordinatesBulk] count differs from setNrOfAllMonomers");
     if (initialized_) throw std::runtime_error("[setMonomerCoordinatesBulk] already initialized");
-    std::memcpy(xyz_.data(), xyz, sizeof(int32_t) * 3 * size_t(n));
+    std::memcpy(this->xyz(), xyz, sizeof(int32_t) * 3 * size_t(n));
 }
 
 // UpdaterGPUScBFM_AB_Type.cu:777-795 (directed: callers register both ways)
@@ -177,9 +204,9 @@ void Updater::populateLattice() {
     codec.init(box_[0], box_[1], box_[2]);
     hostLattice_.assign(size_t(box_[0]) * box_[1] * box_[2], 0);
     for (uint32_t i = 0; i < n_; ++i) {
-        const uint32_t x = uint32_t(xyz_[3 * size_t(i)]) & (box_[0] - 1);
-        const uint32_t y = uint32_t(xyz_[3 * size_t(i) + 1]) & (box_[1] - 1);
-        const uint32_t z = uint32_t(xyz_[3 * size_t(i) + 2]) & (box_[2] - 1);
+        const uint32_t x = uint32_t(xyz()[3 * size_t(i)]) & (box_[0] - 1);
+        const uint32_t y = uint32_t(xyz()[3 * size_t(i) + 1]) & (box_[1] - 1);
+        const uint32_t z = uint32_t(xyz()[3 * size_t(i) + 2]) & (box_[2] - 1);
         hostLattice_[codec.encode(x, y, z)] = 1;
     }
 }
@@ -299,15 +326,15 @@ void Updater::checkSystem() const {
     std::vector<uint8_t> occ(cells, 0);
     for (uint32_t i = 0; i < n_; ++i) {
         for (uint32_t c = 0; c < 8; ++c) {
-            const uint32_t x = uint32_t(xyz_[3 * size_t(i)] + int32_t(c & 1u)) & (box_[0] - 1);
-            const uint32_t y = uint32_t(xyz_[3 * size_t(i) + 1] + int32_t((c >> 1) & 1u)) & (box_[1] - 1);
-            const uint32_t z = uint32_t(xyz_[3 * size_t(i) + 2] + int32_t((c >> 2) & 1u)) & (box_[2] - 1);
+            const uint32_t x = uint32_t(xyz()[3 * size_t(i)] + int32_t(c & 1u)) & (box_[0] - 1);
+            const uint32_t y = uint32_t(xyz()[3 * size_t(i) + 1] + int32_t((c >> 1) & 1u)) & (box_[1] - 1);
+            const uint32_t z = uint32_t(xyz()[3 * size_t(i) + 2] + int32_t((c >> 2) & 1u)) & (box_[2] - 1);
             const uint64_t lin = x + uint64_t(box_[0]) * (y + uint64_t(box_[1]) * z);
             if (occ[lin]) {
                 std::ostringstream msg;
                 msg << "[UpdaterGPUScBFM_AB_Type::checkSystem] excluded volume violated: monomer " << i
-                    << " at (" << xyz_[3 * size_t(i)] << "," << xyz_[3 * size_t(i) + 1] << ","
-                    << xyz_[3 * size_t(i) + 2] << ") overlaps another monomer";
+                    << " at (" << xyz()[3 * size_t(i)] << "," << xyz()[3 * size_t(i) + 1] << ","
+                    << xyz()[3 * size_t(i) + 2] << ") overlaps another monomer";
                 throw std::runtime_error(msg.str());
             }
             occ[lin] = 1;
@@ -322,7 +349,7 @@ void Updater::checkSystem() const {
             int32_t d[3];
             for (int a = 0; a < 3; ++a) {
                 const int32_t L = int32_t(box_[a]);
-                const int32_t raw = xyz_[3 * size_t(j) + a] - xyz_[3 * size_t(i) + a];
+                const int32_t raw = xyz()[3 * size_t(j) + a] - xyz()[3 * size_t(i) + a];
                 d[a] = int32_t(uint32_t(raw + L / 2) & uint32_t(L - 1)) - L / 2;
             }
             const bool tooLong = std::abs(d[0]) > 3 || std::abs(d[1]) > 3 || std::abs(d[2]) > 3;
@@ -338,8 +365,51 @@ void Updater::checkSystem() const {
     }
 }
 
+void HostBuffer::allocate(size_t bytes, size_t keep, bool pinned) {
+    uint8_t* p = nullptr;
+    bool isPinned = false;
+    if (bytes != 0 && pinned) {
+        void* q = nullptr;
+        isPinned = hipHostMalloc(&q, bytes, hipHostMallocDefault) == hipSuccess;
+        p = static_cast<uint8_t*>(q);
+        if (!isPinned) (void)hipGetLastError();  // pageable memory does as well
+    }
+    if (bytes != 0 && !isPinned) {
+        p = static_cast<uint8_t*>(std::calloc(bytes, 1));
+        if (!p) throw std::bad_alloc();
+    }
+    keep = std::min({keep, bytes, bytes_});
+    if (keep) std::memcpy(p, data_, keep);
+    if (isPinned) std::memset(p + keep, 0, bytes - keep);
+    if (pinned_)
+        (void)hipHostFree(data_);
+    else
+        std::free(data_);
+    data_ = p;
+    bytes_ = bytes;
+    pinned_ = isPinned;
+}
+
+// The device's state and accepted totals, and with `positions` the
+// coordinates, decoded on the device in the caller's order, in one copy.
+// Returns the state.
+DevState Updater::readDevice(bool positions) {
+    if (positions) hip_check(launch_unfold(dev_.desc, dev_.slotOfDev, n_, dev_.xyzDev, stream_), "launch unfold");
+    const size_t first = positions ? 0 : dev_.stateAt, last = dev_.totalsAt + 8 * size_t(acceptedMax_);
+    hip_check(hipMemcpyAsync(host_.data() + first, reinterpret_cast<const uint8_t*>(dev_.xyzDev) + first, last - first,
+                             hipMemcpyDeviceToHost, stream_),
+              "read-back D2H");
+    hip_check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
+    DevState st;
+    std::memcpy(&st, host_.data() + dev_.stateAt, sizeof st);
+    return st;
+}
+
 void Updater::freeDevice() {
     dropGraphs();
+    if (timing_[0]) (void)hipEventDestroy(timing_[0]);
+    if (timing_[1]) (void)hipEventDestroy(timing_[1]);
+    timing_[0] = timing_[1] = nullptr;
     dev_.release();
     if (drawTable_) (void)hipFree(drawTable_);
     drawTable_ = nullptr;
@@ -356,7 +426,7 @@ SystemInput Updater::stagedInput() const {
     if (box_[0] == 0) throw std::runtime_error("[UpdaterGPUScBFM_AB_Type::initialize] setLatticeSize first");
     SystemInput in;
     std::memcpy(in.box, box_, sizeof box_);
-    in.xyz = xyz_;
+    in.xyz.assign(xyz(), xyz() + 3 * size_t(n_));
     in.bonds.start.assign(size_t(n_) + 1, 0);
     for (uint32_t i = 0; i < n_; ++i) in.bonds.start[i + 1] = in.bonds.start[i] + degree_[i];
     in.bonds.ids.resize(in.bonds.start[n_]);
@@ -426,6 +496,9 @@ void Updater::initialize() {
     dev_.allocate(layout_, latticeKind_, seed_, /*withLists=*/true, uint32_t(max_grid(layout_.maxColorCount)),
                   stream_);
 
+    host_.allocate(dev_.totalsAt + 8 * size_t(dev_.accEntries), 12 * size_t(n_), n_ >= kPinMonomers);
+    degreeSum_.assign(nColors(), 0);
+    for (uint32_t i = 0; i < n_; ++i) degreeSum_[layout_.color[i]] += degree_[i];
     acceptedMax_ = 0;
     applyLaunchShape();
     substep_ = startMcs_ * nColors();
@@ -554,13 +627,10 @@ void Updater::runImpl(int32_t nMCS, uint32_t* log, bool profile, bool useGraph, 
         total.performLaunches += lastRun_.performLaunches;
     }
     lastRun_ = total;
-    if (readBack_) syncFromDevice();
-    const DevState st = dev_.readState(stream_);
-    std::vector<uint64_t> perBlock(acceptedMax_);
-    hip_check(hipMemcpy(perBlock.data(), st.acceptedByBlock, perBlock.size() * sizeof(uint64_t), hipMemcpyDeviceToHost),
-              "accepted D2H");
+    const DevState st = readDevice(readBack_);
+    const uint64_t* totals = reinterpret_cast<const uint64_t*>(host_.data() + dev_.totalsAt);
     uint64_t acc = 0;
-    for (uint64_t v : perBlock) acc += v;
+    for (uint32_t k = 0; k < acceptedMax_; ++k) acc += totals[k];
     lastRun_.accepted = acc - acceptedTotal_;
     acceptedTotal_ = acc;
     if (st.substep != substep_) throw std::runtime_error("device substep counter out of step with the host");
@@ -637,8 +707,10 @@ void Updater::runChunk(uint64_t S, uint32_t* log, bool profile, bool useGraph, v
     hipEvent_t e0 = nullptr, e1 = nullptr;
     const auto h0 = std::chrono::steady_clock::now();
     if (!scratch) {
-        hip_check(hipEventCreate(&e0), "hipEventCreate");
-        hip_check(hipEventCreate(&e1), "hipEventCreate");
+        for (hipEvent_t& e : timing_)
+            if (!e) hip_check(hipEventCreate(&e), "hipEventCreate");
+        e0 = timing_[0];
+        e1 = timing_[1];
         hip_check(hipEventRecord(e0, stream_), "hipEventRecord");
     }
     std::vector<hipEvent_t> kev;
@@ -702,16 +774,11 @@ void Updater::runChunk(uint64_t S, uint32_t* log, bool profile, bool useGraph, v
         lastRun_.performLaunches = S;
         for (auto& e : kev) (void)hipEventDestroy(e);
     }
-    if (e0) (void)hipEventDestroy(e0);
-    if (e1) (void)hipEventDestroy(e1);
-
     // Attempts and bond terms follow from the host copy of the draws: every
     // member of the drawn species is attempted, with all its bonds.
-    std::vector<uint64_t> deg(nc, 0);
-    for (uint32_t i = 0; i < n_; ++i) deg[layout_.color[i]] += degree_[i];
     for (uint64_t k = 0; k < S; ++k) {
         lastRun_.attempted += layout_.colors[species[k]].count;
-        lastRun_.bondTerms += deg[species[k]];
+        lastRun_.bondTerms += degreeSum_[species[k]];
     }
     lastRun_.substeps = S;
     substep_ += S;
@@ -757,7 +824,7 @@ void Updater::r250State(uint32_t* words250) const {
 // CRITICAL.cu:414-698 (synchronous; returns after copy-back and unsort)
 void Updater::runSimulationOnGPU(int32_t nMCS) { run(nMCS, nullptr, false, true); }
 
-void Updater::syncFromDevice() { dev_.positions(layout_, xyz_.data(), stream_); }
+void Updater::syncFromDevice() { readDevice(true); }
 
 void Updater::readPositionsBack() {
     if (!initialized_) throw std::runtime_error("[readPositionsBack] initialize has not been called");
@@ -801,20 +868,20 @@ void Updater::partnerCodeStats(uint64_t& partners, uint64_t& escapes) const {
 
 int32_t Updater::getMonomerPositionInX(uint32_t i) const {
     requireIndex(i, "getMonomerPositionInX");
-    return xyz_[3 * size_t(i)];
+    return xyz()[3 * size_t(i)];
 }
 int32_t Updater::getMonomerPositionInY(uint32_t i) const {
     requireIndex(i, "getMonomerPositionInY");
-    return xyz_[3 * size_t(i) + 1];
+    return xyz()[3 * size_t(i) + 1];
 }
 int32_t Updater::getMonomerPositionInZ(uint32_t i) const {
     requireIndex(i, "getMonomerPositionInZ");
-    return xyz_[3 * size_t(i) + 2];
+    return xyz()[3 * size_t(i) + 2];
 }
 
 void Updater::getPositionsBulk(int32_t* xyz, uint32_t n) const {
     if (n != n_) throw std::invalid_argument("[getPositionsBulk] count differs from the number of monomers");
-    std::memcpy(xyz, xyz_.data(), sizeof(int32_t) * 3 * size_t(n));
+    copy_out(xyz, this->xyz(), sizeof(int32_t) * 3 * size_t(n));
 }
 
 // UpdaterGPUScBFM_AB_Type.cu:455-465.  Unlike the reference this also forgets
@@ -825,7 +892,8 @@ void Updater::destruct() {
     layout_ = SystemLayout{};
     n_ = 0;
     nSet_ = false;
-    xyz_.clear();
+    host_.allocate(0, 0, false);
+    degreeSum_.clear();
     attr_.clear();
     degree_.clear();
     nbrIds_.clear();

@@ -44,6 +44,24 @@ struct StagedSystem {
 // The 108-bond check of UpdaterGPUScBFM_AB_Type.cu:514-530, then the layout.
 SystemLayout layout_of(const StagedSystem& s);
 
+// Host memory, zeroed, pinned where that is asked for and can be had.
+class HostBuffer {
+public:
+    HostBuffer() = default;
+    HostBuffer(const HostBuffer&) = delete;
+    HostBuffer& operator=(const HostBuffer&) = delete;
+    ~HostBuffer() { allocate(0, 0, false); }
+    // `bytes` bytes, the first `keep` as they were.
+    void allocate(size_t bytes, size_t keep, bool pinned);
+    uint8_t* data() { return data_; }
+    const uint8_t* data() const { return data_; }
+
+private:
+    uint8_t* data_ = nullptr;
+    size_t bytes_ = 0;
+    bool pinned_ = false;
+};
+
 class Updater {
 public:
     Updater();
@@ -198,13 +216,18 @@ private:
     void dropGraphs();
     uint32_t graphChunk() const;
     void syncFromDevice();
+    DevState readDevice(bool positions);
     void applyLaunchShape();
 
     // staging
     int gpu_ = -1;
     uint32_t n_ = 0;
     bool nSet_ = false;
-    std::vector<int32_t> xyz_;
+    // Coordinates (12 bytes per monomer); once initialized followed by the
+    // device's state and accepted totals as the last read-back left them.
+    HostBuffer host_;
+    int32_t* xyz() { return reinterpret_cast<int32_t*>(host_.data()); }
+    const int32_t* xyz() const { return reinterpret_cast<const int32_t*>(host_.data()); }
     std::vector<int32_t> attr_;
     std::vector<uint32_t> degree_;
     std::vector<uint32_t> nbrIds_;   // kMaxConnectivity per monomer
@@ -239,6 +262,8 @@ private:
     uint32_t acceptedMax_ = 0;  // entries of acceptedByBlock that any launch shape so far uses
     uint64_t substep_ = 0;
     uint64_t acceptedTotal_ = 0;
+    std::vector<uint64_t> degreeSum_;  // bonds of each species' members
+    hipEvent_t timing_[2] = {};        // around the timed part of a run
     uint64_t cells_ = 0;
     uint32_t* drawTable_ = nullptr;  // R250 mode: 2 words per substep of one run chunk
     uint64_t drawCapacity_ = 0;      // substeps drawTable_ holds
