@@ -49,11 +49,10 @@ Batch::Batch(int gpu, uint32_t latticeKind, uint32_t tileCapacity, uint32_t repl
     shape_.performBlock = default_perform_block(block);
     shape_.grid = tileCap_;
     hip_check(hipSetDevice(gpu_), "hipSetDevice");
-    // created together: the runtime deals its hardware queues out in turn, and
-    // streams on one queue would not overlap
-    hip_check(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking), "hipStreamCreate");
-    for (hipStream_t& s : side_) hip_check(hipStreamCreateWithFlags(&s, hipStreamNonBlocking), "hipStreamCreate");
-    for (hipEvent_t& e : sideDone_) hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
+    streams_ = acquire_streams(2);
+    stream_ = streams_[0];
+    side_ = streams_[1];
+    hip_check(hipEventCreateWithFlags(&sideDone_, hipEventDisableTiming), "hipEventCreate");
     hip_check(hipEventCreateWithFlags(&fork_, hipEventDisableTiming), "hipEventCreate");
     hip_check(hipMalloc(&dDescs_, sizeof(SysDesc) * replicaCap_), "hipMalloc descs");
     hip_check(hipMalloc(&dStops_, sizeof(uint64_t) * replicaCap_), "hipMalloc stops");
@@ -99,10 +98,7 @@ void Batch::growTiles(uint32_t needed) {
 Batch::~Batch() {
     if (stream_) (void)hipStreamSynchronize(stream_);
     dropGraphs();
-    for (hipStream_t s : side_)
-        if (s) (void)hipStreamDestroy(s);
-    for (hipEvent_t e : sideDone_)
-        if (e) (void)hipEventDestroy(e);
+    if (sideDone_) (void)hipEventDestroy(sideDone_);
     if (fork_) (void)hipEventDestroy(fork_);
     for (auto& r : replicas_) r.dev.reset();
     for (void* p : {static_cast<void*>(dDescs_), static_cast<void*>(dTiles_), static_cast<void*>(dLists_),
@@ -110,7 +106,7 @@ Batch::~Batch() {
                     static_cast<void*>(dJobs_), static_cast<void*>(dXyz_), static_cast<void*>(dResident_)})
         if (p) (void)hipFree(p);
     if (hXyz_) (void)hipHostFree(hXyz_);
-    if (stream_) (void)hipStreamDestroy(stream_);
+    release_streams(streams_, gpu_);
 }
 
 void Batch::setPerformBlock(uint32_t block) {
@@ -206,8 +202,8 @@ void Batch::assignPaths() {
             ++twoPassUsed_;
         }
     }
-    // At most two launches, one to a stream, since launches of one stream wait
-    // for each other.  Up to one replica per compute unit, each gets a full
+    // At most two launches, since launches of one stream wait for each other.
+    // Up to one replica per compute unit, each gets a full
     // workgroup; beyond that small ones take small workgroups, several to a
     // compute unit.  Large replicas first.
     const bool few = chosen.size() <= kComputeUnits;
@@ -240,28 +236,29 @@ void Batch::assignPaths() {
     }
 }
 
-// The resident launches of `substeps` substeps, beside whatever stream_ gets
-// next; join() makes stream_ wait for them.
+// The resident launches of `substeps` substeps: on the side stream, beside
+// the two-pass kernels that stream_ gets next; with no such replicas the last
+// launch goes to stream_ itself.  joinResident() makes stream_ wait for them.
 void Batch::launchResident(uint64_t substeps) {
     if (classes_.empty()) return;
-    hip_check(hipEventRecord(fork_, stream_), "hipEventRecord");
-    for (size_t q = 0; q < classes_.size(); ++q)
-        hip_check(hipStreamWaitEvent(side_[q], fork_, 0), "hipStreamWaitEvent");
+    const size_t onSide = classes_.size() - (twoPassUsed_ == 0 ? 1u : 0u);
+    if (onSide) {
+        hip_check(hipEventRecord(fork_, stream_), "hipEventRecord");
+        hip_check(hipStreamWaitEvent(side_, fork_, 0), "hipStreamWaitEvent");
+    }
     for (size_t k = 0; k < classes_.size(); ++k)
         for (uint64_t left = substeps; left > 0;) {
             const uint32_t part = uint32_t(std::min<uint64_t>(left, kResidentSubsteps));
-            hip_check(launch_resident_batch(dDescs_, dResident_, classes_[k], part, side_[k]),
+            hip_check(launch_resident_batch(dDescs_, dResident_, classes_[k], part, k < onSide ? side_ : stream_),
                       "launch resident sweep");
             left -= part;
         }
 }
 
 void Batch::joinResident() {
-    if (classes_.empty()) return;
-    for (size_t q = 0; q < classes_.size(); ++q) {
-        hip_check(hipEventRecord(sideDone_[q], side_[q]), "hipEventRecord");
-        hip_check(hipStreamWaitEvent(stream_, sideDone_[q], 0), "hipStreamWaitEvent");
-    }
+    if (classes_.size() + (twoPassUsed_ ? 1u : 0u) < 2u) return;
+    hip_check(hipEventRecord(sideDone_, side_), "hipEventRecord");
+    hip_check(hipStreamWaitEvent(stream_, sideDone_, 0), "hipStreamWaitEvent");
 }
 
 uint32_t Batch::tilesNeeded(const SystemLayout& L) const {

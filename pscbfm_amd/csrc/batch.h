@@ -118,7 +118,8 @@ private:
     uint32_t latticeKind_;
     uint32_t tileCap_, replicaCap_;
     LaunchShape shape_;
-    hipStream_t stream_ = nullptr;
+    std::vector<hipStream_t> streams_;
+    hipStream_t stream_ = nullptr;  // streams_[0]
     // device tables
     SysDesc* dDescs_ = nullptr;
     Tile* dTiles_ = nullptr;
@@ -132,15 +133,15 @@ private:
     std::vector<std::vector<uint32_t>> freeSlots_;  // per XCD
     std::vector<Replica> replicas_;
     uint32_t usedTiles_ = 0;  // of every live replica, whichever kernels sweep it
-    // Resident sweep: replicas by launch, and the streams the launches run on
+    // Resident sweep: replicas by launch, and the stream the launches run on
     // beside the two-pass kernels.
     bool pinned_ = false;
     uint32_t twoPassUsed_ = 0;  // live replicas on the two-pass kernels
     std::vector<ResidentClass> classes_;
     std::vector<uint32_t> residentIds_;
     uint32_t* dResident_ = nullptr;
-    hipStream_t side_[2] = {};
-    hipEvent_t sideDone_[2] = {};
+    hipStream_t side_ = nullptr;  // streams_[1]
+    hipEvent_t sideDone_ = nullptr;
     hipEvent_t fork_ = nullptr;
     bool growable_ = false;
     bool tablesDirty_ = true;

@@ -20,9 +20,12 @@
 #include "device_system.h"
 
 #include <algorithm>
+#include <chrono>
 #include <cstring>
 #include <limits>
+#include <map>
 #include <memory>
+#include <mutex>
 #include <sstream>
 #include <stdexcept>
 
@@ -34,6 +37,87 @@ void hip_fail(hipError_t e, const char* what) {
     std::ostringstream msg;
     msg << "HIP error in " << what << ": " << hipGetErrorName(e) << " (" << hipGetErrorString(e) << ")";
     throw std::runtime_error(msg.str());
+}
+
+namespace {
+
+struct StreamPool {
+    std::mutex mu;
+    std::map<std::pair<int, unsigned>, std::vector<std::vector<hipStream_t>>> idle;  // by (device, streams)
+};
+StreamPool& stream_pool() {
+    static StreamPool* pool = new StreamPool();  // never destroyed: owners may outlive static objects
+    return *pool;
+}
+constexpr size_t kMaxIdleSets = 16;
+
+}  // namespace
+
+namespace {
+
+// Milliseconds that a short fixed wait on each of the streams takes together.
+double wait_ms(const std::vector<hipStream_t>& streams) {
+    const auto t = std::chrono::steady_clock::now();
+    for (hipStream_t s : streams) hip_check(launch_wait(s), "launch wait");
+    for (hipStream_t s : streams) hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
+    return std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t).count();
+}
+
+// Whether kernels of the two streams run side by side.
+bool overlap(hipStream_t a, hipStream_t b) {
+    (void)wait_ms({a, b});  // their first kernels
+    const double alone = std::min(wait_ms({a}), wait_ms({a}));
+    return std::min(wait_ms({a, b}), wait_ms({a, b})) < 1.5 * alone;
+}
+
+}  // namespace
+
+std::vector<hipStream_t> acquire_streams(unsigned n) {
+    int device = 0;
+    hip_check(hipGetDevice(&device), "hipGetDevice");
+    StreamPool& pool = stream_pool();
+    std::lock_guard<std::mutex> lock(pool.mu);
+    auto& sets = pool.idle[{device, n}];
+    std::vector<hipStream_t> streams, rejected;
+    if (!sets.empty()) {
+        streams = std::move(sets.back());
+        sets.pop_back();
+        return streams;
+    }
+    try {
+        while (streams.size() < n) {
+            hipStream_t s = nullptr;
+            hip_check(hipStreamCreateWithFlags(&s, hipStreamNonBlocking), "hipStreamCreate");
+            rejected.push_back(s);
+            const bool apart = std::all_of(streams.begin(), streams.end(), [&](hipStream_t q) { return overlap(q, s); });
+            // after a few tries any stream does: it only does not overlap
+            if (apart || rejected.size() > 6) {
+                streams.push_back(s);
+                rejected.pop_back();
+            }
+        }
+    } catch (...) {
+        for (hipStream_t q : streams) (void)hipStreamDestroy(q);
+        for (hipStream_t q : rejected) (void)hipStreamDestroy(q);
+        throw;
+    }
+    for (hipStream_t q : rejected) (void)hipStreamDestroy(q);
+    return streams;
+}
+
+void release_streams(std::vector<hipStream_t>& streams, int device) {
+    if (streams.empty()) return;
+    bool good = true;
+    for (hipStream_t s : streams) good = hipStreamSynchronize(s) == hipSuccess && good;
+    StreamPool& pool = stream_pool();
+    std::lock_guard<std::mutex> lock(pool.mu);
+    auto& sets = pool.idle[{device, unsigned(streams.size())}];
+    if (good && sets.size() < kMaxIdleSets) {
+        sets.push_back(std::move(streams));
+    } else {
+        for (hipStream_t s : streams) (void)hipStreamDestroy(s);
+    }
+    streams.clear();
 }
 
 namespace {

@@ -22,7 +22,7 @@ struct LaunchShape {
     uint32_t listGroup = 0;
     uint32_t listDepth = 4;
     // The pass (1 or 2) of a single system's substep that zeroes the other
-    // parity's proposal buffer.  Batches clear in pass 2.
+    // parity's proposal buffer.  Batches clear in pass 1.
     uint32_t clearPass = 2;
     uint32_t passTwoBlock() const { return performBlock ? performBlock : block; }
     uint32_t listStride() const { return slots * block; }  // list entries per workgroup
@@ -112,6 +112,8 @@ struct UnfoldJob {
 };
 // xyz[3(out+i)..] = unfolded corner of monomer first+i of every job, i < count.
 hipError_t launch_unfold_jobs(const UnfoldJob* jobs, uint32_t nJobs, uint32_t blocks, int32_t* xyz, hipStream_t st);
+// One wave that sleeps for about 0.1 ms.
+hipError_t launch_wait(hipStream_t st);
 // Fills n 32-bit words with v (graph-safe replacement of a memset).
 hipError_t launch_fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t st);
 // Streaming copy of n16 16-byte elements (bandwidth and counter reference).

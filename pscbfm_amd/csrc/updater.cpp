@@ -414,10 +414,8 @@ void Updater::freeDevice() {
     if (drawTable_) (void)hipFree(drawTable_);
     drawTable_ = nullptr;
     drawCapacity_ = 0;
-    if (stream_) {
-        (void)hipStreamDestroy(stream_);
-        stream_ = nullptr;
-    }
+    release_streams(streams_, gpu_);
+    stream_ = nullptr;
 }
 
 // UpdaterGPUScBFM_AB_Type.cu:490-690
@@ -490,7 +488,8 @@ void Updater::initialize() {
     } else {
         hip_check(hipSetDevice(gpu_), "hipSetDevice");
     }
-    hip_check(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking), "hipStreamCreate");
+    if (streams_.empty()) streams_ = acquire_streams(1);
+    stream_ = streams_[0];
 
     cells_ = uint64_t(box_[0]) * box_[1] * box_[2];
     dev_.allocate(layout_, latticeKind_, seed_, /*withLists=*/true, uint32_t(max_grid(layout_.maxColorCount)),

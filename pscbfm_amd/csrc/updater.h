@@ -253,7 +253,8 @@ private:
     // device
     bool initialized_ = false;
     SystemLayout layout_;
-    hipStream_t stream_ = nullptr;
+    std::vector<hipStream_t> streams_;
+    hipStream_t stream_ = nullptr;  // streams_[0]
     DeviceSystem dev_;
     LaunchShape shape_;
     bool shapePinned_ = false;    // setLaunchShape stated a shape
