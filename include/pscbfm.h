@@ -139,11 +139,13 @@ int pscbfm_set_check_on_initialize(pscbfm_updater* h, int on);
 /* Replace the automatic coloring with a proper coloring given per monomer. */
 int pscbfm_set_colors(pscbfm_updater* h, const uint8_t* colors, uint32_t n);
 /* Threads per workgroup (64, 128, 192 or 256; 0 = 256) and monomers per
- * pass-1 thread (1, 2 or 4; 0 = 2).  Results do not depend on the shape. */
+ * pass-1 thread (1, 2 or 4; 0 = 2) of the two-pass kernels; both 0 (the
+ * default): chosen by size, and small systems run in one workgroup's LDS
+ * instead.  Results do not depend on the shape. */
 int pscbfm_set_launch_shape(pscbfm_updater* h, uint32_t block, uint32_t slots);
 /* Pass-2 threads per workgroup (64..256, multiple of 64; 0 = automatic:
- * 128 when at least a quarter of the cells are occupied, else the pass-1
- * block).  Results do not depend on it. */
+ * 128 with one monomer per pass-1 thread or at least a quarter of the cells
+ * occupied, else the pass-1 block).  Results do not depend on it. */
 int pscbfm_set_perform_block(pscbfm_updater* h, uint32_t block);
 /* Pass-2 walk of a single system: threads_per_list threads walk one pass-1
  * list (64..256, multiple of 64), so a pass-2 workgroup walks several lists,
@@ -348,7 +350,8 @@ int pscbfm_batch_footprint(pscbfm_batch* b, const pscbfm_updater* staged, uint64
 int pscbfm_batch_add(pscbfm_batch* b, const pscbfm_updater* staged, uint32_t* id);
 int pscbfm_batch_remove(pscbfm_batch* b, uint32_t id);
 /* Pass-2 threads per workgroup of the batch (0 = the default: the pass-1
- * block, at most 192). */
+ * block, at most 192).  A stated value also keeps every replica on the
+ * two-pass kernels. */
 int pscbfm_batch_set_perform_block(pscbfm_batch* b, uint32_t block);
 /* The replica stops after n_mcs more sweeps (counted from the last synchronize). */
 int pscbfm_batch_set_target(pscbfm_batch* b, uint32_t id, uint64_t n_mcs);

@@ -370,8 +370,8 @@ class UpdaterGPUScBFM_AB_Type:
         self._call("pscbfm_set_launch_shape", int(block), int(slots))
 
     def setPerformBlock(self, block: int = 0) -> None:
-        """Pass-2 threads per workgroup (0: automatic, 128 for systems at least a
-        quarter occupied, else the pass-1 block)."""
+        """Pass-2 threads per workgroup (0: automatic, 128 with one monomer per
+        pass-1 thread or at least a quarter occupied, else the pass-1 block)."""
         self._call("pscbfm_set_perform_block", int(block))
 
     def setPerformWalk(self, threads_per_list: int = 0, entries_per_thread: int = 0) -> None:

@@ -62,7 +62,7 @@ double time_system(const SystemLayout& L, uint32_t kind, uint64_t seed, LaunchSh
     DeviceSystem dev;
     dev.allocate(L, kind, seed, /*withLists=*/true, uint32_t(max_grid(L.maxColorCount)), st);
     s.grid = grid_for(L.maxColorCount, s.block * s.slots);
-    s.performBlock = automatic_perform_block(L, s.block);
+    s.performBlock = automatic_perform_block(L, s.block, s.slots);
     s.clearPass = automatic_clear_pass(L, kind);
     const uint32_t nc = std::max<uint32_t>(1u, uint32_t(L.colors.size()));
     const uint32_t g = nc;  // one sweep per replay
@@ -104,17 +104,39 @@ TuneResult pick(std::vector<TuneTrial> trials) {
 
 }  // namespace
 
-uint32_t automatic_perform_block(const SystemLayout& L, uint32_t block) {
-    // Pass 2 walks one compacted pass-1 list per workgroup.  In a dense
-    // system (at least a quarter of the cells occupied) a list holds about a
-    // fifth of its capacity, so 128 threads have about one entry each: on
-    // the 512^3 melt at 0.5 that sweeps 1.0% faster than 256 threads (1.9%
-    // when pass 2 also clears the proposals) and 64 threads 3.2% slower.
-    // Dilute systems have fuller lists and keep the pass-1 block (the
-    // replica mix at 0.1-0.5 runs pass 2 16% faster with 256 than with 128).
+namespace {
+double occupied_fraction(const SystemLayout& L) {
     const uint32_t log2Cells = L.codec.log2L[0] + L.codec.log2L[1] + L.codec.log2L[2];
-    const double occupied = 8.0 * double(L.nMonomers) / std::ldexp(1.0, int(log2Cells));
-    return occupied >= 0.25 && block > 128u ? 128u : 0u;
+    return 8.0 * double(L.nMonomers) / std::ldexp(1.0, int(log2Cells));
+}
+}  // namespace
+
+void automatic_shape(const SystemLayout& L, uint32_t latticeKind, uint32_t* block, uint32_t* slots) {
+    // Two monomers per thread keep more loads in flight per wave, one gives
+    // twice the waves.  Measured, 256 x 2 against the choice, us per substep
+    // by members of a species:
+    //   up to 2^15, 128 x 1: 8192 6.7 and 6.0 (uint8 7.5 and 6.3), 32768 6.7
+    //     and 6.1 (7.5 and 6.4); 256 x 1 takes 6.1 and 6.5 at 32768;
+    //   else 256 x 1: 65536 6.8 and 6.3, 2^18 8.3 and 8.2, uint8 2^19 12.8 and
+    //     12.3, dense network of 374,400 11.2 and 10.9, at occupied fraction
+    //     0.2 839,000 19.6 and 18.3, 1.7 million 30.1 and 28.6, uint8 2^22 55.9
+    //     and 55.1;
+    //   but 256 x 2 for more than 400,000 on the bit lattice at 0.4 or denser,
+    //     where the waves of 256 x 1 share the caches worse: 2^19 10.6 to 11.1
+    //     with 256 x 1 and 10.7, 2^20 15.4 and 15.2, 2^21 23.9 and 23.4.
+    const bool pairs = latticeKind == kLatticeBit && L.maxColorCount > 400000u && occupied_fraction(L) >= 0.4;
+    *block = L.maxColorCount <= (1u << 15) ? 128u : 256u;
+    *slots = pairs ? 2u : 1u;
+}
+
+uint32_t automatic_perform_block(const SystemLayout& L, uint32_t block, uint32_t slots) {
+    // Pass 2 walks one compacted pass-1 list per workgroup.  With one monomer
+    // per pass-1 thread, or in a dense system (at least a quarter of the cells
+    // occupied), a list of a 256-thread workgroup has about 128 entries or
+    // fewer: 128 threads against 256, us per substep, 18.3 and 18.7 (839,000
+    // members, fraction 0.2, 256 x 1), 38.8 and 39.2 (512^3 melt).  Dilute systems
+    // with two monomers per thread have fuller lists and keep the pass-1 block.
+    return (slots == 1u || occupied_fraction(L) >= 0.25) && block > 128u ? 128u : 0u;
 }
 
 uint32_t automatic_clear_pass(const SystemLayout& L, uint32_t latticeKind) {

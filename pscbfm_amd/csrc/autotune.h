@@ -25,11 +25,13 @@ struct TuneResult {
     bool cached = false;
 };
 
-// The choices a single system's shape makes by itself once its pass-1
-// block is set (the updater's defaults, also applied to every candidate
-// the autotuner times):
+// The shape of a single system's two-pass kernels where none is stated:
+// pass-1 threads per workgroup and monomers per thread.
+void automatic_shape(const SystemLayout& L, uint32_t latticeKind, uint32_t* block, uint32_t* slots);
+// The choices a single system's shape makes by itself once these are set (also
+// applied to every candidate the autotuner times):
 // pass-2 threads per workgroup, 0 = the pass-1 block;
-uint32_t automatic_perform_block(const SystemLayout& L, uint32_t block);
+uint32_t automatic_perform_block(const SystemLayout& L, uint32_t block, uint32_t slots);
 // the pass (1 or 2) that zeroes the other parity's proposal buffer.
 uint32_t automatic_clear_pass(const SystemLayout& L, uint32_t latticeKind);
 

@@ -232,7 +232,7 @@ struct DevState {
     // drawTable[2(t - drawBase)], [2(t - drawBase) + 1]; null = counter draw.
     const uint32_t* drawTable;
     uint64_t drawBase;
-    uint32_t* log;             // optional per-substep accepted counts
+    uint32_t* log;             // optional: accepted moves by substep (resident) or running totals (two-pass)
     uint64_t logFirst;         // substep index stored in log[0]
     uint64_t logCapacity;      // entries in log
     uint64_t* acceptedByBlock; // running totals of accepted moves

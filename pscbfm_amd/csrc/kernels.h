@@ -24,6 +24,8 @@ struct LaunchShape {
     // The pass (1 or 2) of a single system's substep that zeroes the other
     // parity's proposal buffer.  Batches clear in pass 1.
     uint32_t clearPass = 2;
+    // Entries of the accepted totals in use (by any shape so far), for the log.
+    uint32_t totals = 0;
     uint32_t passTwoBlock() const { return performBlock ? performBlock : block; }
     uint32_t listStride() const { return slots * block; }  // list entries per workgroup
     // Pass-1 lists each XCD produces: workgroup w runs on XCD w % 8 and
@@ -41,6 +43,9 @@ struct LaunchShape {
 // captured sequence of substeps stays valid for every replay.
 hipError_t launch_check(const SysDesc& d, uint32_t k, const LaunchShape& s, hipStream_t st);
 hipError_t launch_perform(const SysDesc& d, uint32_t k, const LaunchShape& s, hipStream_t st);
+// Completes the accepted log of the two-pass kernels: entry k of the log is then
+// the accepted moves of the system up to and with that substep, modulo 2^32.
+hipError_t launch_log_last(const DevState* state, const LaunchShape& s, hipStream_t st);
 // DevState::substep += count (after a block of substeps).
 hipError_t launch_advance(DevState* state, uint32_t count, hipStream_t st);
 

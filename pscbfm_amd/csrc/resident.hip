@@ -36,9 +36,12 @@ namespace pscbfm {
 namespace {
 
 // Largest species of a system on its own: us per substep, resident against two
-// passes, on 64^3: 4000 members 4.91 and 7.07, 4921 6.19 and 6.96 (byte
-// lattice 6.67 and 7.61), 6400 7.88 and 6.87.  Five rounds of 1024 threads.
-constexpr uint32_t kResidentMaxSpecies = 5120;
+// passes, on 64^3: 4000 members 4.9 and 6.0, 4921 6.2 and 6.0 (byte lattice 6.7
+// and 6.2).  Four and a half rounds of 1024 threads.
+constexpr uint32_t kResidentAlone = 4608;
+// Of a batch replica whatever else the batch holds: a batch of two-pass
+// replicas takes 7 us per substep or more.
+constexpr uint32_t kResidentInBatch = 5120;
 
 // LDS addresses.  The kernels have no static LDS, so their dynamic LDS starts
 // at address 0; plain numbers let the compiler put the fixed parts into the
@@ -357,7 +360,7 @@ uint64_t resident_lds_bytes(const SysDesc& d) {
 }
 
 uint32_t resident_block(const SysDesc& d) {
-    if (d.maxColorCount == 0u || d.maxColorCount > kResidentMaxSpecies || d.lone != 0u) return 0u;
+    if (d.maxColorCount == 0u || d.maxColorCount > kResidentAlone || d.lone != 0u) return 0u;
     const uint32_t block = std::min((d.maxColorCount + 63u) / 64u * 64u, 1024u);
     return resident_lds_bytes(d) <= kResidentLds ? block : 0u;
 }
@@ -374,7 +377,7 @@ bool resident_fits(const SysDesc& d) {
     return d.maxColorCount != 0u && d.maxColorCount <= 8u * 1024u && d.lone == 0u && resident_lds_bytes(d) <= kResidentLds;
 }
 
-bool resident_always(const SysDesc& d) { return d.maxColorCount <= kResidentMaxSpecies; }
+bool resident_always(const SysDesc& d) { return d.maxColorCount <= kResidentInBatch; }
 double resident_substep_us(const SysDesc& d) { return 1.0 + 1.1e-3 * double(d.maxColorCount); }
 
 hipError_t launch_resident_batch(const SysDesc* descs, const uint32_t* ids, const ResidentClass& c, uint32_t substeps,

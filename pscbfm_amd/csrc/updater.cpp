@@ -287,6 +287,7 @@ void Updater::setClearPass(uint32_t pass) {
 void Updater::applyLaunchShape() {
     shape_.block = blockOverride_ ? blockOverride_ : 256;
     shape_.slots = slotsOverride_ ? slotsOverride_ : 2;
+    if (!blockOverride_ && !slotsOverride_) automatic_shape(layout_, latticeKind_, &shape_.block, &shape_.slots);
     // Pass 2 walks one list per workgroup unless a list group is set: on the
     // 512^3 melt the multi-list walk was no faster (128 x 1: 89.5 against
     // 89.3 G attempts/s; 64 x 4: 84.1), pass 2 being bound by its writes.
@@ -296,7 +297,7 @@ void Updater::applyLaunchShape() {
         shape_.listGroup = walkGroupOverride_;
         shape_.listDepth = walkDepthOverride_ ? walkDepthOverride_ : 4;
     }
-    shape_.performBlock = performOverride_ ? performOverride_ : automatic_perform_block(layout_, shape_.block);
+    shape_.performBlock = performOverride_ ? performOverride_ : automatic_perform_block(layout_, shape_.block, shape_.slots);
     if (shape_.listGroup) {
         // several lists per workgroup: whole lists, at most 256 threads
         if (!performOverride_) shape_.performBlock = 256;
@@ -307,6 +308,7 @@ void Updater::applyLaunchShape() {
     shape_.clearPass = clearPassOverride_ ? clearPassOverride_ : automatic_clear_pass(layout_, latticeKind_);
     const uint32_t waveTotals = shape_.passTwoGrid() * (shape_.passTwoBlock() / 64u);
     acceptedMax_ = std::max(acceptedMax_, std::min(waveTotals, dev_.accEntries));
+    shape_.totals = acceptedMax_;
     const bool pinned = shapePinned_ || performOverride_ || walkGroupOverride_ || clearPassOverride_;
     residentBlock_ = pinned ? 0u : resident_block(dev_.desc);
     dropGraphs();
@@ -613,6 +615,7 @@ void Updater::runImpl(int32_t nMCS, uint32_t* log, bool profile, bool useGraph, 
     const uint64_t drawCap = drawChunk_ ? std::min(drawChunk_, kMaxDrawSubsteps) : kMaxDrawSubsteps;
     const uint64_t chunk = r250Mode_ && !scratch ? std::max<uint64_t>(1u, drawCap / nc) * nc : S;
     RunStats total{};
+    loggedTotal_ = uint32_t(acceptedTotal_);
     for (uint64_t done = 0; done < S; done += chunk) {
         const uint64_t part = std::min(chunk, S - done);
         runChunk(part, log ? log + done : nullptr, profile, useGraph, scratch);
@@ -750,6 +753,7 @@ void Updater::runChunk(uint64_t S, uint32_t* log, bool profile, bool useGraph, v
             left -= blk;
         }
     }
+    if (log && !resident) hip_check(launch_log_last(dev_.desc.state, shape_, stream_), "launch log");
     if (scratch) {
         hip_check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
         lastRun_.gpuMilliseconds =
@@ -782,7 +786,15 @@ void Updater::runChunk(uint64_t S, uint32_t* log, bool profile, bool useGraph, v
     lastRun_.substeps = S;
     substep_ += S;
 
-    if (log) hip_check(hipMemcpy(log, dLog, S * 4, hipMemcpyDeviceToHost), "log D2H");
+    if (log) {
+        hip_check(hipMemcpy(log, dLog, S * 4, hipMemcpyDeviceToHost), "log D2H");
+        if (!resident)  // running totals
+            for (uint64_t k = 0; k < S; ++k) {
+                const uint32_t total = log[k];
+                log[k] = total - loggedTotal_;
+                loggedTotal_ = total;
+            }
+    }
     if (patched) {
         DevState patch = dev_.readState(stream_);
         patch.log = nullptr;

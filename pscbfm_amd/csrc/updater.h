@@ -99,7 +99,8 @@ public:
     void setUniformColoring(bool on) { uniformColors_ = on; }
     void setCheckOnInitialize(bool on) { checkOnInit_ = on; }
     void setColors(const uint8_t* colors, uint32_t n);
-    // Threads per workgroup (0 = 256) and monomers per pass-1 thread (0 = 2).
+    // Threads per workgroup (0 = 256) and monomers per pass-1 thread (0 = 2);
+    // both 0: by size (automatic_shape).
     // A system small enough for the resident sweep (resident_block, kernels.h)
     // runs that instead, unless this, setPerformBlock, setPerformWalk or
     // setClearPass states a shape of the two-pass kernels.
@@ -116,8 +117,7 @@ public:
     // that the run's first launch starts at once (a run builds what is
     // missing itself, before its timing starts).
     void prepareGraphs(int32_t nMCS);
-    // Pass-2 threads per workgroup (0 = automatic: 128 for systems at least a
-    // quarter occupied, else the pass-1 block).
+    // Pass-2 threads per workgroup (0 = automatic_perform_block).
     void setPerformBlock(uint32_t block);
     // Pass-2 walk: `group` threads per pass-1 list (64..256, multiple of 64)
     // with `depth` entries per thread in flight (1 or 4; 0 = 4); group 0 or
@@ -263,6 +263,7 @@ private:
     uint32_t acceptedMax_ = 0;  // entries of acceptedByBlock that any launch shape so far uses
     uint64_t substep_ = 0;
     uint64_t acceptedTotal_ = 0;
+    uint32_t loggedTotal_ = 0;  // accepted total before the log's next entry, modulo 2^32
     std::vector<uint64_t> degreeSum_;  // bonds of each species' members
     hipEvent_t timing_[2] = {};        // around the timed part of a run
     uint64_t cells_ = 0;

@@ -3,8 +3,9 @@ oracle and the two-pass kernels, which setLaunchShape pins.
 
 All results are whole numbers, so every comparison is exact.  Sizes are chosen
 around the workgroup's rounds: a species of 64 and 65 members (one wave and
-two), 1024 and 1025 (one round and two), and 5120 and 5121 (the largest that
-runs resident and the first that does not)."""
+two), 1024 and 1025 (one round and two), 4608 and 4609 (the largest that runs
+resident alone and the first that does not), and 5120 and 5121 (the same for
+a batch replica)."""
 import numpy as np
 import pytest
 
@@ -27,8 +28,8 @@ SYSTEMS = {
     "two_waves": lambda: _dimers((32, 32, 32), 65),
     "one_round": lambda: _dimers((64, 32, 32), 1024),
     "two_rounds": lambda: _dimers((64, 32, 32), 1025),
-    "five_rounds": lambda: _dimers((64, 64, 64), 5120),
-    "too_large": lambda: _dimers((64, 64, 64), 5121),
+    "five_rounds": lambda: _dimers((64, 64, 64), 4608),
+    "too_large": lambda: _dimers((64, 64, 64), 4609),
     "smallest_box": lambda: chains((8, 8, 8), 2, 5, seed=3),
     "flat_box": lambda: chains((64, 16, 8), 9, 21, seed=4),
     "network": lambda: stars((64, 64, 64), 60, 4, 7, seed=5),
@@ -123,7 +124,7 @@ def _batch_systems():
     """Replicas of every path: resident always (up to 5120 members), resident
     only beside long two-pass work (beyond), too large for LDS, and one whose
     monomers without bonds the resident sweep does not take."""
-    return [chains((32, 32, 32), 24, 16, seed=1), ordered_chains((64, 64, 64), 800, 16),
+    return [chains((32, 32, 32), 24, 16, seed=1), _dimers((64, 64, 64), 5120), _dimers((64, 64, 64), 5121), ordered_chains((64, 64, 64), 800, 16),
             stars((64, 64, 32), 30, 4, 9, seed=2), chains((128, 64, 128), 100, 50, seed=3),
             chains((32, 32, 32), 80, 1, seed=4), chains((16, 64, 32), 30, 11, seed=5),
             chains((128, 128, 64), 20, 40, seed=6)]
