@@ -29,6 +29,11 @@ namespace pscbfm {
 // A pointer into global memory, as the ISA's GLOBAL instructions address it.
 template <class T>
 using gptr = __attribute__((address_space(1))) T*;
+// The same memory where no kernel that reads it this way writes it: the
+// compiler then takes uniform loads through the scalar cache wherever they
+// stand, also below stores it cannot tell apart.
+template <class T>
+using cptr = const __attribute__((address_space(4))) T*;
 #endif
 
 // A device buffer as a descriptor carries it.  Host code stores and reads the

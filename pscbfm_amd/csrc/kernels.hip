@@ -44,8 +44,7 @@ namespace pscbfm {
 namespace {
 
 // Logical workgroup id: consecutive ids on the same XCD.
-__device__ __forceinline__ uint32_t xcd_block() {
-    const uint32_t nb = gridDim.x;  // multiple of 8 (grid_for)
+__device__ __forceinline__ uint32_t xcd_block(uint32_t nb) {  // nb: a multiple of 8 (grid_for)
     return (blockIdx.x & 7u) * (nb >> 3) + (blockIdx.x >> 3);
 }
 
@@ -90,13 +89,15 @@ __device__ __forceinline__ void check_body(const SysDesc& d, uint64_t t, Substep
     const ColorInfo ci = load_color(d.colors.global(), draw.species);
     const gptr<uint32_t> proposal = d.proposal.global();
 
-    // The bond table (16 words, the same for every lane: scalar loads) goes
-    // to LDS after the gathers below are issued, and the barrier that
-    // publishes it stands in front of the bond test.  A barrier ahead of the
-    // gathers held every wave's loads back by the table's round trip.
-    uint32_t forbidden[16];
-#pragma unroll
-    for (int w = 0; w < 16; ++w) forbidden[w] = d.bondMask.global()[w];
+    // The bond table goes to LDS after the gathers below are issued, and the
+    // barrier that publishes it stands in front of the bond test.  A barrier
+    // ahead of the gathers held every wave's loads back by the table's round
+    // trip.  Its words are loaded by a lane each, before the gathers: as scalar
+    // loads they were moved down to where one lane stored them, and the barrier
+    // waited for them there (us per substep, 128^3 melt 6.2 and 6.1, 256^3 uint8
+    // 12.4 and 12.2).
+    uint32_t forbidden = 0;
+    if (threadIdx.x < 16u) forbidden = d.bondMask.global()[threadIdx.x];
 
     const uint32_t B = blockDim.x;
     const uint32_t base = lb * (SLOTS * B);
@@ -114,7 +115,7 @@ __device__ __forceinline__ void check_body(const SysDesc& d, uint64_t t, Substep
     uint32_t rb[MAXDEG];
 #pragma unroll
     for (int r = 0; r < MAXDEG; ++r)
-        rb[r] = LAT == kLatticeU8 ? d.rowBase.global()[draw.species * kMaxConnectivity + uint32_t(r)] : 0u;
+        rb[r] = LAT == kLatticeU8 ? ((cptr<uint32_t>)d.rowBase.global())[draw.species * kMaxConnectivity + uint32_t(r)] : 0u;
     const gptr<const uint64_t> lattice = (gptr<const uint64_t>)d.lattice.global();
     const AxisMasks masks = axis_masks(d);
 
@@ -186,11 +187,8 @@ __device__ __forceinline__ void check_body(const SysDesc& d, uint64_t t, Substep
             partnerCode[s][r] = posAll[partner[s][r] != kNoNeighbor ? partner[s][r] : 0u];
         if constexpr (!kBondsFirst) occ[s] = plane_any<kShift>(lattice, m[s], dir[s], mv[s]);
     }
-    if (threadIdx.x == 0) {
-#pragma unroll
-        for (int w = 0; w < 16; ++w) sForbidden[w] = forbidden[w];
-        *sCount = 0;
-    }
+    if (threadIdx.x < 16u) sForbidden[threadIdx.x] = forbidden;
+    if (threadIdx.x == 0) *sCount = 0;
     __syncthreads();
     bool ok[SLOTS];
 #pragma unroll
@@ -280,10 +278,10 @@ __device__ __forceinline__ void add_accepted(const AcceptedTotal& a, uint32_t ac
 
 // The accepted log.  A count per wave and substep, added to the substep's
 // entry, had hundreds of atomics on one address end pass 2 (9.5 instead of 6.7
-// us per substep for 32768 members).  Instead one workgroup of pass 1 sums the
-// waves' running totals and writes the sum, modulo 2^32, as the entry of the
-// substep before; the last substep's is written by k_log_last.  The host takes
-// differences.
+// us per substep for 32768 members).  Instead pass 1 of a logged run has one
+// workgroup more, which sums the waves' running totals and writes the sum,
+// modulo 2^32, as the entry of the substep before; the last substep's is written
+// by k_log_last.  The host takes differences.
 __device__ __forceinline__ void log_totals(gptr<const uint64_t> totals, uint32_t n, gptr<uint32_t> log, uint64_t entry,
                                            uint64_t capacity) {
     if (entry >= capacity) return;
@@ -293,6 +291,14 @@ __device__ __forceinline__ void log_totals(gptr<const uint64_t> totals, uint32_t
     for (int w = 32; w > 0; w >>= 1) sum += uint32_t(__shfl_xor(int(sum), w, 64));
     if ((threadIdx.x & 63u) == 0u)
         __hip_atomic_fetch_add(&log[entry], sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The log's entry of the substep before the one that offset k serves.
+__device__ __forceinline__ void log_before(gptr<const DevState> st, uint32_t k, uint32_t totals) {
+    const uint64_t t = st->substep + k;
+    if (st->log != nullptr && t <= st->stopAt)
+        log_totals((gptr<const uint64_t>)st->acceptedByBlock, totals, (gptr<uint32_t>)st->log, t - 1u - st->logFirst,
+                   st->logCapacity);
 }
 
 // Applies an accepted move of the monomer in `slot` from code m in
@@ -361,32 +367,32 @@ __device__ __forceinline__ void perform_body(const SysDesc& d, const Launch& L, 
 
 // ---- single system ----------------------------------------------------------------
 template <int LAT, int SLOTS, int MAXDEG, bool KEYED>
-__global__ __launch_bounds__(256) void k_check(SysDesc d, uint32_t k, uint32_t clear, uint32_t totals) {
+__global__ __launch_bounds__(256) void k_check(SysDesc d, uint32_t k, uint32_t clear, uint32_t nb,
+                                                                     uint32_t totals) {
     __shared__ uint32_t sForbidden[16];
     __shared__ uint32_t sCount;
+    if (blockIdx.x >= nb) {  // the log's own workgroup
+        log_before(d.state.global(), k, totals);
+        return;
+    }
     Launch L;
     if (!begin_substep(d, k, L)) return;
-    const uint32_t lb = xcd_block();
-    check_body<LAT, SLOTS, MAXDEG, KEYED>(d, L.t, L.draw, lb, gridDim.x, clear != 0u,
+    const uint32_t lb = xcd_block(nb);
+    check_body<LAT, SLOTS, MAXDEG, KEYED>(d, L.t, L.draw, lb, nb, clear != 0u,
                                    (gptr<uint64_t>)d.list.global() + size_t(lb) * (SLOTS * blockDim.x),
                                    d.listCount.global() + lb, sForbidden, &sCount);
-    if (L.log != nullptr && lb == 0u)
-        log_totals(L.acceptedByBlock, totals, L.log, L.t - 1u - L.logFirst, L.logCapacity);
 }
 
 // After the last substep of a logged run (the state's counter stands past it).
 __global__ __launch_bounds__(256) void k_log_last(const DevState* state, uint32_t totals) {
-    const gptr<const DevState> st = (gptr<const DevState>)state;
-    if (st->log != nullptr)
-        log_totals((gptr<const uint64_t>)st->acceptedByBlock, totals, (gptr<uint32_t>)st->log,
-                   st->substep - 1u - st->logFirst, st->logCapacity);
+    log_before((gptr<const DevState>)state, 0u, totals);
 }
 
 template <int LAT>
 __global__ __launch_bounds__(256) void k_perform(SysDesc d, uint32_t k, uint32_t listStride, uint32_t clear) {
     Launch L;
     if (!begin_substep(d, k, L)) return;
-    const uint32_t lb = xcd_block();  // same numbering as pass 1: list lb
+    const uint32_t lb = xcd_block(gridDim.x);  // same numbering as pass 1: list lb
     perform_body<LAT>(d, L, lb, gridDim.x, clear != 0u,
                       (gptr<const uint64_t>)d.list.global() + size_t(lb) * listStride, d.listCount.global()[lb],
                       blockIdx.x);
@@ -459,12 +465,17 @@ __global__ __launch_bounds__(256) void k_perform_lists(SysDesc d, uint32_t k, ui
 // ---- batch of replicas ---------------------------------------------------------------
 // Workgroup w serves tiles[w]: chunk `chunk` of `chunks` of replica `replica`.
 // Lists are indexed by w, accepted counts by (replica, chunk).
+__device__ __forceinline__ Tile load_tile(const Tile* tiles, uint32_t w) {
+    const cptr<uint32_t> p = (cptr<uint32_t>)(const uint32_t*)(tiles + w);
+    return Tile{p[0], p[1], p[2], 0u};
+}
+
 template <int LAT, int SLOTS, int MAXDEG>
 __global__ __launch_bounds__(256) void k_check_batch(const SysDesc* __restrict__ descs, const Tile* __restrict__ tiles,
                                                      uint2* lists, uint32_t* listCounts, uint32_t k) {
     __shared__ uint32_t sForbidden[16];
     __shared__ uint32_t sCount;
-    const Tile tile = tiles[blockIdx.x];
+    const Tile tile = load_tile(tiles, blockIdx.x);
     if (tile.replica == kNoReplica) return;
     const SysDesc& d = descs[tile.replica];
     Launch L;
@@ -486,7 +497,7 @@ template <int LAT>
 __global__ __launch_bounds__(256) void k_perform_batch(const SysDesc* __restrict__ descs,
                                                        const Tile* __restrict__ tiles, const uint2* lists,
                                                        const uint32_t* listCounts, uint32_t k, uint32_t listStride) {
-    const Tile tile = tiles[blockIdx.x];
+    const Tile tile = load_tile(tiles, blockIdx.x);
     if (tile.replica == kNoReplica) return;
     const SysDesc& d = descs[tile.replica];
     Launch L;
@@ -621,11 +632,11 @@ void check_launch(const SysDesc& d, const BatchLaunch* b, uint32_t k, const Laun
         hipLaunchKernelGGL((k_check_batch<LAT, SLOTS, MAXDEG>), dim3(b->tiles), blk, 0, st, b->descs, b->tileTable,
                            b->lists, b->listCounts, k);
     else if (d.keyed != 0u)
-        hipLaunchKernelGGL((k_check<LAT, SLOTS, MAXDEG, true>), dim3(s.grid), blk, 0, st, d, k,
-                           uint32_t(s.clearPass == 1u), s.totals);
+        hipLaunchKernelGGL((k_check<LAT, SLOTS, MAXDEG, true>), dim3(s.grid + (s.logged ? 1u : 0u)), blk, 0, st, d, k,
+                           uint32_t(s.clearPass == 1u), s.grid, s.totals);
     else
-        hipLaunchKernelGGL((k_check<LAT, SLOTS, MAXDEG, false>), dim3(s.grid), blk, 0, st, d, k,
-                           uint32_t(s.clearPass == 1u), s.totals);
+        hipLaunchKernelGGL((k_check<LAT, SLOTS, MAXDEG, false>), dim3(s.grid + (s.logged ? 1u : 0u)), blk, 0, st, d, k,
+                           uint32_t(s.clearPass == 1u), s.grid, s.totals);
 }
 
 template <int LAT, int SLOTS>

@@ -42,7 +42,7 @@ __device__ __forceinline__ uint64_t join64(uint32_t lo, uint32_t hi) { return ui
 // draw is entry t - drawBase of the explicit table when the state holds one,
 // else the counter draw of (seed, t).
 __device__ __forceinline__ bool begin_substep(const SysDesc& d, uint32_t k, Launch& out) {
-    const gptr<const u32x4> w = (gptr<const u32x4>)d.state.global();
+    const cptr<u32x4> w = (cptr<u32x4>)d.state.global();
     const u32x4 w0 = w[0], w1 = w[1], w2 = w[2], w3 = w[3];  // DevState field order
     const uint64_t t = join64(w0.x, w0.y) + k;
     // A state whose draw table, log or accepted counts are not aligned to
@@ -67,9 +67,9 @@ __device__ __forceinline__ bool begin_substep(const SysDesc& d, uint32_t k, Laun
     return true;
 }
 
-// Species record, read word by word through a global pointer.
+// Species record, read word by word.
 __device__ __forceinline__ ColorInfo load_color(gptr<const ColorInfo> colors, uint32_t species) {
-    const gptr<const uint32_t> w = (gptr<const uint32_t>)(colors + species);
+    const cptr<uint32_t> w = (cptr<uint32_t>)(colors + species);
     ColorInfo c{};
     c.slotOffset = w[offsetof(ColorInfo, slotOffset) / 4];
     c.count = w[offsetof(ColorInfo, count) / 4];
