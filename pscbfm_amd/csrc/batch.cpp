@@ -86,7 +86,7 @@ void Batch::growTiles(uint32_t needed) {
     dTiles_ = tiles;
     dLists_ = lists;
     dListCounts_ = counts;
-    tiles_.resize(needed, Tile{kNoReplica, 0, 0, 0});
+    tiles_.resize(needed, Tile{});
     for (uint32_t w = needed; w-- > tileCap_;) freeSlots_[w % 8].push_back(w);
     for (auto& f : freeSlots_) std::sort(f.begin(), f.end(), std::greater<uint32_t>());  // pop_back = lowest
     tileCap_ = needed;
@@ -159,14 +159,14 @@ void Batch::takeTiles(uint32_t id) {
             }
         }
     }
-    for (uint32_t c = 0; c < nT; ++c) tiles_[r.tileSlots[c]] = Tile{id, c, nT, 0};
+    for (uint32_t c = 0; c < nT; ++c) tiles_[r.tileSlots[c]] = Tile{id, c, nT, descs_[id].nColors, descs_[id].state, descs_[id].seed};
 }
 
 void Batch::releaseTiles(uint32_t id) {
     Replica& r = replicas_[id];
     if (r.tileSlots.empty()) return;
     for (uint32_t w : r.tileSlots) {
-        tiles_[w] = Tile{kNoReplica, 0, 0, 0};
+        tiles_[w] = Tile{};
         freeSlots_[w % 8].push_back(w);
     }
     for (auto& f : freeSlots_) std::sort(f.begin(), f.end(), std::greater<uint32_t>());

@@ -246,14 +246,19 @@ static_assert(sizeof(DevState) == 64, "DevState is one 64-byte line");
 static_assert(offsetof(DevState, drawBase) == 24, "the launch words are the first 32 bytes");
 
 // Workgroup assignment of a batched launch: chunk `chunk` of the `chunks`
-// workgroups that cover replica `replica` (kNoReplica: idle workgroup).
+// workgroups that cover replica `replica` (kNoReplica: idle workgroup).  With it
+// what the substep's draw needs of the replica, so that a workgroup reads the
+// state beside the descriptor and not behind it.
 constexpr uint32_t kNoReplica = 0xFFFFFFFFu;
 struct Tile {
-    uint32_t replica;
-    uint32_t chunk;
-    uint32_t chunks;
-    uint32_t pad_;
+    uint32_t replica = kNoReplica;
+    uint32_t chunk = 0;
+    uint32_t chunks = 0;
+    uint32_t nColors = 0;
+    DeviceBuffer<DevState> state{};
+    uint64_t seed = 0;
 };
+static_assert(sizeof(Tile) == 32 && offsetof(Tile, state) == 16, "read as eight words");
 
 // Everything a sweep kernel needs to know about one system.
 struct SysDesc {
@@ -284,6 +289,8 @@ struct SysDesc {
     uint32_t lone;           // 1: some monomer has no bond
     uint32_t resident;       // 1: a batch replica that the resident sweep advances
     uint32_t keyed;          // 1: slots in spatial order, read the draw keys; 0: hash the slot index
+    uint32_t pad_[2];
 };
+static_assert(sizeof(SysDesc) == 192, "the descriptors of a table are three 64-byte lines each");
 
 }  // namespace pscbfm

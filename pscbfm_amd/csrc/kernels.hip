@@ -224,7 +224,7 @@ __device__ __forceinline__ void check_body(const SysDesc& d, uint64_t t, Substep
     }
     uint32_t waveBase = 0;
     if (lane == 0 && total != 0) waveBase = atomicAdd(sCount, total);
-    waveBase = __shfl(waveBase, 0, 64);
+    waveBase = uint32_t(__builtin_amdgcn_readfirstlane(int32_t(waveBase)));
 #pragma unroll
     for (int s = 0; s < SLOTS; ++s) {
         if (ok[s]) {
@@ -329,12 +329,13 @@ __device__ __forceinline__ void apply_move(const SysDesc& d, gptr<uint32_t> pos,
     }
 }
 
-// Pass 2 of substep t over one pass-1 list.  The accepted count is added to
-// the totals of workgroup `owner` of nb.  With `clear` it also zeroes slice lb
-// of nb of the other parity's proposals.
+// Pass 2 of substep t over one pass-1 list of `count` entries, the thread's
+// first of them loaded.  The accepted count is added to the totals of workgroup
+// `owner` of nb.  With `clear` it also zeroes slice lb of nb of the other
+// parity's proposals.
 template <int LAT>
 __device__ __forceinline__ void perform_body(const SysDesc& d, const Launch& L, uint32_t lb, uint32_t nb, bool clear,
-                                             gptr<const uint64_t> list, uint32_t count, uint32_t owner) {
+                                             gptr<const uint64_t> list, uint32_t count, uint64_t e, uint32_t owner) {
     const uint64_t t = L.t;
     const SubstepDraw draw = L.draw;
     const ColorInfo ci = load_color(d.colors.global(), draw.species);
@@ -350,19 +351,30 @@ __device__ __forceinline__ void perform_body(const SysDesc& d, const Launch& L, 
     const gptr<uint8_t> lat = d.lattice.global();
 
     // The list is compacted, so about a fifth of its capacity is filled: walk
-    // only the entries that exist, one per thread and round.
+    // only the entries that exist, one per thread and round.  The first round
+    // stands alone: as the loop's first it waited for every load before it, the
+    // running total's too (us per substep, 128^3 melt 6.03 and 5.83, dense star
+    // network 10.95 and 10.65).
     uint32_t accepted = 0;
-    for (uint32_t idx = threadIdx.x; idx < count; idx += B) {
-        const uint64_t e = list[idx];
-        const uint32_t jj = uint32_t(e) & ((1u << kDirShift) - 1u);
-        const Dir dir = dir_of_number(uint32_t(e) >> kDirShift);
-        const uint32_t m = uint32_t(e >> 32);
+    auto resolve = [&](uint64_t entry) {
+        const uint32_t jj = uint32_t(entry) & ((1u << kDirShift) - 1u);
+        const Dir dir = dir_of_number(uint32_t(entry) >> kDirShift);
+        const uint32_t m = uint32_t(entry >> 32);
         const Move mv = make_move(m, dir, masks);
-        if (plane_any<6>(T64, m, dir, mv)) continue;
+        if (plane_any<6>(T64, m, dir, mv)) return;
         apply_move<LAT>(d, pos, lat, ci.slotOffset + jj, m, dir, masks, mv);
         ++accepted;
-    }
+    };
+    if (threadIdx.x < count) resolve(e);
+    for (uint32_t idx = threadIdx.x + B; idx < count; idx += B) resolve(list[idx]);
     add_accepted(total, accepted);
+}
+
+// A list's length by a vector load, so that it is in flight with the state
+// (mbcnt of no lanes is 0: an address per lane; as a scalar load it was issued
+// behind the wait for the state).
+__device__ __forceinline__ uint32_t list_count(gptr<const uint32_t> count) {
+    return uint32_t(__builtin_amdgcn_readfirstlane(int32_t(count[__builtin_amdgcn_mbcnt_lo(0u, 0u)])));
 }
 
 // ---- single system ----------------------------------------------------------------
@@ -376,7 +388,7 @@ __global__ __launch_bounds__(256) void k_check(SysDesc d, uint32_t k, uint32_t c
         return;
     }
     Launch L;
-    if (!begin_substep(d, k, L)) return;
+    if (!begin_substep(d, k, Early{}, L)) return;
     const uint32_t lb = xcd_block(nb);
     check_body<LAT, SLOTS, MAXDEG, KEYED>(d, L.t, L.draw, lb, nb, clear != 0u,
                                    (gptr<uint64_t>)d.list.global() + size_t(lb) * (SLOTS * blockDim.x),
@@ -390,12 +402,13 @@ __global__ __launch_bounds__(256) void k_log_last(const DevState* state, uint32_
 
 template <int LAT>
 __global__ __launch_bounds__(256) void k_perform(SysDesc d, uint32_t k, uint32_t listStride, uint32_t clear) {
-    Launch L;
-    if (!begin_substep(d, k, L)) return;
     const uint32_t lb = xcd_block(gridDim.x);  // same numbering as pass 1: list lb
-    perform_body<LAT>(d, L, lb, gridDim.x, clear != 0u,
-                      (gptr<const uint64_t>)d.list.global() + size_t(lb) * listStride, d.listCount.global()[lb],
-                      blockIdx.x);
+    const gptr<const uint64_t> list = (gptr<const uint64_t>)d.list.global() + size_t(lb) * listStride;
+    Launch L;
+    if (!begin_substep(d, k, early_of(d, false), L)) return;
+    const uint32_t count = ((cptr<uint32_t>)d.listCount.global())[lb];
+    const uint64_t e = threadIdx.x < count ? list[threadIdx.x] : 0u;
+    perform_body<LAT>(d, L, lb, gridDim.x, clear != 0u, list, count, e, blockIdx.x);
 }
 
 // Pass 2 of a single system with several lists per workgroup: each group
@@ -419,7 +432,7 @@ __global__ __launch_bounds__(256) void k_perform_lists(SysDesc d, uint32_t k, ui
 #pragma unroll
     for (int r = 0; r < DEPTH; ++r) e[r] = list[min(lane + uint32_t(r) * group, listStride - 1u)];
     Launch L;
-    if (!begin_substep(d, k, L)) return;
+    if (!begin_substep(d, k, early_of(d, false), L)) return;
     if (!haveList) count = 0;
     const AcceptedTotal total = accepted_total(L, d, blockIdx.x, gridDim.x);
     const uint64_t t = L.t;
@@ -465,9 +478,22 @@ __global__ __launch_bounds__(256) void k_perform_lists(SysDesc d, uint32_t k, ui
 // ---- batch of replicas ---------------------------------------------------------------
 // Workgroup w serves tiles[w]: chunk `chunk` of `chunks` of replica `replica`.
 // Lists are indexed by w, accepted counts by (replica, chunk).
-__device__ __forceinline__ Tile load_tile(const Tile* tiles, uint32_t w) {
-    const cptr<uint32_t> p = (cptr<uint32_t>)(const uint32_t*)(tiles + w);
-    return Tile{p[0], p[1], p[2], 0u};
+// A workgroup of a few waves spends its time on round trips that depend on each
+// other: tile; state, descriptor and (pass 2) list together; species; monomers.
+// With the state behind the descriptor, and the list behind the state, the mix
+// of 256 systems took 111.0 ms for 2000 sweeps and 96 small byte-lattice systems
+// 14.7 for 1000; so 107.7 and 13.6.  (A single system's descriptor comes with
+// the launch, and its list is read behind the state: ahead of it the dense star
+// network took 10.84 us per substep against 10.65.)
+typedef uint32_t u32x8 __attribute__((ext_vector_type(8)));
+struct TileRef {
+    uint32_t replica, chunk, chunks, nColors;
+    gptr<DevState> state;
+    uint64_t seed;
+};
+__device__ __forceinline__ TileRef load_tile(const Tile* tiles, uint32_t w) {
+    const u32x8 v = *(cptr<u32x8>)(const u32x8*)(tiles + w);
+    return {v[0], v[1], v[2], v[3], (gptr<DevState>)(uintptr_t(join64(v[4], v[5]))), join64(v[6], v[7])};
 }
 
 template <int LAT, int SLOTS, int MAXDEG>
@@ -475,11 +501,12 @@ __global__ __launch_bounds__(256) void k_check_batch(const SysDesc* __restrict__
                                                      uint2* lists, uint32_t* listCounts, uint32_t k) {
     __shared__ uint32_t sForbidden[16];
     __shared__ uint32_t sCount;
-    const Tile tile = load_tile(tiles, blockIdx.x);
-    if (tile.replica == kNoReplica) return;
+    const TileRef tile = load_tile(tiles, blockIdx.x);
+    // never null: named here so that they are loaded with the table's address
+    if (tile.replica == kNoReplica || descs == nullptr || lists == nullptr || listCounts == nullptr) return;
     const SysDesc& d = descs[tile.replica];
     Launch L;
-    if (!begin_substep(d, k, L)) return;
+    if (!begin_substep(tile.state, tile.seed, tile.nColors, k, early_of(d, true), L)) return;
     const gptr<uint64_t> list = global_ptr(reinterpret_cast<uint64_t*>(lists)) + size_t(blockIdx.x) * (SLOTS * blockDim.x);
     // The proposals are cleared here (the mix of 256 systems, whose small ones
     // run resident: 108.8 against 112.3 ms for 2000 sweeps with the clear in
@@ -497,14 +524,17 @@ template <int LAT>
 __global__ __launch_bounds__(256) void k_perform_batch(const SysDesc* __restrict__ descs,
                                                        const Tile* __restrict__ tiles, const uint2* lists,
                                                        const uint32_t* listCounts, uint32_t k, uint32_t listStride) {
-    const Tile tile = load_tile(tiles, blockIdx.x);
-    if (tile.replica == kNoReplica) return;
+    const TileRef tile = load_tile(tiles, blockIdx.x);
+    // never null: named here so that they are loaded with the table's address
+    if (tile.replica == kNoReplica || descs == nullptr || lists == nullptr || listCounts == nullptr) return;
     const SysDesc& d = descs[tile.replica];
+    const gptr<const uint64_t> list = global_ptr(reinterpret_cast<const uint64_t*>(lists)) + size_t(blockIdx.x) * listStride;
+    Early early = early_of(d, false);
+    early.count = list_count(global_ptr(listCounts) + blockIdx.x);
+    early.entry = list[min(threadIdx.x, listStride - 1u)];  // past the count: dropped
     Launch L;
-    if (!begin_substep(d, k, L)) return;
-    perform_body<LAT>(d, L, tile.chunk, tile.chunks, false,
-                      global_ptr(reinterpret_cast<const uint64_t*>(lists)) + size_t(blockIdx.x) * listStride,
-                      global_ptr(listCounts)[blockIdx.x], tile.chunk);
+    if (!begin_substep(tile.state, tile.seed, tile.nColors, k, early, L)) return;
+    perform_body<LAT>(d, L, tile.chunk, tile.chunks, false, list, early.count, early.entry, tile.chunk);
 }
 
 __global__ void k_advance(DevState* st, uint32_t count) {

@@ -38,22 +38,45 @@ struct Launch {
 
 __device__ __forceinline__ uint64_t join64(uint32_t lo, uint32_t hi) { return uint64_t(lo) | (uint64_t(hi) << 32); }
 
+// What a kernel loads ahead of its branch on the state, and waits for with the
+// state.  The compiler moves such loads behind the branch, a round trip later;
+// as operands of an empty statement between the state's loads and the branch
+// they stay in front of it.
+struct Early {
+    uint32_t count = 0;  // pass 2: length of the list and the thread's first entry
+    uint64_t entry = 0;
+    // a field of each line of the descriptor
+    gptr<const ColorInfo> colors = nullptr;
+    gptr<const uint32_t> key = nullptr;
+    uint32_t mask = 0;
+};
+__device__ __forceinline__ Early early_of(const SysDesc& d, bool key) {
+    Early e;
+    e.colors = d.colors.global();
+    if (key) e.key = d.key.global();
+    e.mask = d.mask[0];
+    return e;
+}
+
 // False when substep t is at or past the stop point.  Else fills `out`; the
 // draw is entry t - drawBase of the explicit table when the state holds one,
 // else the counter draw of (seed, t).
-__device__ __forceinline__ bool begin_substep(const SysDesc& d, uint32_t k, Launch& out) {
-    const cptr<u32x4> w = (cptr<u32x4>)d.state.global();
+__device__ __forceinline__ bool begin_substep(gptr<const DevState> state, uint64_t seed, uint32_t nColors, uint32_t k,
+                                              const Early& early, Launch& out) {
+    const cptr<u32x4> w = (cptr<u32x4>)state;
     const u32x4 w0 = w[0], w1 = w[1], w2 = w[2], w3 = w[3];  // DevState field order
-    const uint64_t t = join64(w0.x, w0.y) + k;
+    uint64_t t = join64(w0.x, w0.y);
+    asm volatile("" : "+s"(t) : "v"(early.count), "v"(early.entry), "s"(early.colors), "s"(early.key), "s"(early.mask),
+                 "s"(seed), "s"(nColors), "s"(k), "s"(w1.x), "s"(w2.x), "s"(w3.x));
+    t += k;
     // A state whose draw table, log or accepted counts are not aligned to
-    // their entries is not served.  Testing them here, with the stop point,
-    // also keeps all four loads ahead of the branch as one batch.
+    // their entries is not served.
     const uint32_t misaligned = ((w1.x | w3.z) & 7u) | (w2.x & 3u);
     if (t >= join64(w0.z, w0.w) || misaligned != 0u) return false;
     out.t = t;
     const uint64_t table = join64(w1.x, w1.y);
     if (table == 0u) {
-        out.draw = substep_draw(d.seed, t, d.nColors);
+        out.draw = substep_draw(seed, t, nColors);
     } else {
         // every lane reads the same entry: keep the draw in scalar registers
         const uint64_t e = global_ptr(reinterpret_cast<const uint64_t*>(uintptr_t(table)))[t - join64(w1.z, w1.w)];
@@ -65,6 +88,10 @@ __device__ __forceinline__ bool begin_substep(const SysDesc& d, uint32_t k, Laun
     out.logCapacity = join64(w3.x, w3.y);
     out.acceptedByBlock = (gptr<uint64_t>)(uintptr_t(join64(w3.z, w3.w)));
     return true;
+}
+
+__device__ __forceinline__ bool begin_substep(const SysDesc& d, uint32_t k, const Early& early, Launch& out) {
+    return begin_substep(d.state.global(), d.seed, d.nColors, k, early, out);
 }
 
 // Species record, read word by word.

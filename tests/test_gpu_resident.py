@@ -165,3 +165,18 @@ def test_batch_with_more_replicas_than_compute_units():
         u.run(9)
         assert np.array_equal(batch.positions(ids[k], s.n), u.getPositions(s.n)), k
         u.cleanup()
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_batch_pass_two_wider_and_narrower_than_its_lists(kind):
+    """Pass-2 workgroups of 64 to 256 threads over lists of 64 and of 512 entries, filled past the first round."""
+    s = ordered_chains((64, 64, 64), 800, 16)
+    u = make_updater(s, 9, kind, block=256, slots=2)
+    u.run(12)
+    for block, slots, perform in ((64, 1, 256), (64, 1, 64), (256, 2, 64), (256, 2, 256)):
+        batch = P.Batch(0, 2, kind, block, slots)
+        rid = batch.add(stage_updater(s, 9, kind))
+        batch.set_perform_block(perform)
+        batch.run(12)
+        assert np.array_equal(batch.positions(rid, s.n), u.getPositions(s.n)), (block, slots, perform)
+    u.cleanup()
