@@ -76,15 +76,27 @@ __device__ __forceinline__ void clear_other_parity(const SysDesc& d, uint64_t t,
 // Pass 1 of substep t for logical workgroup lb of nb of one system.  The
 // survivors go to `list` (capacity SLOTS * blockDim), their number to *count.
 // With `clear` it also zeroes slice lb of nb of the other parity's proposals.
+// What bounds it, 512^3 melt (2 x 4.2 million members): lines that its loads
+// touch, about 230 per 64 members at one a cycle and compute unit, and vector
+// issue behind that.  A quarter fewer vector instructions (move geometry from LDS
+// tables) left 38.1 us per substep at 38.3, and fewer, wider loads were slower
+// because a lane's neighbours then held other members: two consecutive members
+// per lane 41.0, exchanged between half waves 39.7, key and partners side by side
+// in one record 38.5 (dense star network 11.2 against 10.65).
 // KEYED: the system's slots are in spatial order and each slot's draw key is
 // read from its `key` piece; else the key is the hash of the slot index.  A
 // compile-time choice: as a runtime branch between the load and the hash
 // inside the load batch, the compiler's wait for the loaded key also lands on
 // the hashing path, which then waits for every load issued before it.
+struct CheckLds {
+    uint32_t forbidden[16];
+    uint32_t count;
+};
+
 template <int LAT, int SLOTS, int MAXDEG, bool KEYED>
 __device__ __forceinline__ void check_body(const SysDesc& d, uint64_t t, SubstepDraw draw, uint32_t lb, uint32_t nb,
                                            bool clear, gptr<uint64_t> list, gptr<uint32_t> count,
-                                           uint32_t* sForbidden, uint32_t* sCount) {
+                                           CheckLds& lds) {
     if (clear) clear_other_parity(d, t, lb, nb);
     const ColorInfo ci = load_color(d.colors.global(), draw.species);
     const gptr<uint32_t> proposal = d.proposal.global();
@@ -119,21 +131,27 @@ __device__ __forceinline__ void check_body(const SysDesc& d, uint64_t t, Substep
     const gptr<const uint64_t> lattice = (gptr<const uint64_t>)d.lattice.global();
     const AxisMasks masks = axis_masks(d);
 
-    // The load phase is branch-free: lanes without a monomer (or without a
-    // partner in a row) load from an in-bounds stand-in address and discard
-    // the value, so every load of a thread sits in one basic block and all of
-    // them are in flight together.
+    // The load phase is branch-free: lanes without a monomer load the first
+    // one's and discard it, and a monomer with fewer bonds than others tests its
+    // first one again, so every load of a thread sits in one basic block and all
+    // of them are in flight together.  Offsets are 32-bit: a monomer takes eight
+    // of at most 2^32 cells.  (With a "no partner" choice per row and 64-bit indices the 512^3 melt
+    // took 38.6 us per substep against 38.1, the uint8 film 6.28 against 6.21.)
     // First batch of loads: own codes and partner ids.
     uint32_t j[SLOTS], m[SLOTS], hj[SLOTS], partner[SLOTS][MAXDEG];
-    bool live[SLOTS];
+    bool live[SLOTS], free[SLOTS];  // free: no bond to test
+    gptr<const uint32_t> row[MAXDEG];
+#pragma unroll
+    for (int r = 0; r < MAXDEG; ++r)  // past the species' rows: the first one again
+        row[r] = ci.maxDegree == 0u ? pos : nbr + ci.nbrOffset + (uint32_t(r) < ci.maxDegree ? size_t(r) * ci.nbrPitch : 0u);
 #pragma unroll
     for (int s = 0; s < SLOTS; ++s) {
         j[s] = base + uint32_t(s) * B + threadIdx.x;
         live[s] = j[s] < ci.count;
         const uint32_t jj = live[s] ? j[s] : 0u;  // count > 0 for every species
-        m[s] = pos[jj];
+        m[s] = at(pos, 4u * jj);
         if constexpr (KEYED)
-            hj[s] = keys[jj];
+            hj[s] = at(keys, 4u * jj);
         else
             hj[s] = move_hash(jj);
         if constexpr (LAT == kLatticeU8) {
@@ -149,18 +167,19 @@ __device__ __forceinline__ void check_body(const SysDesc& d, uint64_t t, Substep
                     // an escape is read only for a real row of this species, so the index stays in its matrix
                     if (have && v == kIdEscape && uint32_t(r) < ci.maxDegree)
                         id = nbr[ci.nbrOffset + size_t(r) * ci.nbrPitch + jj];
-                    id = min(id, d.nSlots - 1u);  // a valid slot whatever the code
                     const bool has = have && v != kIdNone && uint32_t(r) < ci.maxDegree;
-                    partner[s][r] = (live[s] && has) ? id : kNoNeighbor;
+                    if (r == 0) {
+                        free[s] = !has;
+                        partner[s][r] = id;
+                    } else {
+                        partner[s][r] = has ? id : partner[s][0];
+                    }
                 }
             }
         } else {
 #pragma unroll
-            for (int r = 0; r < MAXDEG; ++r) {
-                const bool row = uint32_t(r) < ci.maxDegree;
-                const uint32_t id = nbr[row ? ci.nbrOffset + size_t(r) * ci.nbrPitch + jj : 0u];
-                partner[s][r] = (live[s] && row) ? id : kNoNeighbor;
-            }
+            for (int r = 0; r < MAXDEG; ++r) partner[s][r] = at(row[r], 4u * jj);
+            free[s] = ci.maxDegree == 0u || partner[s][0] == kNoNeighbor;
         }
     }
     // Second batch: partner codes and the front plane.  CRITICAL.cu:322-323: the
@@ -177,18 +196,18 @@ __device__ __forceinline__ void check_body(const SysDesc& d, uint64_t t, Substep
     uint32_t partnerCode[SLOTS][MAXDEG];
     Dir dir[SLOTS];
     Move mv[SLOTS];
-    bool occ[SLOTS];
+    PlaneWords front[SLOTS];
 #pragma unroll
     for (int s = 0; s < SLOTS; ++s) {
         dir[s] = dir_of_hash(move_hash(hj[s] ^ draw.seed));
-        mv[s] = make_move(m[s], dir[s], masks);
+        mv[s] = make_move<kShift>(m[s], dir[s], masks);
 #pragma unroll
         for (int r = 0; r < MAXDEG; ++r)
-            partnerCode[s][r] = posAll[partner[s][r] != kNoNeighbor ? partner[s][r] : 0u];
-        if constexpr (!kBondsFirst) occ[s] = plane_any<kShift>(lattice, m[s], dir[s], mv[s]);
+            partnerCode[s][r] = at(posAll, 4u * min(partner[s][r], d.nSlots - 1u));  // a valid slot whatever was read
+        if constexpr (!kBondsFirst) front[s] = plane_words(lattice, mv[s]);
     }
-    if (threadIdx.x < 16u) sForbidden[threadIdx.x] = forbidden;
-    if (threadIdx.x == 0) *sCount = 0;
+    if (threadIdx.x < 16u) lds.forbidden[threadIdx.x] = forbidden;
+    if (threadIdx.x == 0) lds.count = 0;
     __syncthreads();
     bool ok[SLOTS];
 #pragma unroll
@@ -197,16 +216,18 @@ __device__ __forceinline__ void check_body(const SysDesc& d, uint64_t t, Substep
 #pragma unroll
         for (int r = 0; r < MAXDEG; ++r) {
             const uint32_t key = bond_key(partnerCode[s][r], mv[s].to);
-            if (partner[s][r] != kNoNeighbor) bad |= sForbidden[key >> 5] >> (key & 31u);
+            // With the plane words still to come, the first bond's test is best left to the
+            // lanes that have one (us per substep, dense star network 10.67 and 10.59).
+            if (!kBondsFirst || r > 0 || !free[s]) bad |= lds.forbidden[key >> 5] >> (key & 31u);
         }
-        ok[s] = live[s] && !(bad & 1u);
+        ok[s] = live[s] && (free[s] || !(bad & 1u));
     }
 #pragma unroll
     for (int s = 0; s < SLOTS; ++s) {
         if constexpr (kBondsFirst) {
             if (ok[s]) ok[s] = !plane_any<kShift>(lattice, m[s], dir[s], mv[s]);
         } else {
-            ok[s] = ok[s] && !occ[s];
+            ok[s] = ok[s] && !plane_any<kShift>(front[s], m[s], dir[s]);
         }
     }
 
@@ -223,7 +244,7 @@ __device__ __forceinline__ void check_body(const SysDesc& d, uint64_t t, Substep
         total += uint32_t(__popcll(mask[s]));
     }
     uint32_t waveBase = 0;
-    if (lane == 0 && total != 0) waveBase = atomicAdd(sCount, total);
+    if (lane == 0 && total != 0) waveBase = atomicAdd(&lds.count, total);
     waveBase = uint32_t(__builtin_amdgcn_readfirstlane(int32_t(waveBase)));
 #pragma unroll
     for (int s = 0; s < SLOTS; ++s) {
@@ -233,7 +254,7 @@ __device__ __forceinline__ void check_body(const SysDesc& d, uint64_t t, Substep
         }
     }
     __syncthreads();
-    if (threadIdx.x == 0) *count = *sCount;
+    if (threadIdx.x == 0) *count = lds.count;
 }
 
 // Sum over the wave of small per-lane counts, bit by bit with ballots and
@@ -360,7 +381,7 @@ __device__ __forceinline__ void perform_body(const SysDesc& d, const Launch& L, 
         const uint32_t jj = uint32_t(entry) & ((1u << kDirShift) - 1u);
         const Dir dir = dir_of_number(uint32_t(entry) >> kDirShift);
         const uint32_t m = uint32_t(entry >> 32);
-        const Move mv = make_move(m, dir, masks);
+        const Move mv = make_move<6>(m, dir, masks);
         if (plane_any<6>(T64, m, dir, mv)) return;
         apply_move<LAT>(d, pos, lat, ci.slotOffset + jj, m, dir, masks, mv);
         ++accepted;
@@ -381,8 +402,7 @@ __device__ __forceinline__ uint32_t list_count(gptr<const uint32_t> count) {
 template <int LAT, int SLOTS, int MAXDEG, bool KEYED>
 __global__ __launch_bounds__(256) void k_check(SysDesc d, uint32_t k, uint32_t clear, uint32_t nb,
                                                                      uint32_t totals) {
-    __shared__ uint32_t sForbidden[16];
-    __shared__ uint32_t sCount;
+    __shared__ CheckLds lds;
     if (blockIdx.x >= nb) {  // the log's own workgroup
         log_before(d.state.global(), k, totals);
         return;
@@ -392,7 +412,7 @@ __global__ __launch_bounds__(256) void k_check(SysDesc d, uint32_t k, uint32_t c
     const uint32_t lb = xcd_block(nb);
     check_body<LAT, SLOTS, MAXDEG, KEYED>(d, L.t, L.draw, lb, nb, clear != 0u,
                                    (gptr<uint64_t>)d.list.global() + size_t(lb) * (SLOTS * blockDim.x),
-                                   d.listCount.global() + lb, sForbidden, &sCount);
+                                   d.listCount.global() + lb, lds);
 }
 
 // After the last substep of a logged run (the state's counter stands past it).
@@ -461,7 +481,7 @@ __global__ __launch_bounds__(256) void k_perform_lists(SysDesc d, uint32_t k, ui
             valid[r] = base + lane + uint32_t(r) * group < count;
             const uint32_t m = valid[r] ? uint32_t(e[r] >> 32) : 0u;
             dir[r] = dir_of_number(valid[r] ? uint32_t(e[r]) >> kDirShift : 0u);
-            mv[r] = make_move(m, dir[r], masks);
+            mv[r] = make_move<6>(m, dir[r], masks);
             hit[r] = plane_any<6>(T64, m, dir[r], mv[r]);
         }
 #pragma unroll
@@ -499,8 +519,7 @@ __device__ __forceinline__ TileRef load_tile(const Tile* tiles, uint32_t w) {
 template <int LAT, int SLOTS, int MAXDEG>
 __global__ __launch_bounds__(256) void k_check_batch(const SysDesc* __restrict__ descs, const Tile* __restrict__ tiles,
                                                      uint2* lists, uint32_t* listCounts, uint32_t k) {
-    __shared__ uint32_t sForbidden[16];
-    __shared__ uint32_t sCount;
+    __shared__ CheckLds lds;
     const TileRef tile = load_tile(tiles, blockIdx.x);
     // never null: named here so that they are loaded with the table's address
     if (tile.replica == kNoReplica || descs == nullptr || lists == nullptr || listCounts == nullptr) return;
@@ -514,10 +533,10 @@ __global__ __launch_bounds__(256) void k_check_batch(const SysDesc* __restrict__
     // branch per workgroup.
     if (d.keyed != 0u)
         check_body<LAT, SLOTS, MAXDEG, true>(d, L.t, L.draw, tile.chunk, tile.chunks, true, list,
-                                             global_ptr(listCounts) + blockIdx.x, sForbidden, &sCount);
+                                             global_ptr(listCounts) + blockIdx.x, lds);
     else
         check_body<LAT, SLOTS, MAXDEG, false>(d, L.t, L.draw, tile.chunk, tile.chunks, true, list,
-                                              global_ptr(listCounts) + blockIdx.x, sForbidden, &sCount);
+                                              global_ptr(listCounts) + blockIdx.x, lds);
 }
 
 template <int LAT>

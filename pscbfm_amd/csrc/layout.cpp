@@ -300,6 +300,9 @@ SystemLayout build_layout(const SystemInput& in, const std::vector<uint8_t>* col
         const uint32_t j = L.slotOf[i] - ci.slotOffset;
         for (uint32_t k = 0; k < in.bonds.degree(i); ++k)
             L.nbr[ci.nbrOffset + k * ci.nbrPitch + j] = L.slotOf[in.bonds.neighbor(i, k)];
+        // further rows repeat the first bond, so that the sweep tests every row alike
+        for (uint32_t k = std::max(in.bonds.degree(i), 1u); k < ci.maxDegree; ++k)
+            L.nbr[ci.nbrOffset + k * ci.nbrPitch + j] = L.nbr[ci.nbrOffset + j];
     }
 
     encode_partner_ids(in, L);

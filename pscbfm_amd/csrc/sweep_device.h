@@ -138,19 +138,24 @@ __device__ __forceinline__ Dir dir_of_number(uint32_t d) { return {d < 2u, d >= 
 // r / 3 of the range plus less than 2^24, for t = 3q + r.  One full-rate 24-bit
 // multiply and two compares, whose results are the axis flags themselves.
 __device__ __forceinline__ Dir dir_of_hash(uint32_t rn) {
-    const uint32_t t = (rn >> 17) + ((rn >> 1) & 0xFFFFu);
-    const uint32_t f = __umul24(t << 7, 0xAAAAABu);
+    uint32_t t = ((rn >> 17) + ((rn >> 1) & 0xFFFFu)) << 7;
+    asm("" : "+v"(t));  // else the shift moves to the constant, which then needs a quarter-rate 32-bit multiply
+    const uint32_t f = __umul24(t, 0xAAAAABu);
     return {f < 0x55555555u, f >= 0xAAAAAAAAu, (rn & 1u) != 0u};
 }
 
 struct Move {
     uint32_t to;                  // code of the new corner
-    uint32_t c00, c02, c20, c22;  // corner cells of the 3x3 plane in front: (u-1, v-1), (u-1, v+1), (u+1, v-1), (u+1, v+1)
+    uint32_t c00, c02, c20, c22;  // bytes to the words with the corner cells of the 3x3 plane in front: (u-1, v-1),
+                                  // (u-1, v+1), (u+1, v-1), (u+1, v+1)
 };
 
 // Front plane: p + 2 e_d + a e_u + b e_v, a,b in {-1,0,1} (CRITICAL.cu:62-176),
 // with (u, v) = (y, z), (x, z), (x, y) for a move along x, y, z.  The lowest
 // code bits of x, y and z are bits 0, 1 and 2, their second bits 3, 4 and 5.
+// The words hold 2^SHIFT cells in eight bytes: a cell's word is its code
+// without the low SHIFT bits, at that code >> (SHIFT - 3) in bytes.
+template <int SHIFT>
 __device__ __forceinline__ Move make_move(uint32_t m, const Dir& d, const AxisMasks& mask) {
     const uint32_t Ma = d.x ? mask.x : (d.z ? mask.z : mask.y);
     const uint32_t Mu = d.x ? mask.y : mask.x;
@@ -162,13 +167,14 @@ __device__ __forceinline__ Move make_move(uint32_t m, const Dir& d, const AxisMa
     Move mv;
     const uint32_t ta = m | ~Ma, tu = m | ~Mu, tv = m | ~Mv;
     mv.to = (m & ~Ma) | ((ta + step1) & Ma);
-    const uint32_t fa = (ta + step2) & Ma;
-    const uint32_t u0 = (tu + Mu) & Mu, u2 = (tu + oneU) & Mu;
-    const uint32_t v0 = (tv + Mv) & Mv, v2 = (tv + oneV) & Mv;
-    mv.c00 = fa | u0 | v0;
-    mv.c02 = fa | u0 | v2;
-    mv.c20 = fa | u2 | v0;
-    mv.c22 = fa | u2 | v2;
+    constexpr uint32_t words = ~((1u << SHIFT) - 1u);
+    const uint32_t fa = (ta + step2) & Ma & words;
+    const uint32_t u0 = (tu + Mu) & Mu & words, u2 = (tu + oneU) & Mu & words;
+    const uint32_t v0 = (tv + Mv) & Mv & words, v2 = (tv + oneV) & Mv & words;
+    mv.c00 = (fa | u0 | v0) >> (SHIFT - 3);
+    mv.c02 = (fa | u0 | v2) >> (SHIFT - 3);
+    mv.c20 = (fa | u2 | v0) >> (SHIFT - 3);
+    mv.c22 = (fa | u2 | v2) >> (SHIFT - 3);
     return mv;
 }
 
@@ -232,18 +238,25 @@ __device__ __forceinline__ bool merged_any(uint64_t w00, uint64_t w02, uint64_t 
                                pick(p.vHigh, uint32_t(w20 >> 32), uint32_t(w22 >> 32)));
     return ((low & p.low) | (high & p.high)) != 0u;
 }
-template <class Words>
-__device__ __forceinline__ bool plane_any(Words words, const PlaneMask& p, const Move& mv) {
-    return merged_any(words[mv.c00 >> 6], words[mv.c02 >> 6], words[mv.c20 >> 6], words[mv.c22 >> 6], p);
+// The element `bytes` behind a base that is the same for every lane, by a 32-bit offset
+// (an index scaled in 64 bits costs three or four instructions more).
+template <class T>
+__device__ __forceinline__ T at(gptr<const T> base, uint32_t bytes) {
+    return *(gptr<const T>)((gptr<const char>)base + bytes);
+}
+struct PlaneWords {
+    uint64_t w00, w02, w20, w22;
+};
+__device__ __forceinline__ PlaneWords plane_words(gptr<const uint64_t> words, const Move& mv) {
+    return {at(words, mv.c00), at(words, mv.c02), at(words, mv.c20), at(words, mv.c22)};
 }
 // Either kind of words.
-template <int SHIFT, class Words>
-__device__ __forceinline__ bool plane_any(Words words, uint32_t m, const Dir& d, const Move& mv) {
+template <int SHIFT>
+__device__ __forceinline__ bool plane_any(const PlaneWords& p, uint32_t m, const Dir& d) {
+    const uint64_t w00 = p.w00, w02 = p.w02, w20 = p.w20, w22 = p.w22;
     if constexpr (SHIFT == 6) {
-        return plane_any(words, plane_mask(m, d), mv);
+        return merged_any(w00, w02, w20, w22, plane_mask(m, d));
     } else {
-        const uint64_t w00 = words[mv.c00 >> SHIFT], w02 = words[mv.c02 >> SHIFT];
-        const uint64_t w20 = words[mv.c20 >> SHIFT], w22 = words[mv.c22 >> SHIFT];
         const uint32_t a0 = uint32_t(w00), a1 = uint32_t(w00 >> 32), b0 = uint32_t(w02), b1 = uint32_t(w02 >> 32);
         const uint32_t c0 = uint32_t(w20), c1 = uint32_t(w20 >> 32), e0 = uint32_t(w22), e1 = uint32_t(w22 >> 32);
         const uint32_t sx = spread_bit(m, 0), sy = spread_bit(m, 1), sz = spread_bit(m, 2);
@@ -258,6 +271,11 @@ __device__ __forceinline__ bool plane_any(Words words, uint32_t m, const Dir& d,
         const uint32_t any1 = (((a1 & vl1) | (b1 & vh1)) & ul) | (((c1 & vl1) | (e1 & vh1)) & uh);
         return ((any0 & plane0) | (any1 & plane1)) != 0u;
     }
+}
+
+template <int SHIFT>
+__device__ __forceinline__ bool plane_any(gptr<const uint64_t> words, uint32_t m, const Dir& d, const Move& mv) {
+    return plane_any<SHIFT>(plane_words(words, mv), m, d);
 }
 
 // Rank of this lane among the lanes of its wave whose bit is set in `mask`.
