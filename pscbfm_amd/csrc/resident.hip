@@ -7,7 +7,9 @@
 // the boundary between the passes is a workgroup barrier and the gathers are
 // LDS reads, so a substep costs what its vector instructions cost on one
 // compute unit: 1.0 us for 192 members of the drawn species (two passes: 5.9),
-// then about 1.05 us per 1000 members (160 instructions per member and wave).
+// 1.45 for 512, 4.75 for 4000, 6.1 for 5000: vector issue on one compute unit (150
+// instructions per 64 members; 7% more cost 1.09 us instead of 1.01 for 192 members,
+// 6.6 instead of 6.1 for 5000).
 //
 // LDS: the occupancy lattice and one proposal lattice (1 bit per cell, Z-curve
 // order, whatever lattice kind the system has in memory), the code of every
@@ -51,8 +53,8 @@ constexpr uint32_t kBond = 0;                  // 512 bytes by bond key
 // form; two steps, one in u, one in v, the cells of the words of u-1.
 constexpr uint32_t kDirs = kBond + 512;
 constexpr uint32_t kPlanes = kDirs + 6 * 32;   // plane cells by axis and low six code bits
-constexpr uint32_t kPos = kPlanes + 192 * 8;   // codes of the slots, then occupancy, then proposals
-static_assert(kPos % 16 == 0, "16-byte LDS accesses");
+constexpr uint32_t kLat = kPlanes + 192 * 8;   // occupancy, then proposals, then codes of the slots
+static_assert(kLat % 16 == 0, "16-byte LDS accesses");
 
 template <class T>
 using lptr = __attribute__((address_space(3))) T*;
@@ -64,15 +66,15 @@ __device__ __forceinline__ lptr<T> lds(uint32_t address) {
 // A move from its draw to its resolution.
 struct Held {
     uint32_t to, record;          // new corner; LDS address of the direction record
-    uint32_t q00, q02, q20, q22;  // 64-cell words of the front plane
+    uint32_t q00, q02, q20, q22;  // bytes to the 64-cell words of the front plane
     uint32_t low, high;           // its cells in a word
 };
 
 // Whether a cell of the plane is set in the lattice at LDS address `words`
 // (plane_any of sweep_device.h).
 __device__ __forceinline__ bool held_any(uint32_t words, const Held& h, uint32_t su, bool z) {
-    const uint64_t w00 = *lds<const uint64_t>(words + (h.q00 << 3)), w02 = *lds<const uint64_t>(words + (h.q02 << 3));
-    const uint64_t w20 = *lds<const uint64_t>(words + (h.q20 << 3)), w22 = *lds<const uint64_t>(words + (h.q22 << 3));
+    const uint64_t w00 = *lds<const uint64_t>(words + h.q00), w02 = *lds<const uint64_t>(words + h.q02);
+    const uint64_t w20 = *lds<const uint64_t>(words + h.q20), w22 = *lds<const uint64_t>(words + h.q22);
     return merged_any(w00, w02, w20, w22, PlaneMask{h.low, h.high, su, z ? 0xFFFF0000u : 0u, z ? 0xFFFF0000u : ~0u});
 }
 
@@ -112,24 +114,27 @@ struct Ahead {
 };
 
 // Draw keys and partner ids of a thread's members.  A lane past the species
-// reads its last member's, a row past the species' degree the codes' own
-// buffer; both are dropped by the user.
+// reads its last member's and drops the move.  A row past the species' degree
+// is its first one again, as the matrix repeats the first bond of a monomer with
+// fewer than others (every monomer of a resident system has one).  Without
+// keys in memory the key is that of the member's index, the same for every
+// substep.
 template <int ROUNDS, int MAXDEG>
 struct Static {
     uint32_t key[ROUNDS], id[ROUNDS][MAXDEG];
     __device__ __forceinline__ void load(const SysDesc& d, const Substep& s) {
-        const gptr<const uint32_t> codes = (gptr<const uint32_t>)d.pos.global() + s.slotOffset;
-        const gptr<const uint32_t> keys = d.keyed != 0u ? (gptr<const uint32_t>)d.key.global() + s.slotOffset : codes;
+        const gptr<const uint32_t> keys = (gptr<const uint32_t>)d.key.global() + s.slotOffset;
+        const bool keyed = d.keyed != 0u;
         gptr<const uint32_t> row[MAXDEG];
 #pragma unroll
         for (uint32_t r = 0; r < uint32_t(MAXDEG); ++r)
-            row[r] = r < s.degree ? (gptr<const uint32_t>)d.nbr.global() + s.nbrOffset + r * s.pitch : codes;
+            row[r] = (gptr<const uint32_t>)d.nbr.global() + s.nbrOffset + (r < s.degree ? r * s.pitch : 0u);
 #pragma unroll
         for (uint32_t k = 0; k < uint32_t(ROUNDS); ++k) {
-            const uint32_t j = min(threadIdx.x + k * blockDim.x, s.count - 1u);
-            key[k] = keys[j];
+            const uint32_t o = 4u * min(threadIdx.x + k * blockDim.x, s.count - 1u);
+            if (keyed) key[k] = at(keys, o);
 #pragma unroll
-            for (int r = 0; r < MAXDEG; ++r) id[k][r] = row[r][j];
+            for (int r = 0; r < MAXDEG; ++r) id[k][r] = at(row[r], o);
         }
     }
 };
@@ -139,7 +144,7 @@ __device__ __forceinline__ void resident_body(const SysDesc& d, uint32_t substep
     const uint32_t B = blockDim.x, tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave64 = uint32_t(__builtin_amdgcn_readfirstlane(int32_t(tid & ~63u)));
     const uint32_t latWords = d.latWords;
-    const uint32_t sLat = kPos + 4u * ((d.nSlots + 3u) & ~3u), sProp = sLat + 4u * latWords;
+    const uint32_t sProp = kLat + 4u * latWords, sPos = sProp + 4u * latWords;
 
     const gptr<const u32x4> w = (gptr<const u32x4>)d.state.global();
     const u32x4 w0 = w[0], w1 = w[1], w2 = w[2], w3 = w[3];  // DevState field order
@@ -164,9 +169,9 @@ __device__ __forceinline__ void resident_body(const SysDesc& d, uint32_t substep
         } else {
             v = ((gptr<const uint32_t>)d.lattice.global())[i];
         }
-        *lds<uint32_t>(sLat + 4u * i) = v;
+        *lds<uint32_t>(kLat + 4u * i) = v;
     }
-    for (uint32_t i = tid; i < d.nSlots; i += B) *lds<uint32_t>(kPos + 4u * i) = posAll[i];
+    for (uint32_t i = tid; i < d.nSlots; i += B) *lds<uint32_t>(sPos + 4u * i) = posAll[i];
     for (uint32_t i = tid; i < 512u; i += B)
         *lds<uint8_t>(kBond + i) = uint8_t((d.bondMask.global()[i >> 5] >> (i & 31u)) & 1u);
     const AxisMasks masks = axis_masks(d);
@@ -191,6 +196,8 @@ __device__ __forceinline__ void resident_body(const SysDesc& d, uint32_t substep
     ahead.fill(d, t0 + min(lane, n - 1u), table, drawBase);
     Substep s = ahead.at(0);
     Static<ROUNDS, MAXDEG> st;
+#pragma unroll
+    for (uint32_t k = 0; k < uint32_t(ROUNDS); ++k) st.key[k] = move_hash(tid + k * B);
     if constexpr (kReadAhead) st.load(d, s);
 
     for (uint32_t step = 0; step < n; ++step) {
@@ -206,18 +213,11 @@ __device__ __forceinline__ void resident_body(const SysDesc& d, uint32_t substep
             if (wave64 + k * B >= s.count) break;  // the same for the whole wave
             const uint32_t j = tid + k * B, jj = min(j, s.count - 1u);
             Held& h = held[k];
-            const uint32_t m = *lds<uint32_t>(kPos + 4u * (s.slotOffset + jj));
+            const uint32_t m = *lds<uint32_t>(sPos + 4u * (s.slotOffset + jj));
             uint32_t code[MAXDEG];
-            // A monomer with fewer bonds tests its first one again (every
-            // monomer of a resident system has one).
 #pragma unroll
-            for (uint32_t r = 0; r < uint32_t(MAXDEG); ++r) {
-                uint32_t id = st.id[k][r];
-                if (r > 0u) id = r < s.degree && id != kNoNeighbor ? id : st.id[k][0];
-                code[r] = *lds<uint32_t>(kPos + 4u * id);
-            }
-            const uint32_t hj = d.keyed != 0u ? st.key[k] : move_hash(jj);
-            const uint32_t rn = move_hash(hj ^ s.seed);
+            for (uint32_t r = 0; r < uint32_t(MAXDEG); ++r) code[r] = *lds<uint32_t>(sPos + 4u * st.id[k][r]);
+            const uint32_t rn = move_hash(st.key[k] ^ s.seed);
             const Dir dir = dir_of_hash(rn);
             const uint32_t axis = dir.x ? 0u : (dir.z ? 128u : 64u);
             h.record = axis | (rn & 1u) << 5;
@@ -230,14 +230,14 @@ __device__ __forceinline__ void resident_body(const SysDesc& d, uint32_t substep
             uint32_t bad = 0;
 #pragma unroll
             for (int r = 0; r < MAXDEG; ++r) bad |= *lds<const uint8_t>(kBond + bond_key(code[r], h.to));
-            const uint32_t fa = (ta + rb.x) & ra.x;
-            const uint32_t u0 = fa | ((tu + ra.y) & ra.y), u2 = fa | ((tu + rb.y) & ra.y);
-            const uint32_t v0 = (tv + ra.z) & ra.z, v2 = (tv + rb.z) & ra.z;
-            h.q00 = __builtin_amdgcn_ubfe(u0 | v0, 6, 26);
-            h.q02 = __builtin_amdgcn_ubfe(u0 | v2, 6, 26);
-            h.q20 = __builtin_amdgcn_ubfe(u2 | v0, 6, 26);
-            h.q22 = __builtin_amdgcn_ubfe(u2 | v2, 6, 26);
-            const bool blocked = held_any(sLat, h, rb.w, dir.z);
+            const uint32_t fa = (ta + rb.x) & ra.x & ~63u;
+            const uint32_t u0 = fa | ((tu + ra.y) & ra.y & ~63u), u2 = fa | ((tu + rb.y) & ra.y & ~63u);
+            const uint32_t v0 = (tv + ra.z) & ra.z & ~63u, v2 = (tv + rb.z) & ra.z & ~63u;
+            h.q00 = (u0 | v0) >> 3;
+            h.q02 = (u0 | v2) >> 3;
+            h.q20 = (u2 | v0) >> 3;
+            h.q22 = (u2 | v2) >> 3;
+            const bool blocked = held_any(kLat, h, rb.w, dir.z);
             if (j < s.count && bad == 0u && !blocked) {
                 ok |= 1u << k;
                 atomicOr((uint32_t*)lds<uint32_t>(sProp + 4u * (h.to >> 5)), 1u << (h.to & 31u));
@@ -261,12 +261,12 @@ __device__ __forceinline__ void resident_body(const SysDesc& d, uint32_t substep
             if (go) {
                 go = !held_any(sProp, h, h.record < 64u ? 0xFFFF0000u : 0xFF00FF00u, h.record >= 128u);
                 if (go) {
-                    const uint32_t slot = slot0 + k * B, m = *lds<uint32_t>(kPos + 4u * slot);
-                    *lds<uint32_t>(kPos + 4u * slot) = h.to;
+                    const uint32_t slot = slot0 + k * B, m = *lds<uint32_t>(sPos + 4u * slot);
+                    *lds<uint32_t>(sPos + 4u * slot) = h.to;
                     // one writer per byte, as in apply_move (kernels.hip)
                     const uint32_t bFrom = m >> 3, bTo = h.to >> 3;
-                    if (bFrom != bTo) *lds<uint8_t>(sLat + bFrom) = 0;
-                    *lds<uint8_t>(sLat + bTo) = uint8_t(1u << (h.to & 7u));
+                    if (bFrom != bTo) *lds<uint8_t>(kLat + bFrom) = 0;
+                    *lds<uint8_t>(kLat + bTo) = uint8_t(1u << (h.to & 7u));
                     // a step up has the larger code unless it wraps, a step down the smaller
                     const bool plus = (h.record & 32u) != 0u;
                     if ((h.to > m) != plus) {
@@ -291,11 +291,11 @@ __device__ __forceinline__ void resident_body(const SysDesc& d, uint32_t substep
     // Store.
     if (lane == 0u && total != 0u)
         __hip_atomic_fetch_add(&accepted[0], total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    for (uint32_t i = tid; i < d.nSlots; i += B) posAll[i] = *lds<uint32_t>(kPos + 4u * i);
+    for (uint32_t i = tid; i < d.nSlots; i += B) posAll[i] = *lds<uint32_t>(sPos + 4u * i);
     const gptr<uint32_t> marks = d.proposal.global();
     const uint32_t last = uint32_t((t0 + n - 1u) & 1u);
     for (uint32_t i = tid; i < latWords; i += B) {
-        const uint32_t v = *lds<uint32_t>(sLat + 4u * i);
+        const uint32_t v = *lds<uint32_t>(kLat + 4u * i);
         if (d.latticeKind == kLatticeU8) {
             const gptr<uint32_t> cells = (gptr<uint32_t>)d.lattice.global() + 8u * i;
 #pragma unroll
@@ -356,7 +356,7 @@ hipError_t allow_full_lds(const void* kernel) {
 }  // namespace
 
 uint64_t resident_lds_bytes(const SysDesc& d) {
-    return kPos + 4ull * ((uint64_t(d.nSlots) + 3u) & ~3ull) + 8ull * d.latWords;
+    return kLat + 8ull * d.latWords + 4ull * ((uint64_t(d.nSlots) + 3u) & ~3ull);
 }
 
 uint32_t resident_block(const SysDesc& d) {
