@@ -115,8 +115,11 @@ void automatic_shape(const SystemLayout& L, uint32_t latticeKind, uint32_t* bloc
     // Two monomers per thread keep more loads in flight per wave, one gives
     // twice the waves.  Measured, 256 x 2 against the choice, us per substep
     // by members of a species:
-    //   up to 2^15, 128 x 1: 8192 6.7 and 6.0 (uint8 7.5 and 6.3), 32768 6.7
-    //     and 6.1 (7.5 and 6.4); 256 x 1 takes 6.1 and 6.5 at 32768;
+    //   up to 20,000, 64 x 1: 8192 6.7 and 5.6 (uint8 7.5 and 5.8); 128 x 1
+    //     takes 5.7 (6.0), at 11,800 5.84 against 5.80 (6.35 and 6.15), at
+    //     19,700 6.13 against 5.93 (6.53 and 6.32);
+    //   up to 2^15, 128 x 1: 32768 6.7 and 5.7 (7.5 and 6.0); 64 x 1 takes
+    //     5.8 there, 256 x 1 5.7 and 6.1;
     //   else 256 x 1: 65536 6.8 and 6.3, 2^18 8.3 and 8.2, uint8 2^19 12.8 and
     //     12.3, dense network of 374,400 11.2 and 10.9, at occupied fraction
     //     0.2 839,000 19.6 and 18.3, 1.7 million 30.1 and 28.6, uint8 2^22 55.9
@@ -125,7 +128,7 @@ void automatic_shape(const SystemLayout& L, uint32_t latticeKind, uint32_t* bloc
     //     where the waves of 256 x 1 share the caches worse: 2^19 10.6 to 11.1
     //     with 256 x 1 and 10.7, 2^20 15.4 and 15.2, 2^21 23.9 and 23.4.
     const bool pairs = latticeKind == kLatticeBit && L.maxColorCount > 400000u && occupied_fraction(L) >= 0.4;
-    *block = L.maxColorCount <= (1u << 15) ? 128u : 256u;
+    *block = L.maxColorCount <= 20000u ? 64u : (L.maxColorCount <= (1u << 15) ? 128u : 256u);
     *slots = pairs ? 2u : 1u;
 }
 
