@@ -21,6 +21,7 @@
 namespace pscbfm {
 
 namespace {
+constexpr uint32_t kMaxSplit = 2;  // workgroups per tile
 constexpr uint32_t kMaxWaves = 4;  // of a pass-2 workgroup: each keeps a total of accepted moves
 constexpr size_t kComputeUnits = 256;
 constexpr uint32_t kSpreadTiles = 64;  // replicas with at least this many workgroups use every XCD
@@ -77,9 +78,9 @@ void Batch::growTiles(uint32_t needed) {
     Tile* tiles = nullptr;
     uint2* lists = nullptr;
     uint32_t* counts = nullptr;
-    hip_check(hipMalloc(&tiles, sizeof(Tile) * needed), "hipMalloc tiles");
+    hip_check(hipMalloc(&tiles, sizeof(Tile) * needed * kMaxSplit), "hipMalloc tiles");
     hip_check(hipMalloc(&lists, sizeof(uint2) * uint64_t(needed) * shape_.block * shape_.slots), "hipMalloc lists");
-    hip_check(hipMalloc(&counts, sizeof(uint32_t) * needed), "hipMalloc list counts");
+    hip_check(hipMalloc(&counts, sizeof(uint32_t) * needed * kMaxSplit), "hipMalloc list counts");
     if (dTiles_) (void)hipFree(dTiles_);
     if (dLists_) (void)hipFree(dLists_);
     if (dListCounts_) (void)hipFree(dListCounts_);
@@ -202,6 +203,16 @@ void Batch::assignPaths() {
             ++twoPassUsed_;
         }
     }
+    // Few members leave two per thread short of waves.  Two members per thread
+    // and one, us per substep by members of the two-pass replicas' species: bit
+    // lattice 25,000 6.8 and 6.3, 158,000 8.6 and 8.3, 215,000 8.9 and 8.7, 333,000
+    // 10.2 and 10.4, 1.6 million 25.8 and 28.8; uint8 25,000 7.4 and 6.6, 215,000
+    // 9.9 and 9.8, 521,000 15.5 and 14.6, 1.6 million 32.5 and 35.0.
+    const uint64_t splitMembers = latticeKind_ == kLatticeBit ? 250000u : 600000u;
+    uint64_t members = 0;
+    for (uint32_t i = 0; i < replicaCap_; ++i)
+        if (replicas_[i].live && descs_[i].resident == 0u) members += descs_[i].maxColorCount;
+    split_ = shape_.slots == 2u && !pinned_ && members <= splitMembers ? 2u : 1u;
     // At most two launches, since launches of one stream wait for each other.
     // Up to one replica per compute unit, each gets a full
     // workgroup; beyond that small ones take small workgroups, several to a
@@ -349,15 +360,6 @@ void Batch::uploadTables() {
         assignPaths();
         hip_check(hipMemcpyAsync(dDescs_, descs_.data(), sizeof(SysDesc) * replicaCap_, hipMemcpyHostToDevice, stream_),
                   "descs H2D");
-        hip_check(hipMemcpyAsync(dTiles_, tiles_.data(), sizeof(Tile) * tileCap_, hipMemcpyHostToDevice, stream_),
-                  "tiles H2D");
-        if (!residentIds_.empty())
-            hip_check(hipMemcpyAsync(dResident_, residentIds_.data(), sizeof(uint32_t) * residentIds_.size(),
-                                     hipMemcpyHostToDevice, stream_),
-                      "resident ids H2D");
-        // the host tables may change as soon as this returns
-        hip_check(hipStreamSynchronize(stream_), "sync tables");
-        tablesDirty_ = false;
         uint32_t high = 0;
         for (uint32_t w = tileCap_; w-- > 0;)
             if (tiles_[w].replica != kNoReplica) {
@@ -367,6 +369,22 @@ void Batch::uploadTables() {
         uint32_t grid = 8;
         while (grid < high) grid *= 2;
         activeGrid_ = std::min(grid, tileCap_);
+        std::vector<Tile> table(size_t(activeGrid_) * split_);
+        for (uint32_t w = 0; w < activeGrid_; ++w)
+            for (uint32_t h = 0; h < split_; ++h) {
+                Tile& t = table[size_t(h) * activeGrid_ + w] = tiles_[w];
+                t.chunk = t.chunk * split_ + h;
+                t.chunks *= split_;
+            }
+        hip_check(hipMemcpyAsync(dTiles_, table.data(), sizeof(Tile) * table.size(), hipMemcpyHostToDevice, stream_),
+                  "tiles H2D");
+        if (!residentIds_.empty())
+            hip_check(hipMemcpyAsync(dResident_, residentIds_.data(), sizeof(uint32_t) * residentIds_.size(),
+                                     hipMemcpyHostToDevice, stream_),
+                      "resident ids H2D");
+        // the host tables may change as soon as this returns
+        hip_check(hipStreamSynchronize(stream_), "sync tables");
+        tablesDirty_ = false;
     }
     if (stopsDirty_) {
         std::vector<uint64_t> stops(replicaCap_, 0);
@@ -388,17 +406,22 @@ void Batch::dropGraphs() {
     graphs_.clear();
 }
 
-hipGraphExec_t Batch::graphFor(uint32_t grid, uint32_t substeps) {
-    const auto key = std::make_pair(grid, substeps);
+hipGraphExec_t Batch::graphFor(uint32_t substeps) {
+    const auto key = std::make_tuple(activeGrid_, split_, substeps);
     auto it = graphs_.find(key);
     if (it != graphs_.end()) return it->second;
-    BatchLaunch b{dDescs_, dTiles_, dLists_, dListCounts_, grid, graphDegree_, latticeKind_};
+    const BatchLaunch b{dDescs_, dTiles_, dLists_, dListCounts_, activeGrid_ * split_, graphDegree_, latticeKind_};
+    LaunchShape shape = shape_;
+    if (split_ > 1u) {
+        shape.slots /= split_;
+        shape.performBlock = std::min(shape.performBlock, 128u);  // half the entries: two waves' totals a workgroup
+    }
     hipGraph_t g = nullptr;
     hip_check(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
     hipError_t err = hipSuccess;
     for (uint32_t k = 0; k < substeps && err == hipSuccess; ++k) {
-        err = launch_check_batch(b, k, shape_, stream_);
-        if (err == hipSuccess) err = launch_perform_batch(b, k, shape_, stream_);
+        err = launch_check_batch(b, k, shape, stream_);
+        if (err == hipSuccess) err = launch_perform_batch(b, k, shape, stream_);
     }
     if (err == hipSuccess) err = launch_advance_batch(dDescs_, replicaCap_, substeps, stream_);
     const hipError_t endErr = hipStreamEndCapture(stream_, &g);
@@ -417,14 +440,13 @@ hipGraphExec_t Batch::graphFor(uint32_t grid, uint32_t substeps) {
 Batch::GraphPlan Batch::planGraphs(uint64_t substeps) {
     GraphPlan p;
     if (twoPassUsed_ == 0) return p;
-    const uint32_t grid = activeGrid_;
     p.bulkCount = substeps / kGraphSubsteps;
-    if (p.bulkCount) p.bulk = graphFor(grid, kGraphSubsteps);
+    if (p.bulkCount) p.bulk = graphFor(kGraphSubsteps);
     uint64_t left = substeps - p.bulkCount * kGraphSubsteps;
     // the binary digits of the remainder, each below the bulk size
     for (uint32_t g = kGraphSubsteps / 2; g >= 1u && left > 0; g >>= 1)
         if (left >= g) {
-            p.tail.push_back(graphFor(grid, g));
+            p.tail.push_back(graphFor(g));
             left -= g;
         }
     return p;
@@ -578,8 +600,8 @@ uint32_t Batch::liveReplicas() const {
 }
 
 uint64_t Batch::deviceBytes() const {
-    uint64_t b = sizeof(SysDesc) * uint64_t(replicaCap_) + sizeof(Tile) * uint64_t(tileCap_) +
-                 sizeof(uint2) * uint64_t(tileCap_) * shape_.block * shape_.slots + 4ull * tileCap_ +
+    uint64_t b = sizeof(SysDesc) * uint64_t(replicaCap_) + sizeof(Tile) * uint64_t(tileCap_) * kMaxSplit +
+                 sizeof(uint2) * uint64_t(tileCap_) * shape_.block * shape_.slots + 4ull * tileCap_ * kMaxSplit +
                  36ull * replicaCap_ + sizeof(UnfoldJob) * uint64_t(jobsCap_) + 12 * xyzCap_;
     for (const auto& r : replicas_)
         if (r.live) b += r.dev->bytes;

@@ -8,6 +8,7 @@
 
 #include <cstdint>
 #include <map>
+#include <tuple>
 #include <memory>
 #include <utility>
 #include <vector>
@@ -98,7 +99,7 @@ private:
     void joinResident();
     // Captured graph of `substeps` substeps over workgroups [0, grid) plus
     // their counter advance, instantiated and uploaded on first use.
-    hipGraphExec_t graphFor(uint32_t grid, uint32_t substeps);
+    hipGraphExec_t graphFor(uint32_t substeps);
     // The replays that cover `substeps` substeps at the current grid:
     // `bulkCount` times the bulk graph, then each graph of `tail` once.  Every
     // graph is built here, before anything of the launch is enqueued.
@@ -151,7 +152,11 @@ private:
     // rounded up to a power of two, so a sparsely filled table does not pay
     // for its idle workgroups.  One captured graph per grid size in use.
     uint32_t activeGrid_ = 8;
-    std::map<std::pair<uint32_t, uint32_t>, hipGraphExec_t> graphs_;  // by (grid, substeps)
+    // Workgroups per tile.  With 2 (two members per thread in the launch shape)
+    // each takes half a tile with one member per thread: tile w is workgroups w and
+    // activeGrid_ + w, on the same XCD.
+    uint32_t split_ = 1;
+    std::map<std::tuple<uint32_t, uint32_t, uint32_t>, hipGraphExec_t> graphs_;  // by (grid, split, substeps)
     // Substeps of the bulk graph; a launch replays it, then power-of-two
     // graphs cover the remainder.
     static constexpr uint32_t kGraphSubsteps = 64;
