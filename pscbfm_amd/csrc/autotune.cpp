@@ -132,6 +132,14 @@ void automatic_shape(const SystemLayout& L, uint32_t latticeKind, uint32_t* bloc
     *slots = pairs ? 2u : 1u;
 }
 
+namespace {
+uint32_t max_degree(const SystemLayout& L) {
+    uint32_t v = 0;
+    for (const ColorInfo& ci : L.colors) v = std::max(v, ci.maxDegree);
+    return v;
+}
+}  // namespace
+
 uint32_t automatic_perform_block(const SystemLayout& L, uint32_t block, uint32_t slots) {
     // Pass 2 walks one compacted pass-1 list per workgroup.  With one monomer
     // per pass-1 thread, or in a dense system (at least a quarter of the cells
@@ -139,20 +147,26 @@ uint32_t automatic_perform_block(const SystemLayout& L, uint32_t block, uint32_t
     // fewer: 128 threads against 256, us per substep, 18.3 and 18.7 (839,000
     // members, fraction 0.2, 256 x 1), 38.8 and 39.2 (512^3 melt).  Dilute systems
     // with two monomers per thread have fuller lists and keep the pass-1 block.
-    return (slots == 1u || occupied_fraction(L) >= 0.25) && block > 128u ? 128u : 0u;
+    // In a dense network fewer moves still pass the bond test: 64 threads against
+    // 128, fraction 0.7, 10.2 and 10.4 (uint8 11.5 and 11.6); the 256^3 melt, 0.5,
+    // 11.0 and 10.1.
+    if (block <= 128u) return 0u;
+    if (slots == 1u && max_degree(L) > 2u && occupied_fraction(L) >= 0.4) return 64u;
+    return slots == 1u || occupied_fraction(L) >= 0.25 ? 128u : 0u;
 }
 
 uint32_t automatic_clear_pass(const SystemLayout& L, uint32_t latticeKind) {
-    // The clear (16 bytes per thread and step) goes into pass 1 where that
-    // pass has issue slots to spare: the bit lattice with at most two bonds
-    // per monomer, whose pass 1 gathers the fewest words.  Measured, pass 1
-    // against pass 2: +1.2% sweeps on the 512^3 melt at 0.5, +1.9% at 0.25,
-    // +0.4% on 256^3; the 4-arm star network loses 2.3-3.4% and the uint8
-    // lattice 0.6-2% (its pass 1 moves eight times the plane bytes), so
-    // those clear in pass 2.
-    uint32_t maxDegree = 0;
-    for (const ColorInfo& ci : L.colors) maxDegree = std::max(maxDegree, ci.maxDegree);
-    return latticeKind == kLatticeBit && maxDegree <= 2u ? 1u : 2u;
+    // The clear (16 bytes per thread and step) goes into pass 1, which has issue
+    // slots to spare, on the bit lattice; the uint8 lattice's pass 1 moves eight
+    // times the plane bytes, so it clears in pass 2.  us per substep, pass 1
+    // against pass 2: 512^3 melt 39.1 and 39.8, 839,000 members at fraction 0.2
+    // 16.5 and 17.4, dense star network 10.4 and 10.6, 128^3 melt 5.9 either way;
+    // uint8, 256^3 melt 12.3 and 11.9.  Dense melts of some hundred thousand
+    // members on the bit lattice are the exception: 104,800 at 0.4 6.9 and 6.6, 2^18
+    // at 0.5 8.4 and 8.1, 2^19 10.2 and 10.1; 2^20 14.6 either way.
+    if (latticeKind != kLatticeBit) return 2u;
+    const bool middle = L.maxColorCount > (1u << 16) && L.maxColorCount <= (1u << 19);
+    return middle && max_degree(L) <= 2u && occupied_fraction(L) >= 0.4 ? 2u : 1u;
 }
 
 const std::vector<LaunchShape>& tune_candidates() {

@@ -184,14 +184,15 @@ __device__ __forceinline__ void check_body(const SysDesc& d, uint64_t t, Substep
     }
     // Second batch: partner codes and the front plane.  CRITICAL.cu:322-323: the
     // draw is keyed by the species-local index in the reference's order.
-    // The plane words of moves that fail the bond test are not needed.  On the
-    // byte lattice (eight times the plane bytes) and with more than two bonds
-    // (more moves fail) it pays to wait for the test and read them for the
-    // others only; with two bonds on the bit lattice the reads go out with the
-    // partners'.  us per substep, together against bonds first: 256^3 melt,
-    // uint8 13.9 against 13.2; dense star network 11.4 against 11.3; 512^3
-    // melt, bit 39.2 against 39.7.
-    constexpr bool kBondsFirst = LAT == kLatticeU8 || MAXDEG > 2;
+    // The plane words of moves that fail the bond test are not needed.  It pays
+    // to wait for the test and read them for the others only on the byte lattice
+    // (eight times the plane bytes), with more than two bonds (more moves fail)
+    // and with several members per thread (large systems); else, a chain of round
+    // trips being all that counts, the reads go out with the partners'.  us per
+    // substep, together against bonds first: 256^3 melt, uint8 13.9 against 13.2;
+    // dense star network 10.9 against 10.6; 512^3 melt, bit 38.3 against 38.0; 128^3
+    // melt 5.84 against 6.08.
+    constexpr bool kBondsFirst = LAT == kLatticeU8 || MAXDEG > 2 || SLOTS > 1;
     constexpr int kShift = LAT == kLatticeU8 ? 3 : 6;
     uint32_t partnerCode[SLOTS][MAXDEG];
     Dir dir[SLOTS];
