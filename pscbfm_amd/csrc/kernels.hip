@@ -9,11 +9,12 @@
 //    and every neighbouring cell is a masked add on one axis' bits;
 //  * the forbidden-bond table is a 512-bit mask in LDS, indexed by the
 //    Z-order bond key of two codes;
-//  * both passes are bound by the number of gather instructions and memory
-//    latency more than by bandwidth: a pass-1 thread handles SLOTS monomers
-//    and issues all their loads in two batches (own codes, draw keys and
-//    partner ids; then partner codes and the front plane together, from one
-//    basic block); the 3x3 front plane is read as at most four 64-bit words;
+//  * both passes are bound by the lines their gathers touch and, up to some
+//    hundred thousand members, by dependent round trips, more than by bandwidth:
+//    a pass-1 thread handles SLOTS monomers and issues their loads in batches
+//    (own codes, draw keys and partner ids; then partner codes and the front
+//    plane, or the plane after the bond test: kBondsFirst); the 3x3 front plane
+//    is read as at most four 64-bit words;
 //  * a species' slots may be in the Z-curve order of the starting corners,
 //    so that a wave's members and their partners and lattice words lie
 //    close together; each slot's key is the inner move hash of the member's

@@ -198,7 +198,7 @@ __device__ __forceinline__ uint32_t spread_bit(uint32_t m, uint32_t b) {
 //
 // The cells are picked from the words with masks, in 32-bit halves.  (Nine
 // 64-bit shifts, one per cell, took 65 VALU instructions per move; this takes
-// about 35: the 512^3 melt's pass 1 was bound by VALU issue.)
+// about 35.)
 //  * 4x4x4 words: the plane's own coordinate is a +- 2, the same residue
 //    modulo 4 for both signs, and its transverse coordinates are all residues
 //    but that of u + 2 (v + 2).  So with E_k = the cells whose coordinate k
