@@ -360,22 +360,25 @@ void Batch::uploadTables() {
         assignPaths();
         hip_check(hipMemcpyAsync(dDescs_, descs_.data(), sizeof(SysDesc) * replicaCap_, hipMemcpyHostToDevice, stream_),
                   "descs H2D");
+        // The used tiles of each XCD close up: with the gaps that large replicas
+        // leave behind, a stream of 20 jobs a second with one of 8192 tiles among
+        // them took 8.6 to 9.3 us per substep instead of 7.6.
+        std::vector<uint32_t> used[8];
+        for (uint32_t w = 0; w < tileCap_; ++w)
+            if (tiles_[w].replica != kNoReplica) used[w % 8].push_back(w);
         uint32_t high = 0;
-        for (uint32_t w = tileCap_; w-- > 0;)
-            if (tiles_[w].replica != kNoReplica) {
-                high = w + 1;
-                break;
-            }
+        for (const auto& u : used) high = std::max(high, 8u * uint32_t(u.size()));
         uint32_t grid = 8;
         while (grid < high) grid *= 2;
         activeGrid_ = std::min(grid, tileCap_);
         std::vector<Tile> table(size_t(activeGrid_) * split_);
-        for (uint32_t w = 0; w < activeGrid_; ++w)
-            for (uint32_t h = 0; h < split_; ++h) {
-                Tile& t = table[size_t(h) * activeGrid_ + w] = tiles_[w];
-                t.chunk = t.chunk * split_ + h;
-                t.chunks *= split_;
-            }
+        for (uint32_t x = 0; x < 8; ++x)
+            for (uint32_t i = 0; i < used[x].size(); ++i)
+                for (uint32_t h = 0; h < split_; ++h) {
+                    Tile& t = table[size_t(h) * activeGrid_ + 8u * i + x] = tiles_[used[x][i]];
+                    t.chunk = t.chunk * split_ + h;
+                    t.chunks *= split_;
+                }
         hip_check(hipMemcpyAsync(dTiles_, table.data(), sizeof(Tile) * table.size(), hipMemcpyHostToDevice, stream_),
                   "tiles H2D");
         if (!residentIds_.empty())

@@ -148,13 +148,13 @@ private:
     bool tablesDirty_ = true;
     bool stopsDirty_ = false;
     uint32_t graphDegree_ = 0;
-    // Launches cover workgroups [0, activeGrid_): the highest occupied slot
-    // rounded up to a power of two, so a sparsely filled table does not pay
+    // Launches cover workgroups [0, activeGrid_): the occupied slots, closed up
+    // and rounded up to a power of two, so a sparsely filled table does not pay
     // for its idle workgroups.  One captured graph per grid size in use.
     uint32_t activeGrid_ = 8;
     // Workgroups per tile.  With 2 (two members per thread in the launch shape)
-    // each takes half a tile with one member per thread: tile w is workgroups w and
-    // activeGrid_ + w, on the same XCD.
+    // each takes half a tile with one member per thread: workgroups w and activeGrid_ + w,
+    // on the same XCD, share a tile.
     uint32_t split_ = 1;
     std::map<std::tuple<uint32_t, uint32_t, uint32_t>, hipGraphExec_t> graphs_;  // by (grid, split, substeps)
     // Substeps of the bulk graph; a launch replays it, then power-of-two

@@ -180,3 +180,19 @@ def test_batch_pass_two_wider_and_narrower_than_its_lists(kind):
         batch.run(12)
         assert np.array_equal(batch.positions(rid, s.n), u.getPositions(s.n)), (block, slots, perform)
     u.cleanup()
+
+
+def test_batch_after_a_large_replica_leaves():
+    """The tiles that stay close up: results do not depend on where they were."""
+    large, small = ordered_chains((128, 128, 128), 3000, 32), [chains((128, 64, 128), 100, 50, seed=k) for k in (3, 4)]
+    batch = P.Batch(0, 3)
+    ids = [batch.add(stage_updater(s, 60 + i)) for i, s in enumerate([small[0], large, small[1]])]
+    batch.run(5)
+    batch.remove(ids[1])
+    batch.run(7)
+    for rid, s, seed in ((ids[0], small[0], 60), (ids[2], small[1], 62)):
+        u = make_updater(s, seed)
+        st, _ = u.run(12)
+        assert np.array_equal(batch.positions(rid, s.n), u.getPositions(s.n))
+        assert batch.info(rid).accepted == st.accepted
+        u.cleanup()
