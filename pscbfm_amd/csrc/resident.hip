@@ -7,9 +7,9 @@
 // the boundary between the passes is a workgroup barrier and the gathers are
 // LDS reads, so a substep costs what its vector instructions cost on one
 // compute unit: 1.0 us for 192 members of the drawn species (two passes: 5.9),
-// 1.45 for 512, 4.75 for 4000, 6.1 for 5000: vector issue on one compute unit (150
-// instructions per 64 members; 7% more cost 1.09 us instead of 1.01 for 192 members,
-// 6.6 instead of 6.1 for 5000).
+// 1.45 for 512, 4.75 for 4000, 5.75 for 5000 (6.1 in a batch): vector issue on one
+// compute unit (150 instructions per 64 members; 7% more cost 1.09 us instead of
+// 1.01 for 192 members, in a batch 6.6 instead of 6.1 for 5000).
 //
 // LDS: the occupancy lattice and one proposal lattice (1 bit per cell, Z-curve
 // order, whatever lattice kind the system has in memory), the code of every
@@ -38,11 +38,11 @@ namespace pscbfm {
 namespace {
 
 // Largest species of a system on its own: us per substep, resident against two
-// passes, on 64^3: 4000 members 4.9 and 6.0, 4921 6.2 and 6.0 (byte lattice 6.7
-// and 6.2).  Four and a half rounds of 1024 threads.
-constexpr uint32_t kResidentAlone = 4608;
+// passes, on 64^3: 4088 members 4.8 and 5.7 (byte lattice 4.7 and 6.1), 4800 5.35
+// and 5.8 (5.25 and 6.2), 5000 5.75 and 5.7 (5.65 and 6.1).
+constexpr uint32_t kResidentAlone = 4864;
 // Of a batch replica whatever else the batch holds: a batch of two-pass
-// replicas takes 7 us per substep or more.
+// replicas takes 6.3 us per substep or more.
 constexpr uint32_t kResidentInBatch = 5120;
 
 // LDS addresses.  The kernels have no static LDS, so their dynamic LDS starts

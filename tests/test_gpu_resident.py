@@ -3,7 +3,7 @@ oracle and the two-pass kernels, which setLaunchShape pins.
 
 All results are whole numbers, so every comparison is exact.  Sizes are chosen
 around the workgroup's rounds: a species of 64 and 65 members (one wave and
-two), 1024 and 1025 (one round and two), 4608 and 4609 (the largest that runs
+two), 1024 and 1025 (one round and two), 4864 and 4865 (the largest that runs
 resident alone and the first that does not), and 5120 and 5121 (the same for
 a batch replica)."""
 import numpy as np
@@ -28,8 +28,8 @@ SYSTEMS = {
     "two_waves": lambda: _dimers((32, 32, 32), 65),
     "one_round": lambda: _dimers((64, 32, 32), 1024),
     "two_rounds": lambda: _dimers((64, 32, 32), 1025),
-    "five_rounds": lambda: _dimers((64, 64, 64), 4608),
-    "too_large": lambda: _dimers((64, 64, 64), 4609),
+    "five_rounds": lambda: _dimers((64, 64, 64), 4864),
+    "too_large": lambda: _dimers((64, 64, 64), 4865),
     "smallest_box": lambda: chains((8, 8, 8), 2, 5, seed=3),
     "flat_box": lambda: chains((64, 16, 8), 9, 21, seed=4),
     "network": lambda: stars((64, 64, 64), 60, 4, 7, seed=5),
