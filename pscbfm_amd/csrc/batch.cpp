@@ -98,6 +98,7 @@ void Batch::growTiles(uint32_t needed) {
 
 Batch::~Batch() {
     if (stream_) (void)hipStreamSynchronize(stream_);
+    if (side_) (void)hipStreamSynchronize(side_);  // joined to stream_, unless a launch failed in between
     dropGraphs();
     if (sideDone_) (void)hipEventDestroy(sideDone_);
     if (fork_) (void)hipEventDestroy(fork_);
