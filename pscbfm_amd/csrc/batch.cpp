@@ -98,7 +98,6 @@ void Batch::growTiles(uint32_t needed) {
 
 Batch::~Batch() {
     if (stream_) (void)hipStreamSynchronize(stream_);
-    if (side_) (void)hipStreamSynchronize(side_);  // joined to stream_, unless a launch failed in between
     dropGraphs();
     if (sideDone_) (void)hipEventDestroy(sideDone_);
     if (fork_) (void)hipEventDestroy(fork_);
@@ -456,11 +455,19 @@ Batch::GraphPlan Batch::planGraphs(uint64_t substeps) {
     return p;
 }
 
+// Every other member waits for stream_ alone before it replaces or frees what
+// kernels read, so work on the side stream never outlives this call unjoined:
+// where a launch or the join fails, the host waits for it here.
 void Batch::enqueue(const GraphPlan& plan, uint64_t substeps) {
-    launchResident(substeps);
-    for (uint64_t r = 0; r < plan.bulkCount; ++r) hip_check(hipGraphLaunch(plan.bulk, stream_), "hipGraphLaunch");
-    for (hipGraphExec_t g : plan.tail) hip_check(hipGraphLaunch(g, stream_), "hipGraphLaunch");
-    joinResident();
+    try {
+        launchResident(substeps);
+        for (uint64_t r = 0; r < plan.bulkCount; ++r) hip_check(hipGraphLaunch(plan.bulk, stream_), "hipGraphLaunch");
+        for (hipGraphExec_t g : plan.tail) hip_check(hipGraphLaunch(g, stream_), "hipGraphLaunch");
+        joinResident();
+    } catch (...) {
+        (void)hipStreamSynchronize(side_);
+        throw;
+    }
     launched_ += substeps;
 }
 

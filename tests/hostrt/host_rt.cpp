@@ -1,0 +1,116 @@
+// Host code of the library on the runtime of fake_hip.h: the order of work
+// and memory on error paths, and what is launched where.  One case per call.
+//
+//   host_rt CASE
+#include <cstdio>
+#include <cstring>
+#include <functional>
+#include <map>
+#include <memory>
+#include <stdexcept>
+#include <string>
+#include <vector>
+
+#include "batch.h"
+#include "fake_hip.h"
+#include "generators.h"
+#include "updater.h"
+
+using namespace pscbfm;
+
+namespace {
+
+int failures = 0;
+
+void expect(bool ok, const std::string& what) {
+    if (!ok) {
+        std::fprintf(stderr, "FAIL: %s\n", what.c_str());
+        ++failures;
+    }
+}
+void expect_clean(const std::string& when) {
+    for (const std::string& v : fake::runtime().violations) expect(false, when + ": " + v);
+    fake::runtime().violations.clear();
+}
+
+// The 108 allowed bond vectors (standard set), indexed as copyBondSet takes them.
+bool allowed(int x, int y, int z) {
+    const int d = x * x + y * y + z * z;
+    return d == 4 || d == 5 || d == 6 || d == 9 || d == 10;
+}
+
+// n ordered dimers: two species of n members.
+void stage_dimers(Updater& u, uint32_t edge, uint32_t n) {
+    uint32_t box[3] = {edge, edge, edge};
+    std::vector<int32_t> xyz;
+    if (!place_linear_chains_ordered(box, n, 2, xyz)) throw std::runtime_error("box too small");
+    u.setGpu(0);
+    u.setNrOfAllMonomers(2 * n);
+    u.setMonomerCoordinatesBulk(xyz.data(), 2 * n);
+    for (uint32_t i = 0; i < 2 * n; i += 2) {
+        u.setConnectivity(i, i + 1);
+        u.setConnectivity(i + 1, i);
+    }
+    u.setLatticeSize(box[0], box[1], box[2]);
+    for (int x = -4; x < 4; ++x)
+        for (int y = -4; y < 4; ++y)
+            for (int z = -4; z < 4; ++z) u.copyBondSet(x, y, z, !allowed(x, y, z));
+    u.setSeed(7);
+}
+
+uint32_t add_dimers(Batch& b, uint32_t edge, uint32_t n) {
+    Updater u;
+    stage_dimers(u, edge, n);
+    const StagedSystem s = u.staged();
+    return b.add(layout_of(s), s.seed, 0);
+}
+
+// A launch that fails behind the resident launches of its batch: what the
+// caller does next must not meet their workgroups still running.
+void failed_launch_joins_the_side_stream() {
+    for (const bool first : {true, false}) {
+        Batch b(0, kLatticeBit, 0, 4, 256, 2);
+        const uint32_t resident = add_dimers(b, 32, 100), large = add_dimers(b, 128, 20000);
+        b.setTarget(resident, 50);
+        b.setTarget(large, 50);
+        b.launch(64);
+        b.synchronize();
+        expect_clean("a launch that succeeds");
+        if (first)
+            fake::runtime().failGraphLaunch = 1;
+        else
+            fake::runtime().failGraphLaunch = 2;  // 100 = a bulk graph and others
+        bool threw = false;
+        try {
+            b.launch(100);
+        } catch (const std::runtime_error&) {
+            threw = true;
+        }
+        expect(threw, "the failed graph launch is reported");
+        b.remove(resident);
+        expect_clean("a replica removed after the failed launch");
+        add_dimers(b, 64, 4000);
+        b.synchronize();
+        expect_clean("a replica added after the failed launch");
+    }
+    expect_clean("batches ended");
+}
+
+const std::map<std::string, std::function<void()>> cases = {
+    {"failed_launch_joins_the_side_stream", failed_launch_joins_the_side_stream},
+};
+
+}  // namespace
+
+int main(int argc, char** argv) {
+    if (argc != 2 || !cases.count(argv[1])) return 2;
+    try {
+        cases.at(argv[1])();
+    } catch (const std::exception& e) {
+        std::fprintf(stderr, "FAIL: exception: %s\n", e.what());
+        return 1;
+    }
+    if (failures) return 1;
+    std::printf("%s: passed\n", argv[1]);
+    return 0;
+}
