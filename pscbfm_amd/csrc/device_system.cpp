@@ -278,6 +278,9 @@ DevState DeviceSystem::readState(hipStream_t stream) const {
 }
 
 void DeviceSystem::writeState(const DevState& s, hipStream_t stream) {
+    auto aligned = [](const void* p, uintptr_t to) { return (reinterpret_cast<uintptr_t>(p) & (to - 1u)) == 0u; };
+    if (!aligned(s.drawTable, 8) || !aligned(s.log, 4) || !aligned(s.acceptedByBlock, 8))
+        throw std::invalid_argument("device state: draw table, log or accepted totals not aligned to their entries");
     hip_check(hipMemcpyAsync(desc.state, &s, sizeof s, hipMemcpyHostToDevice, stream), "state H2D");
     hip_check(hipStreamSynchronize(stream), "sync");
 }

@@ -54,6 +54,7 @@ struct DeviceSystem {
     ~DeviceSystem() { release(); }
 
     DevState readState(hipStream_t stream) const;
+    // Refuses (invalid_argument) buffers that are not aligned to their entries.
     void writeState(const DevState& s, hipStream_t stream);
     uint64_t acceptedTotal(uint32_t entries, hipStream_t stream) const;
     // The job that decodes monomers [first, first + count) into records

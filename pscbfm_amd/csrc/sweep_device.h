@@ -58,7 +58,8 @@ __device__ __forceinline__ Early early_of(const SysDesc& d, bool key) {
     return e;
 }
 
-// False when substep t is at or past the stop point.  Else fills `out`; the
+// False when substep t is at or past the stop point.  Else fills `out`, whose
+// pointers the host checked (DeviceSystem::writeState); the
 // draw is entry t - drawBase of the explicit table when the state holds one,
 // else the counter draw of (seed, t).
 __device__ __forceinline__ bool begin_substep(gptr<const DevState> state, uint64_t seed, uint32_t nColors, uint32_t k,
@@ -69,10 +70,7 @@ __device__ __forceinline__ bool begin_substep(gptr<const DevState> state, uint64
     asm volatile("" : "+s"(t) : "v"(early.count), "v"(early.entry), "s"(early.colors), "s"(early.key), "s"(early.mask),
                  "s"(seed), "s"(nColors), "s"(k), "s"(w1.x), "s"(w2.x), "s"(w3.x));
     t += k;
-    // A state whose draw table, log or accepted counts are not aligned to
-    // their entries is not served.
-    const uint32_t misaligned = ((w1.x | w3.z) & 7u) | (w2.x & 3u);
-    if (t >= join64(w0.z, w0.w) || misaligned != 0u) return false;
+    if (t >= join64(w0.z, w0.w)) return false;
     out.t = t;
     const uint64_t table = join64(w1.x, w1.y);
     if (table == 0u) {

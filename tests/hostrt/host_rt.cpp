@@ -96,8 +96,41 @@ void failed_launch_joins_the_side_stream() {
     expect_clean("batches ended");
 }
 
+// Kernels take a state's buffers as they are: what they could not read whole
+// entries from never reaches the device.
+void misaligned_buffers_are_refused() {
+    Updater u;
+    stage_dimers(u, 32, 100);
+    hipStream_t st = nullptr;
+    hip_check(hipStreamCreateWithFlags(&st, hipStreamNonBlocking), "hipStreamCreate");
+    DeviceSystem dev;
+    dev.allocate(layout_of(u.staged()), kLatticeBit, 7, true, 64, st);
+    const DevState good = dev.readState(st);
+    alignas(8) static uint32_t buffer[8];
+    const auto at = [](size_t bytes) { return reinterpret_cast<char*>(buffer) + bytes; };
+    for (int field = 0; field < 3; ++field)
+        for (const size_t bytes : {0, 1, 2, 4, 6}) {
+            DevState s = good;
+            if (field == 0) s.drawTable = reinterpret_cast<uint32_t*>(at(bytes));
+            if (field == 1) s.log = reinterpret_cast<uint32_t*>(at(bytes));
+            if (field == 2) s.acceptedByBlock = reinterpret_cast<uint64_t*>(at(bytes));
+            bool refused = false;
+            try {
+                dev.writeState(s, st);
+            } catch (const std::invalid_argument&) {
+                refused = true;
+            }
+            expect(refused == (bytes % (field == 1 ? 4 : 8) != 0),
+                   "field " + std::to_string(field) + " at " + std::to_string(bytes));
+            dev.writeState(good, st);
+        }
+    dev.release();
+    (void)hipStreamDestroy(st);
+}
+
 const std::map<std::string, std::function<void()>> cases = {
     {"failed_launch_joins_the_side_stream", failed_launch_joins_the_side_stream},
+    {"misaligned_buffers_are_refused", misaligned_buffers_are_refused},
 };
 
 }  // namespace

@@ -9,7 +9,7 @@ import pytest
 
 HOSTRT = Path(__file__).resolve().parent / "hostrt"
 
-CASES = ["failed_launch_joins_the_side_stream"]
+CASES = ["failed_launch_joins_the_side_stream", "misaligned_buffers_are_refused"]
 
 
 @pytest.fixture(scope="module")
