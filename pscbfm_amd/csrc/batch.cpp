@@ -50,7 +50,7 @@ Batch::Batch(int gpu, uint32_t latticeKind, uint32_t tileCapacity, uint32_t repl
     shape_.performBlock = default_perform_block(block);
     shape_.grid = tileCap_;
     hip_check(hipSetDevice(gpu_), "hipSetDevice");
-    streams_ = acquire_streams(2);
+    streams_.acquire(2);
     stream_ = streams_[0];
     side_ = streams_[1];
     hip_check(hipEventCreateWithFlags(&sideDone_, hipEventDisableTiming), "hipEventCreate");
@@ -107,7 +107,7 @@ Batch::~Batch() {
                     static_cast<void*>(dJobs_), static_cast<void*>(dXyz_), static_cast<void*>(dResident_)})
         if (p) (void)hipFree(p);
     if (hXyz_) (void)hipHostFree(hXyz_);
-    release_streams(streams_, gpu_);
+    streams_.release();
 }
 
 void Batch::setPerformBlock(uint32_t block) {

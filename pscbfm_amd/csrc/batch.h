@@ -119,7 +119,7 @@ private:
     uint32_t latticeKind_;
     uint32_t tileCap_, replicaCap_;
     LaunchShape shape_;
-    std::vector<hipStream_t> streams_;
+    StreamSet streams_;
     hipStream_t stream_ = nullptr;  // streams_[0]
     // device tables
     SysDesc* dDescs_ = nullptr;

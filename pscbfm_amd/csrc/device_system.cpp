@@ -43,13 +43,18 @@ namespace {
 
 struct StreamPool {
     std::mutex mu;
-    std::map<std::pair<int, unsigned>, std::vector<std::vector<hipStream_t>>> idle;  // by (device, streams)
+    std::map<std::pair<int, size_t>, std::vector<std::vector<hipStream_t>>> idle;  // by device and streams in a set
 };
 StreamPool& stream_pool() {
     static StreamPool* pool = new StreamPool();  // never destroyed: owners may outlive static objects
     return *pool;
 }
 constexpr size_t kMaxIdleSets = 16;
+
+void destroy_streams(std::vector<hipStream_t>& streams) {
+    for (hipStream_t s : streams) (void)hipStreamDestroy(s);
+    streams.clear();
+}
 
 }  // namespace
 
@@ -72,17 +77,18 @@ bool overlap(hipStream_t a, hipStream_t b) {
 
 }  // namespace
 
-std::vector<hipStream_t> acquire_streams(unsigned n) {
+void StreamSet::acquire(size_t n) {
+    release();
     int device = 0;
     hip_check(hipGetDevice(&device), "hipGetDevice");
     StreamPool& pool = stream_pool();
     std::lock_guard<std::mutex> lock(pool.mu);
     auto& sets = pool.idle[{device, n}];
+    sets.reserve(kMaxIdleSets);
     std::vector<hipStream_t> streams, rejected;
     if (!sets.empty()) {
         streams = std::move(sets.back());
         sets.pop_back();
-        return streams;
     }
     try {
         while (streams.size() < n) {
@@ -97,27 +103,28 @@ std::vector<hipStream_t> acquire_streams(unsigned n) {
             }
         }
     } catch (...) {
-        for (hipStream_t q : streams) (void)hipStreamDestroy(q);
-        for (hipStream_t q : rejected) (void)hipStreamDestroy(q);
+        destroy_streams(streams);
+        destroy_streams(rejected);
         throw;
     }
-    for (hipStream_t q : rejected) (void)hipStreamDestroy(q);
-    return streams;
+    destroy_streams(rejected);
+    streams_ = std::move(streams);
+    device_ = device;
 }
 
-void release_streams(std::vector<hipStream_t>& streams, int device) {
-    if (streams.empty()) return;
+void StreamSet::release() {
+    if (streams_.empty()) return;
     bool good = true;
-    for (hipStream_t s : streams) good = hipStreamSynchronize(s) == hipSuccess && good;
+    for (hipStream_t s : streams_) good = hipStreamSynchronize(s) == hipSuccess && good;
     StreamPool& pool = stream_pool();
     std::lock_guard<std::mutex> lock(pool.mu);
-    auto& sets = pool.idle[{device, unsigned(streams.size())}];
+    auto& sets = pool.idle[{device_, streams_.size()}];
     if (good && sets.size() < kMaxIdleSets) {
-        sets.push_back(std::move(streams));
+        sets.push_back(std::move(streams_));  // within the capacity that acquire() reserved
+        streams_.clear();
     } else {
-        for (hipStream_t s : streams) (void)hipStreamDestroy(s);
+        destroy_streams(streams_);
     }
-    streams.clear();
 }
 
 namespace {

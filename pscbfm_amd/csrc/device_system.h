@@ -19,15 +19,28 @@ inline void hip_check(hipError_t e, const char* what) {
     if (e != hipSuccess) hip_fail(e, what);
 }
 
-// `n` streams of the current device whose kernels run side by side.  The
-// runtime maps streams to four hardware queues in a way it does not tell, and
-// kernels of streams that share a queue wait for each other (the mix of 96
-// small systems: 10.1 instead of 7.7 us per substep), so new streams are tried
-// out, in about a millisecond, and sets are handed on from owner to owner:
-// at most 16 idle ones of a size and device are kept.  Any thread may call.
-std::vector<hipStream_t> acquire_streams(unsigned n);
-// Waits for the streams and takes them back.
-void release_streams(std::vector<hipStream_t>& streams, int device);
+// Streams of one device whose kernels run side by side.  The runtime maps
+// streams to four hardware queues in a way it does not tell, and kernels of
+// streams that share a queue wait for each other (the mix of 96 small systems:
+// 10.1 instead of 7.7 us per substep), so new streams are tried out, in about a
+// millisecond, and sets are handed on from owner to owner: at most 16 idle ones
+// of a size and device are kept.  Sets of any threads.
+class StreamSet {
+public:
+    StreamSet() = default;
+    StreamSet(const StreamSet&) = delete;
+    StreamSet& operator=(const StreamSet&) = delete;
+    ~StreamSet() { release(); }
+    // `n` streams of the current device; a set held before is given back.
+    void acquire(size_t n);
+    // Waits for the streams and gives them back.
+    void release();
+    hipStream_t operator[](size_t i) const { return streams_[i]; }
+
+private:
+    std::vector<hipStream_t> streams_;
+    int device_ = 0;
+};
 
 struct DeviceSystem {
     void* arena = nullptr;

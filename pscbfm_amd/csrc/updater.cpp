@@ -416,7 +416,7 @@ void Updater::freeDevice() {
     if (drawTable_) (void)hipFree(drawTable_);
     drawTable_ = nullptr;
     drawCapacity_ = 0;
-    release_streams(streams_, gpu_);
+    streams_.release();
     stream_ = nullptr;
 }
 
@@ -490,7 +490,7 @@ void Updater::initialize() {
     } else {
         hip_check(hipSetDevice(gpu_), "hipSetDevice");
     }
-    if (streams_.empty()) streams_ = acquire_streams(1);
+    streams_.acquire(1);
     stream_ = streams_[0];
 
     cells_ = uint64_t(box_[0]) * box_[1] * box_[2];

@@ -253,7 +253,7 @@ private:
     // device
     bool initialized_ = false;
     SystemLayout layout_;
-    std::vector<hipStream_t> streams_;
+    StreamSet streams_;
     hipStream_t stream_ = nullptr;  // streams_[0]
     DeviceSystem dev_;
     LaunchShape shape_;

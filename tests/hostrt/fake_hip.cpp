@@ -28,6 +28,7 @@ struct Graph {
 };
 struct Stream {
     Clock clock;
+    int device = 0;
     std::unique_ptr<Graph> capture;
 };
 struct Event {
@@ -41,6 +42,7 @@ struct Global {
     std::set<void*> device, pinned;
     std::map<const void*, std::string> kernels;
     Clock host;
+    int current = 0;
     struct {
         dim3 grid, block;
         size_t lds;
@@ -57,6 +59,12 @@ Stream* find(hipStream_t s, const char* who) {
     if (it != g().streams.end()) return it->second.get();
     g().rt.violations.push_back(std::string(who) + ": no such stream");
     return nullptr;
+}
+// The stream to give work to.
+Stream* target(hipStream_t s, const char* who) {
+    Stream* st = find(s, who);
+    if (st && st->device != g().current) g().rt.violations.push_back(std::string(who) + " on another device's stream");
+    return st;
 }
 // Whether the host has waited for all work of all streams.
 void host_touches(const char* who) {
@@ -114,7 +122,7 @@ hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* lds, hipSt
 }
 
 hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void** args, size_t, hipStream_t s) {
-    Stream* st = find(s, "hipLaunchKernel");
+    Stream* st = target(s, "hipLaunchKernel");
     if (!st) return hipErrorInvalidHandle;
     Work w;
     w.launch.kernel = g().kernels[f];
@@ -140,9 +148,9 @@ hipError_t hipFuncSetAttribute(const void* f, hipFuncAttribute, int) {
     return g().kernels.count(f) ? hipSuccess : hipErrorInvalidDeviceFunction;
 }
 
-hipError_t hipGetDeviceCount(int* n) { return *n = 1, hipSuccess; }
-hipError_t hipGetDevice(int* d) { return *d = 0, hipSuccess; }
-hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipGetDeviceCount(int* n) { return *n = 2, hipSuccess; }
+hipError_t hipGetDevice(int* d) { return *d = g().current, hipSuccess; }
+hipError_t hipSetDevice(int d) { return g().current = d, hipSuccess; }
 hipError_t hipGetLastError(void) { return hipSuccess; }
 const char* hipGetErrorName(hipError_t) { return "hipErrorFake"; }
 const char* hipGetErrorString(hipError_t) { return "made by the test"; }
@@ -190,6 +198,7 @@ hipError_t hipDeviceSynchronize(void) {
 
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
     auto st = std::make_unique<Stream>();
+    st->device = g().current;
     *s = reinterpret_cast<hipStream_t>(std::calloc(1, 1));  // never freed: a handle is not given twice
     g().streams[*s] = std::move(st);
     ++g().rt.streamsCreated;
@@ -254,7 +263,7 @@ hipError_t hipGraphUpload(hipGraphExec_t, hipStream_t) { return hipSuccess; }
 hipError_t hipGraphDestroy(hipGraph_t graph) { return g().graphs.erase(graph) ? hipSuccess : hipErrorInvalidHandle; }
 hipError_t hipGraphExecDestroy(hipGraphExec_t e) { return g().graphs.erase(e) ? hipSuccess : hipErrorInvalidHandle; }
 hipError_t hipGraphLaunch(hipGraphExec_t e, hipStream_t s) {
-    Stream* st = find(s, "hipGraphLaunch");
+    Stream* st = target(s, "hipGraphLaunch");
     if (!st || !g().graphs.count(e)) return hipErrorInvalidHandle;
     if (countdown(g().rt.failGraphLaunch)) return hipErrorLaunchFailure;
     for (const Work& w : g().graphs[e]->work) issue(s, st, w);

@@ -96,6 +96,26 @@ void failed_launch_joins_the_side_stream() {
     expect_clean("batches ended");
 }
 
+// A set of streams belongs to the device it was made on, whatever device its
+// owner is told to use next.
+void streams_stay_with_their_device() {
+    Updater other, u;
+    stage_dimers(other, 32, 100);
+    other.setGpu(1);
+    other.initialize();
+    stage_dimers(u, 32, 100);
+    u.initialize();
+    u.runSimulationOnGPU(3);
+    u.setGpu(1);
+    u.destruct();
+    stage_dimers(u, 64, 4000);
+    u.setGpu(1);
+    u.initialize();
+    u.runSimulationOnGPU(3);
+    u.cleanup();
+    expect_clean("an updater moved to the other device");
+}
+
 // Kernels take a state's buffers as they are: what they could not read whole
 // entries from never reaches the device.
 void misaligned_buffers_are_refused() {
@@ -130,6 +150,7 @@ void misaligned_buffers_are_refused() {
 
 const std::map<std::string, std::function<void()>> cases = {
     {"failed_launch_joins_the_side_stream", failed_launch_joins_the_side_stream},
+    {"streams_stay_with_their_device", streams_stay_with_their_device},
     {"misaligned_buffers_are_refused", misaligned_buffers_are_refused},
 };
 
