@@ -42,8 +42,12 @@ void hip_fail(hipError_t e, const char* what) {
 namespace {
 
 struct StreamPool {
+    struct Device {
+        size_t owners = 0;  // sets handed out
+        std::map<size_t, std::vector<std::vector<hipStream_t>>> idle;  // by streams in a set
+    };
     std::mutex mu;
-    std::map<std::pair<int, size_t>, std::vector<std::vector<hipStream_t>>> idle;  // by device and streams in a set
+    std::map<int, Device> devices;
 };
 StreamPool& stream_pool() {
     static StreamPool* pool = new StreamPool();  // never destroyed: owners may outlive static objects
@@ -83,12 +87,22 @@ void StreamSet::acquire(size_t n) {
     hip_check(hipGetDevice(&device), "hipGetDevice");
     StreamPool& pool = stream_pool();
     std::lock_guard<std::mutex> lock(pool.mu);
-    auto& sets = pool.idle[{device, n}];
+    StreamPool::Device& dev = pool.devices[device];
+    auto& sets = dev.idle[n];
     sets.reserve(kMaxIdleSets);
     std::vector<hipStream_t> streams, rejected;
-    if (!sets.empty()) {
+    while (streams.empty() && !sets.empty()) {
         streams = std::move(sets.back());
         sets.pop_back();
+        // a device reset under a live owner takes the idle sets with it
+        const bool alive = std::all_of(streams.begin(), streams.end(), [](hipStream_t s) {
+            const hipError_t e = hipStreamQuery(s);
+            return e == hipSuccess || e == hipErrorNotReady;
+        });
+        if (!alive) {
+            destroy_streams(streams);
+            (void)hipGetLastError();
+        }
     }
     try {
         while (streams.size() < n) {
@@ -110,6 +124,7 @@ void StreamSet::acquire(size_t n) {
     destroy_streams(rejected);
     streams_ = std::move(streams);
     device_ = device;
+    ++dev.owners;
 }
 
 void StreamSet::release() {
@@ -118,13 +133,19 @@ void StreamSet::release() {
     for (hipStream_t s : streams_) good = hipStreamSynchronize(s) == hipSuccess && good;
     StreamPool& pool = stream_pool();
     std::lock_guard<std::mutex> lock(pool.mu);
-    auto& sets = pool.idle[{device_, streams_.size()}];
+    StreamPool::Device& dev = pool.devices[device_];
+    auto& sets = dev.idle[streams_.size()];
     if (good && sets.size() < kMaxIdleSets) {
         sets.push_back(std::move(streams_));  // within the capacity that acquire() reserved
         streams_.clear();
     } else {
         destroy_streams(streams_);
     }
+    if (--dev.owners == 0)
+        for (auto& [n, idle] : dev.idle) {
+            for (auto& set : idle) destroy_streams(set);
+            idle.clear();
+        }
 }
 
 namespace {

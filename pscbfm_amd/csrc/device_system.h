@@ -24,7 +24,8 @@ inline void hip_check(hipError_t e, const char* what) {
 // streams that share a queue wait for each other (the mix of 96 small systems:
 // 10.1 instead of 7.7 us per substep), so new streams are tried out, in about a
 // millisecond, and sets are handed on from owner to owner: at most 16 idle ones
-// of a size and device are kept.  Sets of any threads.
+// of a size and device are kept, and none after the device's last owner, so
+// that a program may reset the device between its systems.  Sets of any threads.
 class StreamSet {
 public:
     StreamSet() = default;

@@ -27,8 +27,6 @@
 // The system's buffers in memory are as if the two-pass kernels had run: codes,
 // images, lattice, accepted counts, log and both proposal buffers.
 #include <algorithm>
-#include <mutex>
-#include <set>
 
 #include "kernels.h"
 #include "sweep_device.h"
@@ -339,18 +337,11 @@ ResidentBatchKernel resident_batch_by_degree(uint32_t maxDegree) {
                            : (maxDegree <= 4u ? k_resident_batch<ROUNDS, 4> : k_resident_batch<ROUNDS, 8>);
 }
 
-// Dynamic LDS beyond 64 KiB is granted per kernel and device, once.
-hipError_t allow_full_lds(const void* kernel) {
-    static std::mutex mu;
-    static std::set<std::pair<int, const void*>> done;
-    int dev = 0;
-    hipError_t err = hipGetDevice(&dev);
-    if (err != hipSuccess) return err;
-    std::lock_guard<std::mutex> lock(mu);
-    if (done.count({dev, kernel})) return hipSuccess;
-    err = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, int(kResidentLds));
-    if (err == hipSuccess) done.insert({dev, kernel});
-    return err;
+// Dynamic LDS beyond 64 KiB is asked for per kernel and device, ahead of every
+// launch that takes it: a device reset may forget it.
+hipError_t allow_lds(const void* kernel, uint64_t bytes) {
+    if (bytes <= 64u * 1024u) return hipSuccess;
+    return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, int(kResidentLds));
 }
 
 }  // namespace
@@ -367,7 +358,7 @@ uint32_t resident_block(const SysDesc& d) {
 
 hipError_t launch_resident(const SysDesc& d, uint32_t substeps, uint32_t block, hipStream_t st) {
     const ResidentKernel kernel = resident_kernel((d.maxColorCount + block - 1u) / block, d.maxDegree);
-    const hipError_t err = allow_full_lds(reinterpret_cast<const void*>(kernel));
+    const hipError_t err = allow_lds(reinterpret_cast<const void*>(kernel), resident_lds_bytes(d));
     if (err != hipSuccess) return err;
     hipLaunchKernelGGL(kernel, dim3(1), dim3(block), uint32_t(resident_lds_bytes(d)), st, d, substeps);
     return hipGetLastError();
@@ -385,7 +376,7 @@ hipError_t launch_resident_batch(const SysDesc* descs, const uint32_t* ids, cons
     if (c.count == 0u) return hipSuccess;
     const ResidentBatchKernel kernel =
         c.rounds <= 4u ? resident_batch_by_degree<4>(c.maxDegree) : resident_batch_by_degree<8>(c.maxDegree);
-    const hipError_t err = allow_full_lds(reinterpret_cast<const void*>(kernel));
+    const hipError_t err = allow_lds(reinterpret_cast<const void*>(kernel), c.lds);
     if (err != hipSuccess) return err;
     hipLaunchKernelGGL(kernel, dim3(c.count), dim3(c.block), c.lds, st, descs, ids + c.first, substeps);
     return hipGetLastError();

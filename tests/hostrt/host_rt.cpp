@@ -96,6 +96,48 @@ void failed_launch_joins_the_side_stream() {
     expect_clean("batches ended");
 }
 
+// Streams are handed on between owners, but none outlives the device's state:
+// neither past the last owner nor past a reset under a live one.
+void no_stream_outlives_a_device_reset() {
+    auto use_updater = [] {
+        Updater u;
+        stage_dimers(u, 64, 4000);
+        u.initialize();
+        u.runSimulationOnGPU(3);
+    };
+    auto use_batch = [] {
+        Batch b(0, kLatticeBit, 0, 2, 256, 2);
+        b.setTarget(add_dimers(b, 32, 100), 5);
+        b.launch(10);
+        b.synchronize();
+    };
+    use_updater();
+    use_batch();
+    expect(fake::live_streams() == 0, "no owner, no stream");
+    fake::device_reset();
+    use_updater();
+    use_batch();
+    expect_clean("new owners after a reset");
+    {
+        Updater owner;
+        stage_dimers(owner, 32, 100);
+        owner.initialize();
+        use_updater();
+        use_batch();
+        expect(fake::live_streams() == 4, "sets of one and of two wait for their next owner");
+        const uint64_t made = fake::runtime().streamsCreated;
+        use_updater();
+        use_batch();
+        expect(fake::runtime().streamsCreated == made, "and are handed on");
+        fake::device_reset();
+        use_updater();
+        use_batch();
+        expect_clean("new owners after a reset under a live one");
+    }
+    fake::runtime().violations.clear();  // the owner's own stream went with the reset
+    expect(fake::live_streams() == 0, "no owner, no stream");
+}
+
 // A set of streams belongs to the device it was made on, whatever device its
 // owner is told to use next.
 void streams_stay_with_their_device() {
@@ -150,6 +192,7 @@ void misaligned_buffers_are_refused() {
 
 const std::map<std::string, std::function<void()>> cases = {
     {"failed_launch_joins_the_side_stream", failed_launch_joins_the_side_stream},
+    {"no_stream_outlives_a_device_reset", no_stream_outlives_a_device_reset},
     {"streams_stay_with_their_device", streams_stay_with_their_device},
     {"misaligned_buffers_are_refused", misaligned_buffers_are_refused},
 };

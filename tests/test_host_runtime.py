@@ -10,7 +10,7 @@ import pytest
 HOSTRT = Path(__file__).resolve().parent / "hostrt"
 
 CASES = ["failed_launch_joins_the_side_stream", "misaligned_buffers_are_refused",
-         "streams_stay_with_their_device"]
+         "no_stream_outlives_a_device_reset", "streams_stay_with_their_device"]
 
 
 @pytest.fixture(scope="module")
