@@ -24,9 +24,8 @@ struct LaunchShape {
     // The pass (1 or 2) of a single system's substep that zeroes the other
     // parity's proposal buffer.  Batches clear in pass 1.
     uint32_t clearPass = 2;
-    // A run with an accepted log, and the entries of the accepted totals in use
-    // (by any shape so far), which it sums.
-    bool logged = false;
+    // Entries of the accepted totals in use (by any shape so far), which the
+    // accepted log sums.
     uint32_t totals = 0;
     uint32_t passTwoBlock() const { return performBlock ? performBlock : block; }
     uint32_t listStride() const { return slots * block; }  // list entries per workgroup

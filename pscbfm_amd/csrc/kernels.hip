@@ -301,10 +301,13 @@ __device__ __forceinline__ void add_accepted(const AcceptedTotal& a, uint32_t ac
 
 // The accepted log.  A count per wave and substep, added to the substep's
 // entry, had hundreds of atomics on one address end pass 2 (9.5 instead of 6.7
-// us per substep for 32768 members).  Instead pass 1 of a logged run has one
+// us per substep for 32768 members).  Instead pass 1 of a single system has one
 // workgroup more, which sums the waves' running totals and writes the sum,
 // modulo 2^32, as the entry of the substep before; the last substep's is written
-// by k_log_last.  The host takes differences.
+// by k_log_last.  The host takes differences.  Without a log that workgroup
+// ends at once: runs with and without one replay the same graphs, and the
+// launch takes no longer for it (128^3 melt 6.05 and 6.04 us per substep without and
+// with it, chains of 37 on 64^3 5.84 either way).
 __device__ __forceinline__ void log_totals(gptr<const uint64_t> totals, uint32_t n, gptr<uint32_t> log, uint64_t entry,
                                            uint64_t capacity) {
     if (entry >= capacity) return;
@@ -683,10 +686,10 @@ void check_launch(const SysDesc& d, const BatchLaunch* b, uint32_t k, const Laun
         hipLaunchKernelGGL((k_check_batch<LAT, SLOTS, MAXDEG>), dim3(b->tiles), blk, 0, st, b->descs, b->tileTable,
                            b->lists, b->listCounts, k);
     else if (d.keyed != 0u)
-        hipLaunchKernelGGL((k_check<LAT, SLOTS, MAXDEG, true>), dim3(s.grid + (s.logged ? 1u : 0u)), blk, 0, st, d, k,
+        hipLaunchKernelGGL((k_check<LAT, SLOTS, MAXDEG, true>), dim3(s.grid + 1u), blk, 0, st, d, k,
                            uint32_t(s.clearPass == 1u), s.grid, s.totals);
     else
-        hipLaunchKernelGGL((k_check<LAT, SLOTS, MAXDEG, false>), dim3(s.grid + (s.logged ? 1u : 0u)), blk, 0, st, d, k,
+        hipLaunchKernelGGL((k_check<LAT, SLOTS, MAXDEG, false>), dim3(s.grid + 1u), blk, 0, st, d, k,
                            uint32_t(s.clearPass == 1u), s.grid, s.totals);
 }
 

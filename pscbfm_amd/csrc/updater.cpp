@@ -518,18 +518,15 @@ uint32_t Updater::graphChunk() const {
     return nc * std::max<uint32_t>(1u, 256u / nc);
 }
 
-hipGraphExec_t Updater::graphFor(uint32_t g, bool logged) {
-    const auto key = std::make_pair(g, logged);
-    const auto it = graphs_.find(key);
+hipGraphExec_t Updater::graphFor(uint32_t g) {
+    const auto it = graphs_.find(g);
     if (it != graphs_.end()) return it->second;
-    LaunchShape shape = shape_;
-    shape.logged = logged;
     hipGraph_t graph = nullptr;
     hip_check(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
     hipError_t err = hipSuccess;
     for (uint32_t k = 0; k < g && err == hipSuccess; ++k) {
-        err = launch_check(dev_.desc, k, shape, stream_);
-        if (err == hipSuccess) err = launch_perform(dev_.desc, k, shape, stream_);
+        err = launch_check(dev_.desc, k, shape_, stream_);
+        if (err == hipSuccess) err = launch_perform(dev_.desc, k, shape_, stream_);
     }
     if (err == hipSuccess) err = launch_advance(dev_.desc.state, g, stream_);
     const hipError_t endErr = hipStreamEndCapture(stream_, &graph);
@@ -539,7 +536,7 @@ hipGraphExec_t Updater::graphFor(uint32_t g, bool logged) {
     const hipError_t instErr = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
     (void)hipGraphDestroy(graph);
     hip_check(instErr, "hipGraphInstantiate");
-    graphs_[key] = exec;
+    graphs_[g] = exec;
     // the first launch of an exec would otherwise upload it
     hip_check(hipGraphUpload(exec, stream_), "hipGraphUpload");
     return exec;
@@ -555,13 +552,13 @@ void Updater::setGraphChunk(uint32_t substeps) {
 // remaining substeps: every graph launch costs tens of microseconds of device
 // time before its first kernel, so a short run is one launch.  Graphs are
 // cached per size; a caller that repeats one run length builds at most two.
-Updater::GraphPlan Updater::planGraphs(uint64_t S, bool logged) {
+Updater::GraphPlan Updater::planGraphs(uint64_t S) {
     GraphPlan p;
     const uint32_t G = graphChunk();
     p.bulkCount = S / G;
-    if (p.bulkCount) p.bulk = graphFor(G, logged);
+    if (p.bulkCount) p.bulk = graphFor(G);
     const uint64_t left = S - p.bulkCount * G;
-    if (left) p.tail.push_back(graphFor(uint32_t(left), logged));
+    if (left) p.tail.push_back(graphFor(uint32_t(left)));
     return p;
 }
 
@@ -574,8 +571,8 @@ void Updater::prepareGraphs(int32_t nMCS) {
     const uint64_t S = uint64_t(nMCS) * nColors();
     const uint64_t drawCap = drawChunk_ ? std::min(drawChunk_, kMaxDrawSubsteps) : kMaxDrawSubsteps;
     const uint64_t chunk = r250Mode_ ? std::max<uint64_t>(1u, drawCap / nColors()) * nColors() : S;
-    (void)planGraphs(std::min(chunk, S), false);
-    if (S > chunk && S % chunk) (void)planGraphs(S % chunk, false);
+    (void)planGraphs(std::min(chunk, S));
+    if (S > chunk && S % chunk) (void)planGraphs(S % chunk);
     hip_check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
 }
 
@@ -654,7 +651,7 @@ void Updater::runChunk(uint64_t S, uint32_t* log, bool profile, bool useGraph, v
     // work only, and before this run enqueues anything on the stream.
     const bool resident = residentBlock_ != 0 && !profile;
     GraphPlan plan;
-    if (!profile && useGraph && !resident) plan = planGraphs(S, log != nullptr);
+    if (!profile && useGraph && !resident) plan = planGraphs(S);
 
     // Species and kernel seed of every substep, as the kernels will draw them.
     std::vector<uint32_t> species(S);
@@ -718,15 +715,13 @@ void Updater::runChunk(uint64_t S, uint32_t* log, bool profile, bool useGraph, v
         e1 = timing_[1];
         hip_check(hipEventRecord(e0, stream_), "hipEventRecord");
     }
-    LaunchShape shape = shape_;
-    shape.logged = log != nullptr;
     std::vector<hipEvent_t> kev;
     if (profile) {
         kev.resize(3 * S);
         for (auto& e : kev) hip_check(hipEventCreate(&e), "hipEventCreate");
         for (uint64_t k = 0; k < S; ++k) {
             hip_check(hipEventRecord(kev[3 * k], stream_), "hipEventRecord");
-            hip_check(launch_check(dev_.desc, 0, shape, stream_), "launch pass 1");
+            hip_check(launch_check(dev_.desc, 0, shape_, stream_), "launch pass 1");
             hip_check(hipEventRecord(kev[3 * k + 1], stream_), "hipEventRecord");
             hip_check(launch_perform(dev_.desc, 0, shape_, stream_), "launch pass 2");
             hip_check(hipEventRecord(kev[3 * k + 2], stream_), "hipEventRecord");
@@ -751,7 +746,7 @@ void Updater::runChunk(uint64_t S, uint32_t* log, bool profile, bool useGraph, v
         while (left > 0) {
             const uint32_t blk = uint32_t(std::min<uint64_t>(left, 1u << 20));
             for (uint32_t k = 0; k < blk; ++k) {
-                hip_check(launch_check(dev_.desc, k, shape, stream_), "launch pass 1");
+                hip_check(launch_check(dev_.desc, k, shape_, stream_), "launch pass 1");
                 hip_check(launch_perform(dev_.desc, k, shape_, stream_), "launch pass 2");
             }
             hip_check(launch_advance(dev_.desc.state, blk, stream_), "launch advance");

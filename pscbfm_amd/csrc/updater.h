@@ -204,7 +204,7 @@ private:
     void runChunk(uint64_t S, uint32_t* log, bool profile, bool useGraph, void* scratch);
     // Captured graph of `substeps` substeps plus their counter advance,
     // instantiated and uploaded on first use.
-    hipGraphExec_t graphFor(uint32_t substeps, bool logged);
+    hipGraphExec_t graphFor(uint32_t substeps);
     // The replays that cover S substeps: `bulkCount` times the bulk graph,
     // then each graph of `tail` once (the remainder's, if any).
     struct GraphPlan {
@@ -212,7 +212,7 @@ private:
         uint64_t bulkCount = 0;
         std::vector<hipGraphExec_t> tail;
     };
-    GraphPlan planGraphs(uint64_t S, bool logged);
+    GraphPlan planGraphs(uint64_t S);
     void dropGraphs();
     uint32_t graphChunk() const;
     void syncFromDevice();
@@ -259,7 +259,7 @@ private:
     LaunchShape shape_;
     bool shapePinned_ = false;    // setLaunchShape stated a shape
     uint32_t residentBlock_ = 0;  // threads of the resident sweep's workgroup; 0: two-pass kernels
-    std::map<std::pair<uint32_t, bool>, hipGraphExec_t> graphs_;  // by substeps per replay and whether logged
+    std::map<uint32_t, hipGraphExec_t> graphs_;  // by substeps per replay
     uint32_t acceptedMax_ = 0;  // entries of acceptedByBlock that any launch shape so far uses
     uint64_t substep_ = 0;
     uint64_t acceptedTotal_ = 0;

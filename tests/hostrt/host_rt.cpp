@@ -158,6 +158,20 @@ void streams_stay_with_their_device() {
     expect_clean("an updater moved to the other device");
 }
 
+// prepareGraphs builds what a run of that many sweeps replays, logged or not.
+void prepared_graphs_serve_logged_runs() {
+    for (const bool logged : {false, true}) {
+        Updater u;
+        stage_dimers(u, 128, 20000);
+        u.initialize();
+        u.prepareGraphs(150);  // 300 substeps: the bulk graph and the rest's
+        const uint64_t built = fake::runtime().graphsBuilt;
+        std::vector<uint32_t> log(300);
+        u.run(150, logged ? log.data() : nullptr, false, true);
+        expect(fake::runtime().graphsBuilt == built, logged ? "a logged run builds nothing" : "a run builds nothing");
+    }
+}
+
 // Kernels take a state's buffers as they are: what they could not read whole
 // entries from never reaches the device.
 void misaligned_buffers_are_refused() {
@@ -194,6 +208,7 @@ const std::map<std::string, std::function<void()>> cases = {
     {"failed_launch_joins_the_side_stream", failed_launch_joins_the_side_stream},
     {"no_stream_outlives_a_device_reset", no_stream_outlives_a_device_reset},
     {"streams_stay_with_their_device", streams_stay_with_their_device},
+    {"prepared_graphs_serve_logged_runs", prepared_graphs_serve_logged_runs},
     {"misaligned_buffers_are_refused", misaligned_buffers_are_refused},
 };
 

@@ -10,7 +10,8 @@ import pytest
 HOSTRT = Path(__file__).resolve().parent / "hostrt"
 
 CASES = ["failed_launch_joins_the_side_stream", "misaligned_buffers_are_refused",
-         "no_stream_outlives_a_device_reset", "streams_stay_with_their_device"]
+         "no_stream_outlives_a_device_reset", "streams_stay_with_their_device",
+         "prepared_graphs_serve_logged_runs"]
 
 
 @pytest.fixture(scope="module")
