@@ -137,6 +137,40 @@ struct Static {
     }
 };
 
+// Copies items 0..n-1, thread by thread, N loads in flight per thread: one at a
+// time, the copies at a launch's ends were a chain of round trips (a call of one
+// sweep, a chain of 128 in 128 x 64 x 64: 56.6 us, on the byte lattice 94.7; so,
+// and with the threads that resident_block adds, 9.8 and 21.9; two passes 23).
+template <int N, class Load, class Store>
+__device__ __forceinline__ void in_batches(uint32_t n, Load load, Store store) {
+    for (uint32_t first = 0; first < n; first += N * blockDim.x) {
+        decltype(load(0u)) v[N];
+#pragma unroll
+        for (uint32_t q = 0; q < uint32_t(N); ++q)
+            if (first + q * blockDim.x < n) v[q] = load(min(first + q * blockDim.x + threadIdx.x, n - 1u));
+#pragma unroll
+        for (uint32_t q = 0; q < uint32_t(N); ++q) {
+            const uint32_t i = first + q * blockDim.x + threadIdx.x;
+            if (i < n) store(i, v[q]);
+        }
+    }
+}
+
+// 16 cells of the byte lattice and of a bit lattice: four 0/1 bytes times 2^24 +
+// 2^17 + 2^10 + 2^3 have their bits side by side in bits 24..27.
+__device__ __forceinline__ uint32_t pack_cells(u32x4 cells) {
+    uint32_t v = 0;
+#pragma unroll
+    for (uint32_t q = 0; q < 4u; ++q) v |= ((((cells[q] & 0x01010101u) * 0x01020408u) >> 24) & 15u) << (4u * q);
+    return v;
+}
+__device__ __forceinline__ u32x4 unpack_cells(uint32_t v) {
+    u32x4 cells;
+#pragma unroll
+    for (uint32_t q = 0; q < 4u; ++q) cells[q] = (((v >> (4u * q)) & 15u) * 0x00204081u) & 0x01010101u;
+    return cells;
+}
+
 template <int ROUNDS, int MAXDEG>
 __device__ __forceinline__ void resident_body(const SysDesc& d, uint32_t substeps) {
     const uint32_t B = blockDim.x, tid = threadIdx.x, lane = tid & 63u;
@@ -155,21 +189,16 @@ __device__ __forceinline__ void resident_body(const SysDesc& d, uint32_t substep
     const uint64_t logFirst = join64(w2.z, w2.w), logCapacity = join64(w3.x, w3.y);
     const gptr<uint64_t> accepted = (gptr<uint64_t>)(uintptr_t(join64(w3.z, w3.w)));
 
-    // Load.  The byte lattice packs to bits: four 0/1 bytes times
-    // 2^24 + 2^17 + 2^10 + 2^3 have their bits side by side in bits 24..27.
+    // Load.
     const gptr<uint32_t> posAll = d.pos.global();
-    for (uint32_t i = tid; i < latWords; i += B) {
-        uint32_t v = 0;
-        if (d.latticeKind == kLatticeU8) {
-            const gptr<const uint32_t> cells = (gptr<const uint32_t>)d.lattice.global() + 8u * i;
-#pragma unroll
-            for (uint32_t q = 0; q < 8u; ++q) v |= ((((cells[q] & 0x01010101u) * 0x01020408u) >> 24) & 15u) << (4u * q);
-        } else {
-            v = ((gptr<const uint32_t>)d.lattice.global())[i];
-        }
-        *lds<uint32_t>(kLat + 4u * i) = v;
-    }
-    for (uint32_t i = tid; i < d.nSlots; i += B) *lds<uint32_t>(sPos + 4u * i) = posAll[i];
+    if (d.latticeKind == kLatticeU8)
+        in_batches<4>(latWords * 2u, [&](uint32_t i) { return ((gptr<const u32x4>)d.lattice.global())[i]; },
+                      [&](uint32_t i, u32x4 v) { *lds<uint16_t>(kLat + 2u * i) = uint16_t(pack_cells(v)); });
+    else
+        in_batches<4>(latWords / 4u, [&](uint32_t i) { return ((gptr<const u32x4>)d.lattice.global())[i]; },
+                      [&](uint32_t i, u32x4 v) { *lds<u32x4>(kLat + 16u * i) = v; });
+    in_batches<4>(d.nSlots, [&](uint32_t i) { return posAll[i]; },
+                  [&](uint32_t i, uint32_t v) { *lds<uint32_t>(sPos + 4u * i) = v; });
     for (uint32_t i = tid; i < 512u; i += B)
         *lds<uint8_t>(kBond + i) = uint8_t((d.bondMask.global()[i >> 5] >> (i & 31u)) & 1u);
     const AxisMasks masks = axis_masks(d);
@@ -289,21 +318,21 @@ __device__ __forceinline__ void resident_body(const SysDesc& d, uint32_t substep
     // Store.
     if (lane == 0u && total != 0u)
         __hip_atomic_fetch_add(&accepted[0], total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    for (uint32_t i = tid; i < d.nSlots; i += B) posAll[i] = *lds<uint32_t>(sPos + 4u * i);
-    const gptr<uint32_t> marks = d.proposal.global();
-    const uint32_t last = uint32_t((t0 + n - 1u) & 1u);
-    for (uint32_t i = tid; i < latWords; i += B) {
-        const uint32_t v = *lds<uint32_t>(kLat + 4u * i);
-        if (d.latticeKind == kLatticeU8) {
-            const gptr<uint32_t> cells = (gptr<uint32_t>)d.lattice.global() + 8u * i;
-#pragma unroll
-            for (uint32_t q = 0; q < 8u; ++q) cells[q] = (((v >> (4u * q)) & 15u) * 0x00204081u) & 0x01010101u;
-        } else {
-            ((gptr<uint32_t>)d.lattice.global())[i] = v;
-        }
-        marks[last * latWords + i] = *lds<uint32_t>(sProp + 4u * i);
-        marks[(last ^ 1u) * latWords + i] = 0u;
-    }
+    in_batches<2>(d.nSlots, [&](uint32_t i) { return *lds<uint32_t>(sPos + 4u * i); },
+                  [&](uint32_t i, uint32_t v) { posAll[i] = v; });
+    if (d.latticeKind == kLatticeU8)
+        in_batches<2>(latWords * 2u, [&](uint32_t i) { return uint32_t(*lds<uint16_t>(kLat + 2u * i)); },
+                      [&](uint32_t i, uint32_t v) { ((gptr<u32x4>)d.lattice.global())[i] = unpack_cells(v); });
+    else
+        in_batches<2>(latWords / 4u, [&](uint32_t i) { return *lds<u32x4>(kLat + 16u * i); },
+                      [&](uint32_t i, u32x4 v) { ((gptr<u32x4>)d.lattice.global())[i] = v; });
+    const gptr<u32x4> marks = (gptr<u32x4>)d.proposal.global();
+    const uint32_t last = uint32_t((t0 + n - 1u) & 1u), quads = latWords / 4u;
+    in_batches<2>(quads, [&](uint32_t i) { return *lds<u32x4>(sProp + 16u * i); },
+                  [&](uint32_t i, u32x4 v) {
+                      marks[last * quads + i] = v;
+                      marks[(last ^ 1u) * quads + i] = u32x4{0u, 0u, 0u, 0u};
+                  });
     if (tid == 0u) d.state.global()->substep = t0 + n;
 }
 
@@ -352,7 +381,13 @@ uint64_t resident_lds_bytes(const SysDesc& d) {
 
 uint32_t resident_block(const SysDesc& d) {
     if (d.maxColorCount == 0u || d.maxColorCount > kResidentAlone || d.lone != 0u) return 0u;
-    const uint32_t block = std::min((d.maxColorCount + 63u) / 64u * 64u, 1024u);
+    // A thread per member, but no fewer than one per 16 bytes of the lattice, up
+    // to 512: every substep clears the proposals, every launch loads and stores
+    // all.  One chain of 128, us per substep with 64, 256, 512 and 1024 threads:
+    // 32^3 0.81, 0.77, 0.77 and 0.78; 64^3 1.64, 0.96, 0.91 and 0.92; 128 x 64 x 64
+    // 2.60, 1.21, 1.08 and 1.09 (a call of one sweep 21.9, 10.9, 9.5 and 9.5).
+    const uint32_t lanes = std::min(d.latWords / 4u, 512u);
+    const uint32_t block = std::min((std::max(d.maxColorCount, lanes) + 63u) / 64u * 64u, 1024u);
     return resident_lds_bytes(d) <= kResidentLds ? block : 0u;
 }
 
