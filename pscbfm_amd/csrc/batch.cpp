@@ -175,15 +175,16 @@ void Batch::releaseTiles(uint32_t id) {
 }
 
 // Which replicas the resident sweep takes, and their launches.  A replica
-// that fits a workgroup's LDS takes its own compute unit.  A large one then
-// needs longer per substep than the two-pass kernels would alone, so it does
-// so only when the replicas that must use those kernels need longer still:
-// they were measured at about 7 us per substep and 75 members of the drawn
-// species per ns on the replica mix.
+// that fits a workgroup's LDS takes its own compute unit.  A large or branched
+// one then needs longer per substep than the two-pass kernels would alone, so it
+// does so only when those need longer still with all such replicas: they were
+// measured at about 7 us per substep (byte lattice 7.3) and 75 members of the
+// drawn species per ns on the replica mix.  (40 replicas of 4574 members and
+// eight bonds: 8.0 us resident, 9.4 on two passes; four of them: 8.1 and 6.8.)
 void Batch::assignPaths() {
-    double twoPassUs = 7.0;
+    double twoPassUs = latticeKind_ == kLatticeU8 ? 7.3 : 7.0;
     for (uint32_t i = 0; i < replicaCap_; ++i)
-        if (replicas_[i].live && (pinned_ || !resident_fits(descs_[i])))
+        if (replicas_[i].live && (pinned_ || !resident_fits(descs_[i]) || !resident_always(descs_[i])))
             twoPassUs += double(replicas_[i].info.nMonomers) / std::max(1u, replicas_[i].info.nColors) / 75e3;
     std::vector<std::pair<ResidentClass, uint32_t>> chosen;
     twoPassUsed_ = 0;

@@ -39,8 +39,9 @@ namespace {
 // passes, on 64^3: 4088 members 4.8 and 5.7 (byte lattice 4.7 and 6.1), 4800 5.35
 // and 5.8 (5.25 and 6.2), 5000 5.75 and 5.7 (5.65 and 6.1).
 constexpr uint32_t kResidentAlone = 4864;
-// Of a batch replica whatever else the batch holds: a batch of two-pass
-// replicas takes 6.3 us per substep or more.
+// Of a batch replica of up to two bonds whatever else the batch holds: with
+// 5120 members 5.7 us per substep (byte lattice 5.6), where a batch of one to
+// four such two-pass replicas takes 6.0 to 6.2 (6.2 to 6.6).
 constexpr uint32_t kResidentInBatch = 5120;
 
 // LDS addresses.  The kernels have no static LDS, so their dynamic LDS starts
@@ -399,12 +400,32 @@ hipError_t launch_resident(const SysDesc& d, uint32_t substeps, uint32_t block, 
     return hipGetLastError();
 }
 
+// Eight members per thread with more than four bonds do not fit the registers
+// (62 spilled; 13 us per substep for 5000 members).
 bool resident_fits(const SysDesc& d) {
-    return d.maxColorCount != 0u && d.maxColorCount <= 8u * 1024u && d.lone == 0u && resident_lds_bytes(d) <= kResidentLds;
+    return d.maxColorCount != 0u && d.maxColorCount <= (d.maxDegree <= 4u ? 8u : 5u) * 1024u && d.lone == 0u &&
+           resident_lds_bytes(d) <= kResidentLds;
 }
 
-bool resident_always(const SysDesc& d) { return d.maxColorCount <= kResidentInBatch; }
-double resident_substep_us(const SysDesc& d) { return 1.0 + 1.1e-3 * double(d.maxColorCount); }
+// Measured, us per substep by members: up to two bonds 3840 4.3, 5120 5.7, 6400
+// 7.2, 7680 8.3; up to four 4317 5.85, 4934 6.6, 5304 (eight members per thread,
+// 18 registers spilled) 8.0; more 3267 6.3, 4084 7.3, 4574 8.1.
+double resident_substep_us(const SysDesc& d) {
+    double perMember = 1.1e-3;
+    if (d.maxDegree > 4u)
+        perMember = 1.55e-3;
+    else if (d.maxDegree > 2u)
+        perMember = d.maxColorCount <= 5u * 1024u ? 1.25e-3 : 1.35e-3;
+    return 1.0 + perMember * double(d.maxColorCount);
+}
+// More bonds: up to the same time.  Four two-pass replicas take 6.5 us per substep
+// with up to four bonds (byte lattice 6.9), 6.8 (7.4) with more.
+bool resident_always(const SysDesc& d) {
+    SysDesc chain{};
+    chain.maxDegree = 2u;
+    chain.maxColorCount = kResidentInBatch;
+    return resident_substep_us(d) <= resident_substep_us(chain);
+}
 
 hipError_t launch_resident_batch(const SysDesc* descs, const uint32_t* ids, const ResidentClass& c, uint32_t substeps,
                                  hipStream_t st) {

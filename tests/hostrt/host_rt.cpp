@@ -39,23 +39,42 @@ bool allowed(int x, int y, int z) {
     return d == 4 || d == 5 || d == 6 || d == 9 || d == 10;
 }
 
-// n ordered dimers: two species of n members.
-void stage_dimers(Updater& u, uint32_t edge, uint32_t n) {
-    uint32_t box[3] = {edge, edge, edge};
-    std::vector<int32_t> xyz;
-    if (!place_linear_chains_ordered(box, n, 2, xyz)) throw std::runtime_error("box too small");
+// A system in a cubic box; bonds by pairs of monomers.
+void stage(Updater& u, uint32_t edge, const std::vector<int32_t>& xyz, const std::vector<uint32_t>& bonds) {
     u.setGpu(0);
-    u.setNrOfAllMonomers(2 * n);
-    u.setMonomerCoordinatesBulk(xyz.data(), 2 * n);
-    for (uint32_t i = 0; i < 2 * n; i += 2) {
-        u.setConnectivity(i, i + 1);
-        u.setConnectivity(i + 1, i);
+    u.setNrOfAllMonomers(uint32_t(xyz.size() / 3));
+    u.setMonomerCoordinatesBulk(xyz.data(), uint32_t(xyz.size() / 3));
+    for (size_t i = 0; i + 1 < bonds.size(); i += 2) {
+        u.setConnectivity(bonds[i], bonds[i + 1]);
+        u.setConnectivity(bonds[i + 1], bonds[i]);
     }
-    u.setLatticeSize(box[0], box[1], box[2]);
+    u.setLatticeSize(edge, edge, edge);
     for (int x = -4; x < 4; ++x)
         for (int y = -4; y < 4; ++y)
             for (int z = -4; z < 4; ++z) u.copyBondSet(x, y, z, !allowed(x, y, z));
     u.setSeed(7);
+}
+
+// Stars of `arms` arms of 9, ends crosslinked.
+uint32_t add_stars(Batch& b, uint32_t edge, uint32_t stars, uint32_t arms) {
+    const uint32_t box[3] = {edge, edge, edge};
+    std::vector<int32_t> xyz;
+    std::vector<uint32_t> bonds;
+    if (!build_star_network(box, stars, arms, 9, 1, xyz, bonds)) throw std::runtime_error("box too small");
+    Updater u;
+    stage(u, edge, xyz, bonds);
+    const StagedSystem s = u.staged();
+    return b.add(layout_of(s), s.seed, 0);
+}
+
+// n ordered dimers: two species of n members.
+void stage_dimers(Updater& u, uint32_t edge, uint32_t n) {
+    const uint32_t box[3] = {edge, edge, edge};
+    std::vector<int32_t> xyz;
+    if (!place_linear_chains_ordered(box, n, 2, xyz)) throw std::runtime_error("box too small");
+    std::vector<uint32_t> bonds(2 * n);
+    for (uint32_t i = 0; i < 2 * n; ++i) bonds[i] = i;
+    stage(u, edge, xyz, bonds);
 }
 
 uint32_t add_dimers(Batch& b, uint32_t edge, uint32_t n) {
@@ -172,6 +191,42 @@ void prepared_graphs_serve_logged_runs() {
     }
 }
 
+// Launches of a kernel by a batch of the replicas that `add` puts in.
+struct Paths {
+    bool resident = false, twoPass = false;
+};
+Paths paths(const std::function<void(Batch&)>& add) {
+    Batch b(0, kLatticeBit, 0, 64, 256, 2);
+    add(b);
+    for (uint32_t i = 0; i < b.liveReplicas(); ++i) b.setTarget(i, 1);
+    fake::runtime().launches.clear();
+    b.launch(2);
+    b.synchronize();
+    Paths p;
+    for (const fake::Launch& l : fake::runtime().launches) {
+        p.resident = p.resident || l.kernel.find("k_resident") != std::string::npos;
+        p.twoPass = p.twoPass || l.kernel.find("k_check_batch") != std::string::npos;
+    }
+    return p;
+}
+
+// Bonds cost the resident sweep more than the two-pass kernels: 5304 members of
+// up to four bonds take 8.0 us per substep resident, where four such replicas
+// take 6.5 on two passes.
+void branched_replicas_take_the_faster_path() {
+    const Paths few = paths([](Batch& b) { add_stars(b, 64, 430, 4); });
+    expect(!few.resident && few.twoPass, "5304 members of up to four bonds: two passes");
+    const Paths beside = paths([](Batch& b) {
+        add_stars(b, 64, 430, 4);
+        for (int k = 0; k < 4; ++k) add_dimers(b, 128, 40000);
+    });
+    expect(beside.resident && beside.twoPass, "beside longer two-pass work: resident");
+    const Paths chains = paths([](Batch& b) { add_dimers(b, 64, 5120); });
+    expect(chains.resident && !chains.twoPass, "5120 members of chains: resident");
+    const Paths small = paths([](Batch& b) { add_stars(b, 64, 300, 4); });
+    expect(small.resident && !small.twoPass, "3700 members of up to four bonds: resident");
+}
+
 // Kernels take a state's buffers as they are: what they could not read whole
 // entries from never reaches the device.
 void misaligned_buffers_are_refused() {
@@ -209,6 +264,7 @@ const std::map<std::string, std::function<void()>> cases = {
     {"no_stream_outlives_a_device_reset", no_stream_outlives_a_device_reset},
     {"streams_stay_with_their_device", streams_stay_with_their_device},
     {"prepared_graphs_serve_logged_runs", prepared_graphs_serve_logged_runs},
+    {"branched_replicas_take_the_faster_path", branched_replicas_take_the_faster_path},
     {"misaligned_buffers_are_refused", misaligned_buffers_are_refused},
 };
 
