@@ -186,7 +186,7 @@ void Batch::assignPaths() {
     for (uint32_t i = 0; i < replicaCap_; ++i)
         if (replicas_[i].live && (pinned_ || !resident_fits(descs_[i]) || !resident_always(descs_[i])))
             twoPassUs += double(replicas_[i].info.nMonomers) / std::max(1u, replicas_[i].info.nColors) / 75e3;
-    std::vector<std::pair<ResidentClass, uint32_t>> chosen;
+    std::vector<uint32_t> chosen;
     twoPassUsed_ = 0;
     for (uint32_t i = 0; i < replicaCap_; ++i) {
         if (!replicas_[i].live) continue;
@@ -195,10 +195,7 @@ void Batch::assignPaths() {
         d.resident = resident ? 1u : 0u;
         if (resident) {
             releaseTiles(i);
-            ResidentClass c;
-            c.lds = uint32_t(resident_lds_bytes(d));
-            c.maxDegree = d.maxDegree;
-            chosen.emplace_back(c, i);
+            chosen.push_back(i);
         } else {
             if (replicas_[i].tileSlots.empty()) takeTiles(i);
             ++twoPassUsed_;
@@ -219,31 +216,24 @@ void Batch::assignPaths() {
     // workgroup; beyond that small ones take small workgroups, several to a
     // compute unit.  Large replicas first.
     const bool few = chosen.size() <= kComputeUnits;
-    for (auto& [c, id] : chosen) {
-        const uint32_t species = descs_[id].maxColorCount;
-        const bool small = !few && species <= 1024u && c.lds <= kResidentLds / 4u;
-        c.block = small ? 256u : 1024u;
-    }
-    auto key = [&](const ResidentClass& c) { return c.block; };
-    std::sort(chosen.begin(), chosen.end(), [&](const auto& a, const auto& b) {
-        const auto ka = key(a.first), kb = key(b.first);
-        if (ka != kb) return ka > kb;
-        const uint32_t na = descs_[a.second].maxColorCount, nb = descs_[b.second].maxColorCount;
-        return na != nb ? na > nb : a.second < b.second;
+    auto block = [&](uint32_t id) {
+        const SysDesc& d = descs_[id];
+        return !few && d.maxColorCount <= 1024u && resident_lds_bytes(d) <= kResidentLds / 4u ? 256u : 1024u;
+    };
+    std::sort(chosen.begin(), chosen.end(), [&](uint32_t a, uint32_t b) {
+        if (block(a) != block(b)) return block(a) > block(b);
+        const uint32_t na = descs_[a].maxColorCount, nb = descs_[b].maxColorCount;
+        return na != nb ? na > nb : a < b;
     });
     classes_.clear();
     residentIds_.clear();
-    for (const auto& [c, id] : chosen) {
-        if (classes_.empty() || key(classes_.back()) != key(c)) {
-            classes_.push_back(c);
+    for (const uint32_t id : chosen) {
+        if (classes_.empty() || classes_.back().block != block(id)) {
+            classes_.emplace_back();
+            classes_.back().block = block(id);
             classes_.back().first = uint32_t(residentIds_.size());
-            classes_.back().count = 0;
         }
-        ResidentClass& q = classes_.back();
-        q.lds = std::max(q.lds, c.lds);
-        q.maxDegree = std::max(q.maxDegree, c.maxDegree);
-        q.rounds = std::max(q.rounds, (descs_[id].maxColorCount + q.block - 1u) / q.block);
-        ++q.count;
+        add_to_class(classes_.back(), descs_[id]);
         residentIds_.push_back(id);
     }
 }

@@ -66,11 +66,15 @@ hipError_t launch_resident(const SysDesc& d, uint32_t substeps, uint32_t block, 
 // Replicas of a batch that share a launch of the resident sweep, one
 // workgroup each: workgroup w serves descs[ids[first + w]].
 struct ResidentClass {
-    uint32_t block = 0, rounds = 0;  // threads; members of a species per thread (4 or 8)
-    uint32_t lds = 0;                // bytes: the largest of the class
-    uint32_t maxDegree = 0;
-    uint32_t first = 0, count = 0;   // range of `ids`
+    uint32_t block = 0;             // threads
+    uint32_t rounds = 0;            // build: members of a species per thread
+    uint32_t maxDegree = 0;         // build: bonds per member
+    bool mixed = false;             // replicas of several builds
+    uint32_t lds = 0;               // bytes: the largest of the class
+    uint32_t first = 0, count = 0;  // range of `ids`
 };
+// Counts a replica into a class whose block is set.
+void add_to_class(ResidentClass& c, const SysDesc& d);
 // Whether a replica of a batch can run resident.
 bool resident_fits(const SysDesc& d);
 // Whether the replica is worth its own compute unit whatever else the batch

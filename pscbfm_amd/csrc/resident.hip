@@ -81,6 +81,11 @@ __device__ __forceinline__ uint32_t lane_value(uint32_t v, uint32_t lane) {
     return uint32_t(__builtin_amdgcn_readlane(int32_t(v), int32_t(lane)));
 }
 
+// Words that are the same for every lane, in scalar registers (outside a kernel
+// the compiler keeps what it loads from memory that is written in vector ones).
+__device__ __forceinline__ uint32_t uniform(uint32_t v) { return uint32_t(__builtin_amdgcn_readfirstlane(int32_t(v))); }
+__device__ __forceinline__ u32x4 uniform(u32x4 v) { return u32x4{uniform(v.x), uniform(v.y), uniform(v.z), uniform(v.w)}; }
+
 // A substep's draw and its species' record, the same for every lane.
 struct Substep {
     uint32_t seed, slotOffset, count, nbrOffset, pitch, degree;
@@ -180,7 +185,7 @@ __device__ __forceinline__ void resident_body(const SysDesc& d, uint32_t substep
     const uint32_t sProp = kLat + 4u * latWords, sPos = sProp + 4u * latWords;
 
     const gptr<const u32x4> w = (gptr<const u32x4>)d.state.global();
-    const u32x4 w0 = w[0], w1 = w[1], w2 = w[2], w3 = w[3];  // DevState field order
+    const u32x4 w0 = uniform(w[0]), w1 = uniform(w[1]), w2 = uniform(w[2]), w3 = uniform(w[3]);  // DevState field order
     const uint64_t t0 = join64(w0.x, w0.y), stopAt = join64(w0.z, w0.w);
     if (t0 >= stopAt || substeps == 0u) return;
     const uint32_t n = uint32_t(min(uint64_t(substeps), stopAt - t0));
@@ -337,15 +342,57 @@ __device__ __forceinline__ void resident_body(const SysDesc& d, uint32_t substep
     if (tid == 0u) d.state.global()->substep = t0 + n;
 }
 
+// Members per thread of the batch builds.
+__host__ __device__ __forceinline__ uint32_t batch_rounds(uint32_t members, uint32_t block) {
+    return members <= 4u * block ? 4u : (members <= 5u * block ? 5u : 8u);
+}
+
 template <int ROUNDS, int MAXDEG>
 __global__ __launch_bounds__(1024) void k_resident(SysDesc d, uint32_t substeps) {
     resident_body<ROUNDS, MAXDEG>(d, substeps);
 }
 
+// A function of its own per build, so that each has the registers it needs and
+// no others; its arguments, the same for every lane, go back to scalar registers.
+template <int ROUNDS, int MAXDEG>
+__device__ __attribute__((noinline)) void resident_build(const SysDesc* desc, uint32_t substeps) {
+    const uint64_t p = uint64_t(uintptr_t(desc));
+    const uint64_t u = join64(uniform(uint32_t(p)), uniform(uint32_t(p >> 32)));
+    resident_body<ROUNDS, MAXDEG>(*(const SysDesc*)(cptr<SysDesc>)uintptr_t(u), uniform(substeps));
+}
+
+template <int ROUNDS>
+__device__ __forceinline__ void resident_of_degree(const SysDesc* desc, uint32_t substeps) {
+    if (desc->maxDegree <= 2u)
+        resident_build<ROUNDS, 2>(desc, substeps);
+    else if (desc->maxDegree <= 4u)
+        resident_build<ROUNDS, 4>(desc, substeps);
+    else
+        resident_build<ROUNDS, 8>(desc, substeps);
+}
+
+// Replicas of one build.
 template <int ROUNDS, int MAXDEG>
 __global__ __launch_bounds__(1024) void k_resident_batch(const SysDesc* __restrict__ descs,
                                                          const uint32_t* __restrict__ ids, uint32_t substeps) {
     resident_body<ROUNDS, MAXDEG>(descs[ids[blockIdx.x]], substeps);
+}
+
+// Replicas of several builds, each swept by its own.  Eight replicas of 5000
+// members and a small eight-arm star, us per sweep: 26.1 with all of them on the
+// build that holds both, 11.9 so, 11.8 without the star.
+__global__ __launch_bounds__(1024) void k_resident_mix(const SysDesc* __restrict__ descs,
+                                                       const uint32_t* __restrict__ ids, uint32_t substeps) {
+    const SysDesc* desc = descs + ids[blockIdx.x];
+    const uint32_t rounds = batch_rounds(desc->maxColorCount, blockDim.x);
+    if (rounds == 4u)
+        resident_of_degree<4>(desc, substeps);
+    else if (rounds == 5u)
+        resident_of_degree<5>(desc, substeps);
+    else if (desc->maxDegree <= 2u)
+        resident_build<8, 2>(desc, substeps);
+    else
+        resident_build<8, 4>(desc, substeps);
 }
 
 using ResidentKernel = void (*)(SysDesc, uint32_t);
@@ -365,6 +412,12 @@ template <int ROUNDS>
 ResidentBatchKernel resident_batch_by_degree(uint32_t maxDegree) {
     return maxDegree <= 2u ? k_resident_batch<ROUNDS, 2>
                            : (maxDegree <= 4u ? k_resident_batch<ROUNDS, 4> : k_resident_batch<ROUNDS, 8>);
+}
+ResidentBatchKernel resident_batch_kernel(const ResidentClass& c) {
+    if (c.mixed) return k_resident_mix;
+    if (c.rounds == 4u) return resident_batch_by_degree<4>(c.maxDegree);
+    if (c.rounds == 5u) return resident_batch_by_degree<5>(c.maxDegree);
+    return c.maxDegree <= 2u ? k_resident_batch<8, 2> : k_resident_batch<8, 4>;
 }
 
 // Dynamic LDS beyond 64 KiB is asked for per kernel and device, ahead of every
@@ -427,11 +480,19 @@ bool resident_always(const SysDesc& d) {
     return resident_substep_us(d) <= resident_substep_us(chain);
 }
 
+void add_to_class(ResidentClass& c, const SysDesc& d) {
+    const uint32_t rounds = batch_rounds(d.maxColorCount, c.block), degree = d.maxDegree <= 2u ? 2u : (d.maxDegree <= 4u ? 4u : 8u);
+    c.mixed = c.mixed || (c.count != 0u && (rounds != c.rounds || degree != c.maxDegree));
+    c.rounds = rounds;
+    c.maxDegree = degree;
+    c.lds = std::max(c.lds, uint32_t(resident_lds_bytes(d)));
+    ++c.count;
+}
+
 hipError_t launch_resident_batch(const SysDesc* descs, const uint32_t* ids, const ResidentClass& c, uint32_t substeps,
                                  hipStream_t st) {
     if (c.count == 0u) return hipSuccess;
-    const ResidentBatchKernel kernel =
-        c.rounds <= 4u ? resident_batch_by_degree<4>(c.maxDegree) : resident_batch_by_degree<8>(c.maxDegree);
+    const ResidentBatchKernel kernel = resident_batch_kernel(c);
     const hipError_t err = allow_lds(reinterpret_cast<const void*>(kernel), c.lds);
     if (err != hipSuccess) return err;
     hipLaunchKernelGGL(kernel, dim3(c.count), dim3(c.block), c.lds, st, descs, ids + c.first, substeps);

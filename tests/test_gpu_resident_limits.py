@@ -1,10 +1,10 @@
 """The resident sweep at its limits: LDS that is nearly full, lattices much larger
-than their systems, and calls of a few sweeps."""
+than their systems, calls of a few sweeps, and batches of every build."""
 import numpy as np
 import pytest
 
 import pscbfm_amd as P
-from helpers import chains, make_updater, oracle_for, ordered_chains
+from helpers import Sys, chains, make_updater, oracle_for, ordered_chains, stage_updater, stars
 
 pytestmark = pytest.mark.gpu
 
@@ -55,3 +55,63 @@ def test_one_sweep_in_a_large_box_takes_no_longer_than_two_passes(kind):
         u.cleanup()
     print({k: f"{v * 1e3:.1f} us" for k, v in ms.items()}, flush=True)
     assert ms[(0, 0)] < 1.5 * ms[(64, 1)]
+
+
+def _branched(n):
+    """n dimers, closely packed in part of 64^3, with one monomer bonded to its six
+    neighbours in the packing: degrees 1, 2 and 6."""
+    s = ordered_chains((64, 64, 64), 32 * 32 * 21 // 2, 2)
+    s = Sys(s.box, s.xyz[:2 * n], P.chain_bonds(n, 2))
+    at = {tuple(c): i for i, c in enumerate(s.xyz % 64)}
+    bonded = {frozenset(b) for b in s.bonds.tolist()}
+    steps = [(2, 0, 0), (-2, 0, 0), (0, 2, 0), (0, -2, 0), (0, 0, 3), (0, 0, -3)]
+    for i, c in enumerate(s.xyz % 64):
+        near = [at.get(tuple((c + d) % 64)) for d in steps]
+        if None not in near:
+            extra = [(i, j) for j in near if frozenset((i, j)) not in bonded]
+            return Sys(s.box, s.xyz, np.concatenate([s.bonds, np.array(extra, s.bonds.dtype)]))
+    raise AssertionError("no monomer with six neighbours")
+
+
+def _builds():
+    """Replicas of every resident build of a batch (up to 4096, 5120 and 8192
+    members; up to two, four and eight bonds), some only resident beside long
+    two-pass work, and that work; the last stays on two passes beside it."""
+    return [chains((32, 32, 32), 24, 16, seed=1), ordered_chains((64, 64, 64), 4097, 2),
+            ordered_chains((64, 64, 64), 5200, 2), stars((64, 64, 64), 60, 4, 7, seed=5),
+            stars((64, 64, 64), 380, 4, 9, seed=1), stars((64, 64, 64), 430, 4, 9, seed=1),
+            stars((64, 32, 64), 40, 8, 6, seed=6), _branched(4200), _branched(6000),
+            ordered_chains((256, 256, 128), 100000, 2)]
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_batch_of_every_build_equals_runs_alone(kind):
+    systems = _builds()
+    batch = P.Batch(0, len(systems), kind)
+    ids = [batch.add(stage_updater(s, 40 + i, kind)) for i, s in enumerate(systems)]
+    for m in (1, 40):
+        batch.run(m)
+    for i, (rid, s) in enumerate(zip(ids, systems)):
+        u = make_updater(s, 40 + i, kind, block=256, slots=2)
+        st, _ = u.run(41)
+        assert np.array_equal(batch.positions(rid, s.n), u.getPositions(s.n)), i
+        assert batch.info(rid).accepted == st.accepted, i
+        u.cleanup()
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_a_branched_replica_does_not_slow_the_others(kind):
+    """Eight replicas of 5000 members, alone and beside a small star of eight
+    arms.  With one build for all of them the star doubled the time of a sweep;
+    beside it, on a compute unit of its own, it costs nothing, and the bound
+    of 1.3 leaves the measurement's spread to it."""
+    large, star = ordered_chains((64, 64, 64), 5000, 2), stars((32, 32, 32), 5, 8, 7, 1)
+    ms = []
+    for systems in ([large] * 8, [large] * 8 + [star]):
+        batch = P.Batch(0, len(systems), kind)
+        for i, s in enumerate(systems):
+            batch.add(stage_updater(s, 7 + i, kind))
+        batch.run(20)
+        ms.append(min(batch.run(100) for _ in range(8)))
+    print([f"{v * 10:.2f} us per sweep" for v in ms], flush=True)
+    assert ms[1] < 1.3 * ms[0]
