@@ -119,14 +119,7 @@ PSCBFM_HD SubstepDraw substep_draw(uint64_t key, uint64_t t, uint32_t nColors) {
 // x + c for a dilated constant c:  ((m | ~M) + c) & M   (carries ride over
 // the bits of the other axes because they are forced to 1).  Adding the
 // all-ones pattern M is "minus one" modulo the axis length.
-PSCBFM_HD uint32_t dil_add(uint32_t m, uint32_t M, uint32_t c) {
-    return ((m | ~M) + c) & M;
-}
-// (a - b) on one axis, result dilated and wrapped.
-PSCBFM_HD uint32_t dil_sub(uint32_t a, uint32_t b, uint32_t M) {
-    return ((a & M) - (b & M)) & M;
-}
-
+//
 // Low nine bits of a Z-curve code interleave x,y,z three times whenever every
 // box edge is at least 8.  The masked differences of two codes in that window
 // are the bond vector components modulo 8, i.e. exactly the

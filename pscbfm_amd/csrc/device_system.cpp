@@ -313,18 +313,6 @@ void DeviceSystem::writeState(const DevState& s, hipStream_t stream) {
     hip_check(hipStreamSynchronize(stream), "sync");
 }
 
-uint64_t DeviceSystem::acceptedTotal(uint32_t entries, hipStream_t stream) const {
-    const DevState s = readState(stream);
-    std::vector<uint64_t> v(std::min(entries, accEntries));
-    if (!v.empty()) {
-        hip_check(hipMemcpyAsync(v.data(), s.acceptedByBlock, v.size() * 8, hipMemcpyDeviceToHost, stream), "D2H");
-        hip_check(hipStreamSynchronize(stream), "sync");
-    }
-    uint64_t total = 0;
-    for (uint64_t x : v) total += x;
-    return total;
-}
-
 UnfoldJob DeviceSystem::unfoldJob(uint32_t first, uint32_t count, uint64_t out) const {
     UnfoldJob j{};
     j.pos = desc.pos;

@@ -70,7 +70,6 @@ struct DeviceSystem {
     DevState readState(hipStream_t stream) const;
     // Refuses (invalid_argument) buffers that are not aligned to their entries.
     void writeState(const DevState& s, hipStream_t stream);
-    uint64_t acceptedTotal(uint32_t entries, hipStream_t stream) const;
     // The job that decodes monomers [first, first + count) into records
     // out.. of a shared buffer (launch_unfold_jobs; firstBlock left 0).
     UnfoldJob unfoldJob(uint32_t first, uint32_t count, uint64_t out) const;
