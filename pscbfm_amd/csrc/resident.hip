@@ -81,8 +81,9 @@ __device__ __forceinline__ uint32_t lane_value(uint32_t v, uint32_t lane) {
     return uint32_t(__builtin_amdgcn_readlane(int32_t(v), int32_t(lane)));
 }
 
-// Words that are the same for every lane, in scalar registers (outside a kernel
-// the compiler keeps what it loads from memory that is written in vector ones).
+// Words that are the same for every lane, in scalar registers: in a function that
+// is no kernel the compiler keeps what it loads from memory that is written in
+// vector ones (four-arm stars of 580 members: 2.10 us per substep, so 2.01).
 __device__ __forceinline__ uint32_t uniform(uint32_t v) { return uint32_t(__builtin_amdgcn_readfirstlane(int32_t(v))); }
 __device__ __forceinline__ u32x4 uniform(u32x4 v) { return u32x4{uniform(v.x), uniform(v.y), uniform(v.z), uniform(v.w)}; }
 
@@ -177,7 +178,7 @@ __device__ __forceinline__ u32x4 unpack_cells(uint32_t v) {
     return cells;
 }
 
-template <int ROUNDS, int MAXDEG>
+template <int ROUNDS, int MAXDEG, bool IN_KERNEL>
 __device__ __forceinline__ void resident_body(const SysDesc& d, uint32_t substeps) {
     const uint32_t B = blockDim.x, tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave64 = uint32_t(__builtin_amdgcn_readfirstlane(int32_t(tid & ~63u)));
@@ -185,7 +186,8 @@ __device__ __forceinline__ void resident_body(const SysDesc& d, uint32_t substep
     const uint32_t sProp = kLat + 4u * latWords, sPos = sProp + 4u * latWords;
 
     const gptr<const u32x4> w = (gptr<const u32x4>)d.state.global();
-    const u32x4 w0 = uniform(w[0]), w1 = uniform(w[1]), w2 = uniform(w[2]), w3 = uniform(w[3]);  // DevState field order
+    auto word = [&](int i) { return IN_KERNEL ? w[i] : uniform(w[i]); };
+    const u32x4 w0 = word(0), w1 = word(1), w2 = word(2), w3 = word(3);  // DevState field order
     const uint64_t t0 = join64(w0.x, w0.y), stopAt = join64(w0.z, w0.w);
     if (t0 >= stopAt || substeps == 0u) return;
     const uint32_t n = uint32_t(min(uint64_t(substeps), stopAt - t0));
@@ -349,7 +351,7 @@ __host__ __device__ __forceinline__ uint32_t batch_rounds(uint32_t members, uint
 
 template <int ROUNDS, int MAXDEG>
 __global__ __launch_bounds__(1024) void k_resident(SysDesc d, uint32_t substeps) {
-    resident_body<ROUNDS, MAXDEG>(d, substeps);
+    resident_body<ROUNDS, MAXDEG, true>(d, substeps);
 }
 
 // A function of its own per build, so that each has the registers it needs and
@@ -358,7 +360,7 @@ template <int ROUNDS, int MAXDEG>
 __device__ __attribute__((noinline)) void resident_build(const SysDesc* desc, uint32_t substeps) {
     const uint64_t p = uint64_t(uintptr_t(desc));
     const uint64_t u = join64(uniform(uint32_t(p)), uniform(uint32_t(p >> 32)));
-    resident_body<ROUNDS, MAXDEG>(*(const SysDesc*)(cptr<SysDesc>)uintptr_t(u), uniform(substeps));
+    resident_body<ROUNDS, MAXDEG, false>(*(const SysDesc*)(cptr<SysDesc>)uintptr_t(u), uniform(substeps));
 }
 
 template <int ROUNDS>
@@ -375,7 +377,7 @@ __device__ __forceinline__ void resident_of_degree(const SysDesc* desc, uint32_t
 template <int ROUNDS, int MAXDEG>
 __global__ __launch_bounds__(1024) void k_resident_batch(const SysDesc* __restrict__ descs,
                                                          const uint32_t* __restrict__ ids, uint32_t substeps) {
-    resident_body<ROUNDS, MAXDEG>(descs[ids[blockIdx.x]], substeps);
+    resident_body<ROUNDS, MAXDEG, true>(descs[ids[blockIdx.x]], substeps);
 }
 
 // Replicas of several builds, each swept by its own.  Eight replicas of 5000
