@@ -35,10 +35,19 @@ namespace pscbfm {
 
 namespace {
 
-// Largest species of a system on its own: us per substep, resident against two
-// passes, on 64^3: 4088 members 4.8 and 5.7 (byte lattice 4.7 and 6.1), 4800 5.35
-// and 5.8 (5.25 and 6.2), 5000 5.75 and 5.7 (5.65 and 6.1).
-constexpr uint32_t kResidentAlone = 4864;
+// Largest species of a system on its own, by lattice and bonds per member: us per
+// substep, resident against two passes, on 64^3 (byte lattice in brackets).  Up to
+// two bonds: 4088 members 4.8 and 5.8 (4.8 and 6.1), 4800 5.5 and 5.9 (5.4 and 6.2),
+// 5000 5.75 and 5.7 (5.65 and 6.1).  Up to four: 4317 5.9 and 6.1 (5.7 and 6.4),
+// 4687 6.2 and 6.0 (6.0 and 6.3), 4810 (6.0 and 6.45).  More: 2614 5.0 and 6.2 (4.8
+// and 6.7), 3267 6.25 and 6.2 (6.0 and 6.6), 3594 6.6 and 6.1 (6.3 and 6.6), 4084 7.3
+// and 6.2 (7.0 and 6.75).
+uint32_t resident_alone(const SysDesc& d) {
+    const bool bytes = d.latticeKind == kLatticeU8;
+    if (d.maxDegree <= 2u) return 4864u;
+    if (d.maxDegree <= 4u) return bytes ? 4864u : 4480u;
+    return bytes ? 3776u : 3200u;
+}
 // Of a batch replica of up to two bonds whatever else the batch holds: with
 // 5120 members 5.7 us per substep (byte lattice 5.6), where a batch of one to
 // four such two-pass replicas takes 6.0 to 6.2 (6.2 to 6.6).
@@ -407,7 +416,7 @@ ResidentKernel resident_kernel(uint32_t rounds, uint32_t maxDegree) {
     if (rounds <= 2u) return resident_by_degree<2>(maxDegree);
     if (rounds <= 3u) return resident_by_degree<3>(maxDegree);
     if (rounds <= 4u) return resident_by_degree<4>(maxDegree);
-    return resident_by_degree<5>(maxDegree);
+    return maxDegree <= 2u ? k_resident<5, 2> : k_resident<5, 4>;  // more bonds: at most four (resident_alone)
 }
 using ResidentBatchKernel = void (*)(const SysDesc*, const uint32_t*, uint32_t);
 template <int ROUNDS>
@@ -436,7 +445,7 @@ uint64_t resident_lds_bytes(const SysDesc& d) {
 }
 
 uint32_t resident_block(const SysDesc& d) {
-    if (d.maxColorCount == 0u || d.maxColorCount > kResidentAlone || d.lone != 0u) return 0u;
+    if (d.maxColorCount == 0u || d.maxColorCount > resident_alone(d) || d.lone != 0u) return 0u;
     // A thread per member, but no fewer than one per 16 bytes of the lattice, up
     // to 512: every substep clears the proposals, every launch loads and stores
     // all.  One chain of 128, us per substep with 64, 256, 512 and 1024 threads:

@@ -55,14 +55,18 @@ void stage(Updater& u, uint32_t edge, const std::vector<int32_t>& xyz, const std
     u.setSeed(7);
 }
 
-// Stars of `arms` arms of 9, ends crosslinked.
-uint32_t add_stars(Batch& b, uint32_t edge, uint32_t stars, uint32_t arms) {
+// Stars of `arms` arms of 9 (6 for more than four), ends crosslinked.
+void stage_stars(Updater& u, uint32_t edge, uint32_t stars, uint32_t arms) {
     const uint32_t box[3] = {edge, edge, edge};
     std::vector<int32_t> xyz;
     std::vector<uint32_t> bonds;
-    if (!build_star_network(box, stars, arms, 9, 1, xyz, bonds)) throw std::runtime_error("box too small");
-    Updater u;
+    if (!build_star_network(box, stars, arms, arms > 4 ? 6 : 9, 1, xyz, bonds)) throw std::runtime_error("box too small");
     stage(u, edge, xyz, bonds);
+}
+
+uint32_t add_stars(Batch& b, uint32_t edge, uint32_t stars, uint32_t arms) {
+    Updater u;
+    stage_stars(u, edge, stars, arms);
     const StagedSystem s = u.staged();
     return b.add(layout_of(s), s.seed, 0);
 }
@@ -227,6 +231,30 @@ void branched_replicas_take_the_faster_path() {
     expect(small.resident && !small.twoPass, "3700 members of up to four bonds: resident");
 }
 
+// The same of a system on its own: three species, 37 members a star of four arms
+// and 49 of eight.
+void branched_systems_take_the_faster_path() {
+    struct {
+        uint32_t stars, arms, lattice;
+        bool resident;
+    } const cases[] = {{350, 4, kLatticeBit, true},  {380, 4, kLatticeBit, false}, {390, 4, kLatticeU8, true},
+                       {160, 8, kLatticeBit, true},  {220, 8, kLatticeBit, false}, {220, 8, kLatticeU8, true},
+                       {250, 8, kLatticeU8, false}};
+    for (const auto& c : cases) {
+        Updater u;
+        stage_stars(u, 64, c.stars, c.arms);
+        u.setLatticeKind(c.lattice);
+        u.initialize();
+        fake::runtime().launches.clear();
+        u.runSimulationOnGPU(2);
+        bool resident = false;
+        for (const fake::Launch& l : fake::runtime().launches)
+            resident = resident || l.kernel.find("k_resident") != std::string::npos;
+        expect(resident == c.resident, std::to_string(c.stars) + " stars of " + std::to_string(c.arms) + " arms, lattice " +
+                                           std::to_string(c.lattice));
+    }
+}
+
 // Kernels take a state's buffers as they are: what they could not read whole
 // entries from never reaches the device.
 void misaligned_buffers_are_refused() {
@@ -265,6 +293,7 @@ const std::map<std::string, std::function<void()>> cases = {
     {"streams_stay_with_their_device", streams_stay_with_their_device},
     {"prepared_graphs_serve_logged_runs", prepared_graphs_serve_logged_runs},
     {"branched_replicas_take_the_faster_path", branched_replicas_take_the_faster_path},
+    {"branched_systems_take_the_faster_path", branched_systems_take_the_faster_path},
     {"misaligned_buffers_are_refused", misaligned_buffers_are_refused},
 };
 

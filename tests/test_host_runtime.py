@@ -11,7 +11,8 @@ HOSTRT = Path(__file__).resolve().parent / "hostrt"
 
 CASES = ["failed_launch_joins_the_side_stream", "misaligned_buffers_are_refused",
          "no_stream_outlives_a_device_reset", "streams_stay_with_their_device",
-         "prepared_graphs_serve_logged_runs", "branched_replicas_take_the_faster_path"]
+         "prepared_graphs_serve_logged_runs", "branched_replicas_take_the_faster_path",
+         "branched_systems_take_the_faster_path"]
 
 
 @pytest.fixture(scope="module")
