@@ -143,15 +143,19 @@ int pscbfm_set_colors(pscbfm_updater* h, const uint8_t* colors, uint32_t n);
  * default): chosen by size, and small systems run in one workgroup's LDS
  * instead.  Results do not depend on the shape. */
 int pscbfm_set_launch_shape(pscbfm_updater* h, uint32_t block, uint32_t slots);
-/* Pass-2 threads per workgroup (64..256, multiple of 64; 0 = automatic:
- * 128 with one monomer per pass-1 thread or at least a quarter of the cells
- * occupied, else the pass-1 block).  Results do not depend on it. */
+/* Pass-2 threads per workgroup (64..256, multiple of 64; 0 = automatic: a
+ * pass-1 block of up to 128 threads as it is; else 64 with one monomer per
+ * pass-1 thread, more than two bonds on some monomer and at least 0.4 of the
+ * cells occupied, 128 with one monomer per thread or at least a quarter
+ * occupied, and the pass-1 block otherwise).  A stated value keeps a small
+ * system on the two-pass kernels.  Results do not depend on it. */
 int pscbfm_set_perform_block(pscbfm_updater* h, uint32_t block);
 /* Pass-2 walk of a single system: threads_per_list threads walk one pass-1
  * list (64..256, multiple of 64), so a pass-2 workgroup walks several lists,
  * with entries_per_thread entries in flight per thread (1 or 4; 0 = 4);
  * threads_per_list = 0 or 0xFFFFFFFF (the default) walks one list per
- * workgroup.  Results do not depend on it. */
+ * workgroup.  Any value but 0 keeps a small system on the two-pass kernels.
+ * Results do not depend on it. */
 int pscbfm_set_perform_walk(pscbfm_updater* h, uint32_t threads_per_list, uint32_t entries_per_thread);
 /* Slot order inside each species, before initialize: 1 places the members
  * of a species in the Z-curve order of their starting corners, 0 in
@@ -163,10 +167,12 @@ int pscbfm_set_perform_walk(pscbfm_updater* h, uint32_t threads_per_list, uint32
  * (CRITICAL.cu:322-323), so results do not depend on it.  Other values:
  * PSCBFM_INVALID_ARGUMENT. */
 int pscbfm_set_slot_order(pscbfm_updater* h, int order);
-/* The pass of each substep (1 or 2; 0 = automatic: pass 1 on the bit
- * lattice with at most two bonds per monomer, else pass 2) that zeroes the
- * other parity's proposal buffer, the reference's separate clear
- * (CRITICAL.cu:561-573).  Results do not depend on it. */
+/* The pass of each substep (1 or 2; 0 = automatic: pass 2 on the byte
+ * lattice and for systems on the bit lattice with at most two bonds per
+ * monomer, 2^16 to 2^19 members of a species and at least 0.4 of the cells
+ * occupied, else pass 1) that zeroes the other parity's proposal buffer, the
+ * reference's separate clear (CRITICAL.cu:561-573).  A stated pass keeps a
+ * small system on the two-pass kernels.  Results do not depend on it. */
 int pscbfm_set_clear_pass(pscbfm_updater* h, uint32_t pass);
 /* Substeps per captured graph (0 = automatic, at most 4096:
  * PSCBFM_INVALID_ARGUMENT above). */

@@ -370,13 +370,15 @@ class UpdaterGPUScBFM_AB_Type:
         self._call("pscbfm_set_launch_shape", int(block), int(slots))
 
     def setPerformBlock(self, block: int = 0) -> None:
-        """Pass-2 threads per workgroup (0: automatic, 128 with one monomer per
-        pass-1 thread or at least a quarter occupied, else the pass-1 block)."""
+        """Pass-2 threads per workgroup (0: automatic, by the pass-1 shape, the
+        occupied fraction and the bonds, see pscbfm_set_perform_block in
+        pscbfm.h).  A stated value keeps a small system on the two-pass kernels."""
         self._call("pscbfm_set_perform_block", int(block))
 
     def setPerformWalk(self, threads_per_list: int = 0, entries_per_thread: int = 0) -> None:
         """Pass-2 walk: threads per pass-1 list (0 or LEGACY_WALK, the default:
-        one list per workgroup) and entries in flight per thread (1 or 4; 0: 4)."""
+        one list per workgroup) and entries in flight per thread (1 or 4; 0: 4).
+        Any value but 0 keeps a small system on the two-pass kernels."""
         self._call("pscbfm_set_perform_walk", int(threads_per_list), int(entries_per_thread))
 
     def setSlotOrder(self, order=None) -> None:
@@ -391,9 +393,10 @@ class UpdaterGPUScBFM_AB_Type:
         self._call("pscbfm_set_slot_order", codes[order])
 
     def setClearPass(self, pass_: int = 0) -> None:
-        """The pass (1 or 2; 0: automatic, pass 1 on the bit lattice with at
-        most two bonds per monomer, else pass 2) that zeroes the other
-        parity's proposal buffer each substep."""
+        """The pass (1 or 2; 0: automatic) that zeroes the other parity's
+        proposal buffer each substep.  Automatic: pass 2 on the byte lattice and
+        for dense unbranched systems of 2^16 to 2^19 members of a species, else
+        pass 1.  A stated pass keeps a small system on the two-pass kernels."""
         self._call("pscbfm_set_clear_pass", int(pass_))
 
     def setReadBack(self, on: bool) -> None:

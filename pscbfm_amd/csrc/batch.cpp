@@ -29,9 +29,10 @@ constexpr uint32_t kSpreadTiles = 64;  // replicas with at least this many workg
 uint32_t degree_bucket(uint32_t d) { return d <= 2 ? 2u : (d <= 4 ? 4u : 8u); }
 
 // Pass-2 threads per workgroup of a batch with pass-1 block `block`: at most
-// 192.  On the 1024-replica mix (pass 1 at 256 x 2) pass 2 with 192 threads
-// took 128.6-129.3 ms for 500 MCS, with 128 130.1, with 256 131.2-134.0 and
-// with 64 137.5.
+// 192.  ms for 300 sweeps with 64, 128, 192 and 256 threads (pass 1 at 256 x 2,
+// small replicas resident): mix of 1024 systems 59.7, 56.9, 57.2 and 57.7, byte
+// lattice 86.7, 85.1, 86.0 and 86.6; of 256 systems 15.8, 15.2, 15.1 and 15.3;
+// of 60 larger ones 11.6, 11.4, 11.1 and 11.1 (14.2, 13.7, 13.5 and 13.6).
 uint32_t default_perform_block(uint32_t block) { return block > 192u ? 192u : block; }
 }  // namespace
 

@@ -6,10 +6,10 @@
 // it the kernel boundaries and the round trips of a few dependent loads.  Here
 // the boundary between the passes is a workgroup barrier and the gathers are
 // LDS reads, so a substep costs what its vector instructions cost on one
-// compute unit: 1.0 us for 192 members of the drawn species (two passes: 5.9),
-// 1.45 for 512, 4.75 for 4000, 5.75 for 5000 (6.1 in a batch): vector issue on one
-// compute unit (150 instructions per 64 members; 7% more cost 1.09 us instead of
-// 1.01 for 192 members, in a batch 6.6 instead of 6.1 for 5000).
+// compute unit: 0.9 us for 192 members of the drawn species (two passes: 5.1),
+// 1.1 to 1.25 for 512 (5.8), 3.2 for 2500, 4.8 for 4000 and 5.5 for 4800 (5.9), in a
+// batch 5.9 for 5000: vector issue on one compute unit (150 instructions per 64
+// members; when it was 7% more, 192 members took 1.09 us instead of 1.01).
 //
 // LDS: the occupancy lattice and one proposal lattice (1 bit per cell, Z-curve
 // order, whatever lattice kind the system has in memory), the code of every

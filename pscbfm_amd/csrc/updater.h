@@ -129,8 +129,7 @@ public:
     // monomer index); see SystemInput::slotOrder.  Results do not depend on it.
     void setSlotOrder(SlotOrder order);
     // The pass (1 or 2) that zeroes the other parity's proposal buffer each
-    // substep; 0 = automatic (pass 1 on the bit lattice with at most two
-    // bonds per monomer, else pass 2).
+    // substep; 0 = automatic_clear_pass.
     void setClearPass(uint32_t pass);
     // R250 mode: from the next run on, every substep draws its species
     // (r250 % nColors) and kernel seed (r250) from this generator in the

@@ -27,12 +27,15 @@ KERNELS = {"k_check_batch": "pass 1, batch (k_check_batch)", "k_perform_batch": 
            "k_set_stops": "stop points, batch", "k_check": "pass 1 (k_check)", "k_perform": "pass 2 (k_perform)",
            "k_copy_u4": "copy reference", "k_advance": "counter advance", "k_fill_u32": "fill",
            "k_unfold": "coordinate decode (read-back)", "k_perform_lists": "pass 2, several lists (k_perform_lists)",
-           "k_unfold_jobs": "coordinate decode, batch (read-back)"}
+           "k_unfold_jobs": "coordinate decode, batch (read-back)", "k_resident": "resident sweep (k_resident)",
+           "k_resident_batch": "resident sweep, batch (k_resident_batch)",
+           "k_resident_mix": "resident sweep, batch of several builds (k_resident_mix)",
+           "k_log_last": "last log entry", "k_wait": "stream overlap probe"}
 
 
 _NAME = re.compile(r"\b(k_[a-z0-9_]+?)(?=[<(]|$)")
 _LATTICE = re.compile(r"\b(k_(?:check|perform)(?:_batch)?)<(\d+)")
-SWEEP = ("k_check", "k_perform", "k_check_batch", "k_perform_batch")
+SWEEP = ("k_check", "k_perform", "k_check_batch", "k_perform_batch", "k_resident", "k_resident_batch", "k_resident_mix")
 
 
 def _short(name: str) -> str:
